@@ -128,6 +128,8 @@ THM_HD constexpr uint32_t xtr_frag_off(int k0, int half, int c0, int lane, int r
 constexpr int kWyPitch = 20;
 THM_HD constexpr int wy_put_off(int lane, int r) { return (4 * (lane >> 4) + r) * kWyPitch + (lane & 15); }
 THM_HD constexpr int wy_a_off(int lane, int q) { return (lane & 15) * kWyPitch + 4 * q + (lane >> 4); }
+//   (wy_row_off: A operand row l, columns 4 g .. 4 g + 3 in one 16-byte read)
+THM_HD constexpr int wy_row_off(int lane) { return (lane & 15) * kWyPitch + 4 * (lane >> 4); }
 THM_HD constexpr int wy_b_off(int lane, int q) { return (4 * q + (lane >> 4)) * kWyPitch + (lane & 15); }
 
 // recompute_w_u's output staging tile: the w (or u) rows of the tile's 64

@@ -21,7 +21,7 @@ namespace wy {
 constexpr int kBT = 64;
 constexpr int kBP = hl::kWyPitch;  // LDS pitch (floats) of a 16x16 block (h_layout.h)
 constexpr int kBlk = 16 * kBP;  // floats per block
-constexpr int kLdsFloats = 10 * kBlk + 10 * kBlk + 3 * kBlk;  // L, X, per-level T
+constexpr int kLdsFloats = 10 * kBlk + 10 * kBlk;  // L, X
 
 // Packed index of lower block (i, j), j <= i < 4.
 __host__ __device__ constexpr int blk(int i, int j) { return i * (i + 1) / 2 + j; }
@@ -30,19 +30,23 @@ __device__ __forceinline__ f32x4 mfma16x16x4f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// acc += P Q for 16x16 blocks P, Q in LDS (pitch kBP): lane (g, l) feeds
-// P[l][4q + g] and Q[4q + g][l] at k-step q; acc[r] = row 4g + r, column l.
-__device__ __forceinline__ f32x4 block_mm(const float* P, const float* Q, f32x4 acc) {
-  const int lane = lane_id();
+// acc += P X for a 16x16 block P in LDS (pitch kBP) and X in accumulator form
+// (lane (g, l): rows 4g + r of column l in x[r]): at k-step q lane (g, l) feeds
+// P[l][4g + q] and X[4g + q][l] = x[q], so an accumulator is the next product's
+// B operand as it stands and P is one 16-byte row read per lane.
+__device__ __forceinline__ f32x4 block_row4(const float* P) {
+  return *reinterpret_cast<const f32x4*>(P + hl::wy_row_off(lane_id()));
+}
+__device__ __forceinline__ f32x4 block_mm(f32x4 p, f32x4 x, f32x4 acc) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc = mfma16x16x4f32(P[hl::wy_a_off(lane, q)], Q[hl::wy_b_off(lane, q)], acc);
+  for (int q = 0; q < 4; ++q) acc = mfma16x16x4f32(p[q], x[q], acc);
   return acc;
 }
 
-__device__ __forceinline__ void block_put(float* D, f32x4 acc, float sgn) {
+__device__ __forceinline__ void block_put(float* D, f32x4 acc) {
   const int lane = lane_id();
 #pragma unroll
-  for (int r = 0; r < 4; ++r) D[hl::wy_put_off(lane, r)] = sgn * acc[r];
+  for (int r = 0; r < 4; ++r) D[hl::wy_put_off(lane, r)] = acc[r];
 }
 
 // L blocks of one chunk from k fragments fh[tb][s] = k[16 tb + li][32 s + 8 grp .. + 7]
@@ -108,17 +112,46 @@ __device__ __forceinline__ void form_L_lds(Frag frag, const float* sb, const flo
   }
 }
 
+// Column J of X below the diagonal, X_{J+1,J} .. X_{3,J}, by one wave:
+// T = sum_m L_im X_mJ, X_iJ = -X_ii T.  T and the X_mJ stay in accumulators,
+// which are the next products' B operands; only L_im and X_ii come from LDS
+// (row reads with no dependence on the chain, so they run ahead of it).
+template <int J>
+__device__ __forceinline__ void invert_column(const float* Lb, float* Xb) {
+  if constexpr (J < 3) {
+    f32x4 x[4];
+    const float* D = Xb + blk(J, J) * kBlk;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[J][r] = D[hl::wy_put_off(lane_id(), r)];
+    f32x4 l[4][3], xi[4];
+#pragma unroll
+    for (int i = J + 1; i < 4; ++i) {
+      xi[i] = block_row4(Xb + blk(i, i) * kBlk);
+#pragma unroll
+      for (int m = J; m < i; ++m) l[i][m] = block_row4(Lb + blk(i, m) * kBlk);
+    }
+#pragma unroll
+    for (int i = J + 1; i < 4; ++i) {
+      f32x4 t = zero4();
+#pragma unroll
+      for (int m = J; m < i; ++m) t = block_mm(l[i][m], x[m], t);
+      x[i] = -block_mm(xi[i], t, zero4());
+      block_put(Xb + blk(i, J) * kBlk, x[i]);
+    }
+  }
+}
+
 // X = (I + L)^{-1} from the L blocks (all four waves; ends with a barrier):
 //   diagonal blocks: wave w, lane c < 16 owns column c of X_ww (16-row
 //   forward substitution), then one barrier;
-//   off-diagonal blocks: wave j forms column j of X, X_{j+1,j} .. X_{3,j}
-//   (3, 2, 1 and 0 blocks), each two fp32 MFMA products (exact fp32
-//   multiplies): T = sum L_im X_mj, then X_ij = -X_ii T, T passing through
-//   the wave's own LDS block to change from the accumulator to the operand
-//   layout.  One barrier at the end (a barrier per level measured 266 against
-//   251 us for the fused WY kernel at config 4, 146 against 141 for the
-//   A-builder, bit-identical).
-__device__ __forceinline__ void invert_L(const float* Lb, float* Xb, float* Tb, int wv) {
+//   off-diagonal blocks: wave j forms column j of X (invert_column), exact
+//   fp32 multiplies; one barrier at the end.
+// The products' latency chain costs, not their count.  With T and X_mj passed
+// through LDS between products -> handed over in accumulators (HIP events):
+// fused WY at config 4 254 -> 246 us, at K = V = 64 190 -> 179; A-builder at
+// 2048 tiles of K = 128 20.6 -> 20.0, at 48 tiles 9.4 -> 9.0; at config 4 it
+// is bound by its bytes (111-113 either way).  Error against float64 unchanged.
+__device__ __forceinline__ void invert_L(const float* Lb, float* Xb, int wv) {
   const int lane = lane_id();
   {
     const float* L = Lb + blk(wv, wv) * kBlk;
@@ -139,28 +172,9 @@ __device__ __forceinline__ void invert_L(const float* Lb, float* Xb, float* Tb, 
     }
   }
   lds_barrier();
-  // Column j of X is wave j's alone: X_ij needs X_mj (m < i, this wave's own
-  // earlier blocks), the L blocks and X_ii (both behind the barrier above), so
-  // the levels need no workgroup barrier.  Each block a wave writes (T, then
-  // X_ij) is read back by other lanes of the same wave, so every write is
-  // followed by a wave-scope sync.
-#pragma unroll
-  for (int d = 1; d < 4; ++d) {
-    const int j = wv, i = wv + d;
-    if (i < 4) {  // wave-uniform
-      f32x4 acc = zero4();
-#pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        const int mm = j + m;
-        if (mm < i) acc = block_mm(Lb + blk(i, mm) * kBlk, Xb + blk(mm, j) * kBlk, acc);
-      }
-      block_put(Tb + wv * kBlk, acc, 1.f);
-      wave_lds_sync();
-      acc = block_mm(Xb + blk(i, i) * kBlk, Tb + wv * kBlk, zero4());
-      block_put(Xb + blk(i, j) * kBlk, acc, -1.f);
-      wave_lds_sync();
-    }
-  }
+  if (wv == 0) invert_column<0>(Lb, Xb);
+  else if (wv == 1) invert_column<1>(Lb, Xb);
+  else if (wv == 2) invert_column<2>(Lb, Xb);
   lds_barrier();
 }
 

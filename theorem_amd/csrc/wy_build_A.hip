@@ -65,9 +65,8 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
                   int64_t NT) {
   constexpr bool kSplit = std::is_same<IT, float>::value;
   constexpr int KS = K / 32;  // contraction steps
-  __shared__ float Lb[10 * kBlk];  // L = sign M, lower blocks (diagonal blocks: strict lower part)
-  __shared__ float Xb[10 * kBlk];  // X = A_c, lower blocks
-  __shared__ float Tb[3 * kBlk];   // per-level partial products
+  __shared__ __attribute__((aligned(16))) float Lb[10 * kBlk];  // L = sign M, lower blocks (diagonal blocks: strict lower part)
+  __shared__ __attribute__((aligned(16))) float Xb[10 * kBlk];  // X = A_c, lower blocks
   __shared__ float sb[kBT], sg[kBT];
 
   const TileCoord tc = tile_coord(blockIdx.x, H, NT, T);
@@ -105,7 +104,7 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
   // 2. L blocks; 3.-4. X = (I + L)^{-1}.
   wy::form_L<SIGN, KS, kSplit>(fh, fl, sb, sg, Lb, wv);
   lds_barrier();
-  wy::invert_L(Lb, Xb, Tb, wv);
+  wy::invert_L(Lb, Xb, wv);
 
   // 5. A_c rows.
   store_A(Xb, A + (tok0 * H + h) * kBT, H);
@@ -149,12 +148,11 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
   // The k tile is read only up to the barrier after form_L and restaged
   // after the barrier that follows the store of A, so the inversion's X and T
   // blocks share its LDS.
-  constexpr int kKBytes = kBT * kPitch * 2, kXTBytes = 13 * kBlk * 4;
-  __shared__ __attribute__((aligned(16))) char kxt[kKBytes > kXTBytes ? kKBytes : kXTBytes];
+  constexpr int kKBytes = kBT * kPitch * 2, kXBytes = 10 * kBlk * 4;
+  __shared__ __attribute__((aligned(16))) char kxt[kKBytes > kXBytes ? kKBytes : kXBytes];
   bf16* const ks = reinterpret_cast<bf16*>(kxt);
   float* const Xb = reinterpret_cast<float*>(kxt);
-  float* const Tb = Xb + 10 * kBlk;
-  __shared__ float Lb[10 * kBlk];
+  __shared__ __attribute__((aligned(16))) float Lb[10 * kBlk];
   __shared__ float sb[kBT], sg[kBT];
 
   const int tid = threadIdx.x;
@@ -215,7 +213,7 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
     wy::form_L_lds<SIGN, KS>([&](int tb, int s) { return load8(ks + (16 * tb + li) * kPitch + 32 * s + 8 * grp); },
                              sb, sg, Lb, wv);
     lds_barrier();  // every wave's k fragment reads are done: X may overwrite ks
-    wy::invert_L(Lb, Xb, Tb, wv);  // ends with a barrier
+    wy::invert_L(Lb, Xb, wv);  // ends with a barrier
     store_A(Xb, A + (tok0 * H + h) * kBT, H);
 
     if (tn >= tiles) break;

@@ -129,7 +129,6 @@ wy_fwd_kernel(const bf16* __restrict__ k, const bf16* __restrict__ v,
   __shared__ float sb[kBT], sg[kBT];
   float* const Lb = reinterpret_cast<float*>(lds);  // L = sign M, lower blocks
   float* const Xb = Lb + 10 * kBlk;                  // X = A_c, lower blocks
-  float* const Tb = Xb + 10 * kBlk;                  // per-level partial products
   char* const xs = lds;                              // [k | v] tile, after the inversion
 
   const TileCoord tc = tile_coord(blockIdx.x, H, NT, T);
@@ -169,7 +168,7 @@ wy_fwd_kernel(const bf16* __restrict__ k, const bf16* __restrict__ v,
   lds_barrier();
 
   // 3. X = (I + L)^{-1}.
-  wy::invert_L(Lb, Xb, Tb, wv);
+  wy::invert_L(Lb, Xb, wv);
 
   // 4. Scaled A operands of this wave (read from X before the tile overwrites it).
   const WyOperands op = wy_operands(Xb, sb, sg, wv);
@@ -214,9 +213,8 @@ wy_fwd_pipe_kernel(const bf16* __restrict__ k, const bf16* __restrict__ v,
   using C = WyCfg<K, V>;
   constexpr int KS = C::KS;
   __shared__ __attribute__((aligned(16))) char xs[kBT * C::kPitch];  // [k | v] tile
-  __shared__ float Lb[10 * kBlk];  // L = sign M, lower blocks
-  __shared__ float Xb[10 * kBlk];  // X = A_c, lower blocks
-  __shared__ float Tb[3 * kBlk];   // per-level partial products
+  __shared__ __attribute__((aligned(16))) float Lb[10 * kBlk];  // L = sign M, lower blocks
+  __shared__ __attribute__((aligned(16))) float Xb[10 * kBlk];  // X = A_c, lower blocks
   __shared__ float sb[kBT], sg[kBT];
 
   const int tid = threadIdx.x;
@@ -298,7 +296,7 @@ wy_fwd_pipe_kernel(const bf16* __restrict__ k, const bf16* __restrict__ v,
         fh[tb][s] = load8(reinterpret_cast<const bf16*>(xs + hl::ntile_off(16 * tb + li, 32 * s + 8 * grp, C::kPitch)));
     wy::form_L<SIGN, KS, false>(fh, fl, sb, sg, Lb, wv);
     lds_barrier();
-    wy::invert_L(Lb, Xb, Tb, wv);  // ends with a barrier
+    wy::invert_L(Lb, Xb, wv);  // ends with a barrier
     const WyOperands op = wy_operands(Xb, sb, sg, wv);
     wy_products<K, V>(xs, C::kPitch, op, w, u, (tok0 + 16 * wv + li) * H + h);
 
