@@ -20,7 +20,9 @@ namespace wy {
 
 constexpr int kBT = 64;
 constexpr int kBP = hl::kWyPitch;  // LDS pitch (floats) of a 16x16 block (h_layout.h)
-constexpr int kBlk = 16 * kBP;  // floats per block
+// Floats per block, 4 over the rows: the four diagonal blocks (the substitution
+// reads all of them in one instruction) then start on different banks.
+constexpr int kBlk = 16 * kBP + 4;
 constexpr int kLdsFloats = 10 * kBlk + 10 * kBlk;  // L, X
 
 // Packed index of lower block (i, j), j <= i < 4.
@@ -75,8 +77,8 @@ __device__ __forceinline__ void form_L(const bf16x8 (&fh)[4][KS], const bf16x8 (
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * ib + 4 * grp + r;
-      Lb[p * kBlk + hl::wy_put_off(lane, r)] =
-          (j < i) ? (float)SIGN * sb[i] * acc[r] * fast_exp(sg[i] - sg[j]) : 0.f;
+      const float l = (float)SIGN * sb[i] * acc[r] * fast_exp(sg[i] - sg[j]);
+      Lb[p * kBlk + hl::wy_put_off(lane, r)] = (jb < ib || j < i) ? l : 0.f;
     }
   }
 }
@@ -106,8 +108,8 @@ __device__ __forceinline__ void form_L_lds(Frag frag, const float* sb, const flo
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * ib + 4 * grp + r;
-      Lb[p * kBlk + hl::wy_put_off(lane, r)] =
-          (j < i) ? (float)SIGN * sb[i] * acc[r] * fast_exp(sg[i] - sg[j]) : 0.f;
+      const float l = (float)SIGN * sb[i] * acc[r] * fast_exp(sg[i] - sg[j]);
+      Lb[p * kBlk + hl::wy_put_off(lane, r)] = (jb < ib || j < i) ? l : 0.f;
     }
   }
 }
@@ -141,40 +143,41 @@ __device__ __forceinline__ void invert_column(const float* Lb, float* Xb) {
   }
 }
 
-// X = (I + L)^{-1} from the L blocks (all four waves; ends with a barrier):
-//   diagonal blocks: wave w, lane c < 16 owns column c of X_ww (16-row
-//   forward substitution), then one barrier;
-//   off-diagonal blocks: wave j forms column j of X (invert_column), exact
-//   fp32 multiplies; one barrier at the end.
+// X = (I + L)^{-1} from the L blocks (all four waves, `role` a permutation of
+// them; ends with a barrier):
+//   diagonal blocks: role 3, lane (d, c) owns column c of X_dd (16-row
+//   forward substitution of all four blocks at once), then one barrier;
+//   off-diagonal blocks: role j < 3 forms column j of X (invert_column, 9, 5
+//   and 2 products), exact fp32 multiplies; one barrier at the end.
 // The products' latency chain costs, not their count.  With T and X_mj passed
-// through LDS between products -> handed over in accumulators (HIP events):
-// fused WY at config 4 254 -> 246 us, at K = V = 64 190 -> 179; A-builder at
-// 2048 tiles of K = 128 20.6 -> 20.0, at 48 tiles 9.4 -> 9.0; at config 4 it
-// is bound by its bytes (111-113 either way).  Error against float64 unchanged.
-__device__ __forceinline__ void invert_L(const float* Lb, float* Xb, int wv) {
-  const int lane = lane_id();
-  {
-    const float* L = Lb + blk(wv, wv) * kBlk;
-    float* X = Xb + blk(wv, wv) * kBlk;
-    if (lane < 16) {
-      float x[16];
+// through LDS between products -> handed over in accumulators -> the four
+// substitutions in one wave (a quarter of their issue slots; HIP events):
+// fused WY at config 4 254 -> 246 -> 230 us, at K = V = 64 190 -> 179 -> 168;
+// A-builder at config 4 (its roles also rotated over the SIMDs) 112 -> 112 ->
+// 101, at 2048 tiles of K = 128 20.6 -> 20.0 -> 19.0, at 48 tiles 9.4 -> 9.0
+// -> 8.1.  Error against float64 unchanged.
+__device__ __forceinline__ void invert_L(const float* Lb, float* Xb, int role) {
+  if (role == 3) {
+    const int lane = lane_id(), d = lane >> 4, col = lane & 15;
+    const float* L = Lb + blk(d, d) * kBlk;
+    float* X = Xb + blk(d, d) * kBlk;
+    float x[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float a0 = (r == lane) ? 1.f : 0.f, a1 = 0.f;
+    for (int r = 0; r < 16; ++r) {
+      float a0 = (r == col) ? 1.f : 0.f, a1 = 0.f;
 #pragma unroll
-        for (int s = 0; s < r; ++s) {
-          if (s & 1) a1 = fmaf(-L[r * kBP + s], x[s], a1);
-          else a0 = fmaf(-L[r * kBP + s], x[s], a0);
-        }
-        x[r] = a0 + a1;
-        X[r * kBP + lane] = x[r];
+      for (int s = 0; s < r; ++s) {
+        if (s & 1) a1 = fmaf(-L[r * kBP + s], x[s], a1);
+        else a0 = fmaf(-L[r * kBP + s], x[s], a0);
       }
+      x[r] = a0 + a1;
+      X[r * kBP + col] = x[r];
     }
   }
   lds_barrier();
-  if (wv == 0) invert_column<0>(Lb, Xb);
-  else if (wv == 1) invert_column<1>(Lb, Xb);
-  else if (wv == 2) invert_column<2>(Lb, Xb);
+  if (role == 0) invert_column<0>(Lb, Xb);
+  else if (role == 1) invert_column<1>(Lb, Xb);
+  else if (role == 2) invert_column<2>(Lb, Xb);
   lds_barrier();
 }
 

@@ -200,6 +200,11 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
     }
   };
 
+  // Wave w of every workgroup sits on SIMD w, and the roles of the inversion
+  // differ in work: rotated over the workgroups of a CU (launch order i,
+  // i + 256, ...), each SIMD gets one of each.
+  const int role = (wv + (int)(blockIdx.x * ab_pipe_wgs_per_cu<K>() / gridDim.x)) & 3;
+
   int64_t t = blockIdx.x;
   if (t >= tiles) return;  // whole workgroup
   prefetch(t);
@@ -213,7 +218,7 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
     wy::form_L_lds<SIGN, KS>([&](int tb, int s) { return load8(ks + (16 * tb + li) * kPitch + 32 * s + 8 * grp); },
                              sb, sg, Lb, wv);
     lds_barrier();  // every wave's k fragment reads are done: X may overwrite ks
-    wy::invert_L(Lb, Xb, wv);  // ends with a barrier
+    wy::invert_L(Lb, Xb, role);  // ends with a barrier
     store_A(Xb, A + (tok0 * H + h) * kBT, H);
 
     if (tn >= tiles) break;
