@@ -49,6 +49,7 @@ extern "C" {
 /* Gate transforms for thm_chunk_local_cumsum. */
 #define THM_GATE_IDENTITY 0   /* g = chunk-local cumsum of a              */
 #define THM_GATE_LOGSIGMOID 1 /* g = chunk-local cumsum of log(sigmoid(a)) */
+#define THM_GATE_CUMULATIVE 2 /* the gate is g itself (thm_chunk_gated_delta_rule_fwd only) */
 
 /* Flags for thm_chunk_fwd_h. */
 #define THM_H_DELTA 1 /* delta-rule form: v_new = u - w.S, h[c] stored BEFORE the
@@ -212,6 +213,32 @@ int thm_chunk_gated_delta_fwd_a(const void* q, const void* k, const void* v, con
                                 const void* A, const void* g, const void* h0, void* o, void* v_new,
                                 void* ht, float scale, int64_t B, int64_t T, int64_t H, int64_t K,
                                 int64_t V, int32_t chunk_size, int32_t qkv_dtype, void* stream);
+
+/*
+ * The whole chunked forward in one call: WY matrix (thm_wy_build_A, sign =
+ * +1), state recurrence and output from q, k, v, beta and the gate, o and ht
+ * as thm_chunk_gated_delta_fwd_a.  Replaces the composition of `_build_A`
+ * (kernels/recompute_w_u/reference.py:48-91), recompute_w_u, chunk_fwd_h
+ * (delta form) and chunk_fwd_o; no single reference function does this.
+ *   gate [B, T, H] or NULL (no gate); gate_kind THM_GATE_IDENTITY or
+ *   THM_GATE_LOGSIGMOID: per-token log decay a (F32 or BF16), as
+ *   thm_chunk_local_cumsum; THM_GATE_CUMULATIVE: g (F32).
+ *   bf16 only: q, k, v, o bf16; beta [B, T, H], h0, ht fp32 (h0, ht may be
+ *   NULL).  K, V in {64, 128}; T % 64 == 0.  q, k, v and workspace 16-byte
+ *   aligned, o 8-byte, beta, h0, ht 4-byte.
+ *   workspace: device scratch of at least thm_chunk_gated_delta_rule_workspace
+ *   bytes (its contents before and after are undefined), owned by the call
+ *   until it has run on `stream`.  Long sequences of few heads are cut into
+ *   segments that run side by side, chosen from the shape and the device's CU
+ *   count only, so results are deterministic per shape.
+ */
+int64_t thm_chunk_gated_delta_rule_workspace(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V);
+int thm_chunk_gated_delta_rule_fwd(const void* q, const void* k, const void* v, const void* beta,
+                                   const void* gate, const void* h0, void* o, void* ht,
+                                   void* workspace, int64_t workspace_bytes, float scale, int64_t B,
+                                   int64_t T, int64_t H, int64_t K, int64_t V, int32_t chunk_size,
+                                   int32_t qkv_dtype, int32_t gate_dtype, int32_t gate_kind,
+                                   void* stream);
 
 /*
  * WY matrix of the chunked Gated DeltaNet forward, per chunk c of

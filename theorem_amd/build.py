@@ -33,6 +33,7 @@ SOURCES = [
     "chunk_fwd_h_f32.hip",
     "chunk_fwd_o.hip",
     "chunk_fwd_fused.hip",
+    "chunk_fwd_rec.hip",
     "wy_build_A.hip",
     "wy_fwd.hip",
     "gates.hip",

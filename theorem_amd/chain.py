@@ -122,6 +122,36 @@ def chunk_fwd_fused_a(q, k, v, beta, A, g, scale: float, initial_state=None, out
     return o, vn, ht
 
 
+def _fwd_records(q, k, v, beta, gate, gate_kind: int, scale: float, initial_state, output_final_state: bool):
+    """The bf16 forward from (q, k, v, beta, gate) in one C call
+    (thm_chunk_gated_delta_rule_fwd): (o, ht or None)."""
+    B, T, H, K = k.shape
+    V = v.shape[-1]
+    assert T % BT == 0, f"T={T} must be a multiple of {BT}"
+    assert q.shape == k.shape and v.shape[:3] == (B, T, H) and beta.shape == (B, T, H)
+    assert gate is None or gate.shape == (B, T, H)
+    assert q.dtype == k.dtype == v.dtype == torch.bfloat16, "the fused path is bf16-only"
+    _capi.require_device(q, k, v, beta, gate, initial_state)
+    for name, t in (("beta", beta), ("initial_state", initial_state)):
+        _capi.require_f32(t, name)
+    if gate_kind == _capi.THM_GATE_CUMULATIVE:
+        _capi.require_f32(gate, "g")
+    code = 0 if gate is None else _capi.dtype_code(gate, "a")
+    q, k, v, beta, gate, h0 = (_capi.prep(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v"), (beta, "beta"),
+                                                            (gate, "gate"), (initial_state, "initial_state")))
+    lib = _capi.load_library()
+    nws = lib.thm_chunk_gated_delta_rule_workspace(B, T, H, K, V)
+    ws = torch.empty(max(nws, 0), dtype=torch.uint8, device=k.device)
+    o = torch.empty_like(v)
+    ht = torch.empty(B, H, K, V, dtype=torch.float32, device=k.device) if output_final_state else None
+    status = lib.thm_chunk_gated_delta_rule_fwd(
+        _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(beta), _capi.ptr(gate), _capi.ptr(h0), _capi.ptr(o),
+        _capi.ptr(ht), _capi.ptr(ws), ws.numel(), float(scale), B, T, H, K, V, BT, _capi.THM_DTYPE[torch.bfloat16],
+        code, gate_kind, _capi.stream_of(k))
+    _capi.check(status, "thm_chunk_gated_delta_rule_fwd")
+    return o, ht
+
+
 def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=None,
                                output_final_state: bool = False, A: torch.Tensor | None = None,
                                return_intermediates: bool = False, a: torch.Tensor | None = None,
@@ -131,9 +161,10 @@ def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=Non
 
     bf16 inputs run fused kernels (``fused``, default for bf16 unless
     ``return_intermediates``, which needs w, u and the per-chunk states h):
-    with ``fused_form`` "A" (default) build_A (unless ``A`` is given) and
-    chunk_fwd_fused_a (w and u never formed: recurrence and output from A);
-    with "wy" wy_fwd (A and w, u in one kernel; unless ``A`` is given) and
+    with ``fused_form`` "A" (default) one C call that forms per-chunk records
+    (A and the gates) and runs recurrence and output from them, long sequences
+    of few heads in segments side by side (w, u and the per-chunk states never
+    formed), or chunk_fwd_fused_a when ``A`` is given; with "wy" wy_fwd (A and w, u in one kernel; unless ``A`` is given) and
     chunk_fwd_fused.  Otherwise build_A, recompute_w_u, chunk_fwd_h,
     chunk_fwd_o.
     ``g`` is the chunk-local cumulative log decay [B, T, H] fp32 (or None: no
@@ -144,13 +175,17 @@ def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=Non
     V = v.shape[-1]
     if a is not None:
         assert g is None, "pass either g or a"
-        g = chunk_local_cumsum(a, logsigmoid=a_logsigmoid)
     if fused is None:
         fused = k.dtype == torch.bfloat16 and not return_intermediates
     assert fused_form in ("A", "wy"), fused_form
+    if fused and fused_form == "A" and A is None:
+        if a is None:
+            return _fwd_records(q, k, v, beta, g, _capi.THM_GATE_CUMULATIVE, scale, initial_state, output_final_state)
+        kind = _capi.THM_GATE_LOGSIGMOID if a_logsigmoid else _capi.THM_GATE_IDENTITY
+        return _fwd_records(q, k, v, beta, a, kind, scale, initial_state, output_final_state)
+    if a is not None:
+        g = chunk_local_cumsum(a, logsigmoid=a_logsigmoid)
     if fused and fused_form == "A":
-        if A is None:
-            A = build_A(k, beta, g)
         o, _, ht = chunk_fwd_fused_a(q, k, v, beta, A, g, scale, initial_state, output_final_state)
         return o, ht
     if fused and A is None:

@@ -72,17 +72,18 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// Head index and first token row of tile `tile` of a [B, T / 64, H] tile
+// Head index, first token row, batch row and chunk of tile `tile` of a [B, T / 64, H] tile
 // grid with the head fastest.  Every entry point that uses it checks that the
 // tile count is below 2^31, so 32-bit unsigned division is exact; it replaces
 // the 64-bit division sequences of int64_t % and /.
 struct TileCoord {
   int64_t hh, tok0;
+  uint32_t b, c;  // batch row, chunk
 };
 __device__ __forceinline__ TileCoord tile_coord(int64_t tile, int64_t H, int64_t NT, int64_t T) {
   const uint32_t t = (uint32_t)tile, h = (uint32_t)H, nt = (uint32_t)NT;
   const uint32_t bc = t / h, b = bc / nt;
-  return {(int64_t)(t - bc * h), (int64_t)b * T + (int64_t)(bc - b * nt) * 64};
+  return {(int64_t)(t - bc * h), (int64_t)b * T + (int64_t)(bc - b * nt) * 64, b, bc - b * nt};
 }
 
 // HIP rejects a launch of more than 2^32 - 1 work-items in total.  Every entry

@@ -16,19 +16,12 @@
 // tokens left one wave per CU at config 4: 26 us for 8 MB).  The sums are
 // formed in scan order, not left to right: they agree with a sequential
 // fp32 sum to rounding.
-#include <math.h>
-
-#include "common.h"
+#include "gate.h"
 
 namespace thm {
 namespace {
 
 constexpr int kBT = 64;
-
-__device__ __forceinline__ float logsigmoid(float x) {
-  // log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|)), exact in both tails.
-  return fminf(x, 0.f) - log1pf(expf(-fabsf(x)));
-}
 
 constexpr int kCsThreads = 256;
 constexpr int kCsHeads = 16;           // heads per workgroup

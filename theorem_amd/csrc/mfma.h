@@ -93,6 +93,18 @@ __device__ __forceinline__ void split_bf16x8(const float* v, bf16x8& hi, bf16x8&
   }
 }
 
+// 4 fp32 as 4 bf16 hi then 4 bf16 lo.
+__device__ __forceinline__ u32x4 hi_lo4(f32x4 x) {
+  bf16x4 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = (bf16)x[e];
+    lo[e] = (bf16)(x[e] - (float)hi[e]);
+  }
+  const u32x2 h2 = __builtin_bit_cast(u32x2, hi), l2 = __builtin_bit_cast(u32x2, lo);
+  return u32x4{h2[0], h2[1], l2[0], l2[1]};
+}
+
 // Load 8 consecutive elements of type T (16-byte aligned for bf16, 32-byte for
 // fp32) as floats; `nt` selects a non-temporal (streaming) load.
 __device__ __forceinline__ void load8f(const bf16* p, float* v, bool nt = false) {

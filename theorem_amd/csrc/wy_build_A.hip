@@ -25,9 +25,21 @@
 //   5. All 256 threads write A_c: 16-byte stores, 4 full 256-byte rows per
 //      wavefront instruction.
 // HBM traffic per tile: k, beta, g read once, A written once.
+//
+// The record form (REC, bf16 k, sign +1; thm_chunk_gated_delta_rule_fwd) takes
+// the gate as the caller has it (per-token log decay or its chunk-local
+// cumulative sum) and writes, instead of A rows, one contiguous record per
+// tile (rec_cfg.h): the ten lower 16 x 16 blocks of A as bf16 hi + lo in the
+// lane order of the recurrence kernels' MFMA operands, the gates, their
+// factors and beta.  That is 11 KiB against the 16 KiB of A rows (whose upper
+// blocks are zero), 1 KiB runs instead of 256-byte rows H x 256 bytes apart,
+// no cumsum launch, and nothing left to convert in the recurrence's serial
+// chain.
 #include <type_traits>
 
+#include "gate.h"
 #include "h_layout.h"
+#include "rec_cfg.h"
 #include "wy_blocks.h"
 
 namespace thm {
@@ -58,10 +70,42 @@ __device__ __forceinline__ void store_A(const float* Xb, float* out, int64_t H) 
   }
 }
 
-template <typename IT, int K, int SIGN>
+// The tile's record from the inverted blocks Xb and sb, sg (beta, g).
+__device__ __forceinline__ void store_rec(const float* Xb, const float* sb, const float* sg, char* out, int wv) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int p = wv + 4 * i;
+    if (p < rec::kBlocks) {  // wave-uniform
+      *reinterpret_cast<u32x4*>(out + p * rec::kBlockBytes + 16 * lane) = hi_lo4(wy::block_row4(Xb + p * kBlk));
+    }
+  }
+  if (wv == 3) {
+    float* const gp = reinterpret_cast<float*>(out + rec::kGateOff);
+    const float g = sg[lane];
+    gp[rec::kG + lane] = g;
+    gp[rec::kEg + lane] = fast_exp(g);
+    gp[rec::kEgl + lane] = fast_exp(sg[kBT - 1] - g);
+    gp[rec::kBeta + lane] = sb[lane];
+  }
+}
+
+// Raw gate value of one token-head (row = its index in [B, T, H]); 0 without a gate.
+__device__ __forceinline__ float load_gate(const void* p, int mode, int64_t row) {
+  if (mode == rec::kGateNone) return 0.f;
+  if (mode & rec::kGateBf16) return (float)reinterpret_cast<const bf16*>(p)[row];
+  return reinterpret_cast<const float*>(p)[row];
+}
+// The chunk's cumulative gates from its raw values, one token per lane.
+__device__ __forceinline__ float form_gate(float x, int mode) {
+  if (mode & rec::kGateLogsigmoid) x = logsigmoid(x);
+  return mode & rec::kGatePerToken ? wave_inclusive_sum(x) : x;
+}
+
+template <typename IT, int K, int SIGN, bool REC>
 __global__ void __launch_bounds__(kABThreads)
 wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
-                  const float* __restrict__ g, float* __restrict__ A, int64_t T, int64_t H,
+                  const void* __restrict__ g, int gate_mode, void* __restrict__ out, int64_t T, int64_t H,
                   int64_t NT) {
   constexpr bool kSplit = std::is_same<IT, float>::value;
   constexpr int KS = K / 32;  // contraction steps
@@ -97,7 +141,7 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
   }
   if (tid < kBT) {
     sb[tid] = beta[(tok0 + tid) * H + h];
-    sg[tid] = g ? g[(tok0 + tid) * H + h] : 0.f;
+    sg[tid] = form_gate(load_gate(g, gate_mode, (tok0 + tid) * H + h), gate_mode);
   }
   lds_barrier();
 
@@ -106,8 +150,9 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
   lds_barrier();
   wy::invert_L(Lb, Xb, wv);
 
-  // 5. A_c rows.
-  store_A(Xb, A + (tok0 * H + h) * kBT, H);
+  // 5. A_c rows, or the record.
+  if constexpr (REC) store_rec(Xb, sb, sg, reinterpret_cast<char*>(out) + rec::offset(tc.b * H + h, tc.c, NT), wv);
+  else store_A(Xb, reinterpret_cast<float*>(out) + (tok0 * H + h) * kBT, H);
 }
 
 // ---------------------------------------------------------------------------
@@ -133,10 +178,10 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
 template <int K>
 constexpr int ab_pipe_wgs_per_cu() { return 4; }
 
-template <int K, int SIGN>
+template <int K, int SIGN, bool REC>
 __global__ void __launch_bounds__(kABThreads, ab_pipe_wgs_per_cu<K>())
 wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ beta,
-                       const float* __restrict__ g, float* __restrict__ A, int64_t T, int64_t H,
+                       const void* __restrict__ g, int gate_mode, void* __restrict__ out, int64_t T, int64_t H,
                        int64_t NT, int64_t tiles) {
   constexpr int KS = K / 32;
   // bf16 elements per k row: a 32-byte pad (h_layout.h tr_pitch), under which
@@ -167,24 +212,20 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
   // per XCD.  Measured traffic 1.108 -> 1.00 of the algorithmic bytes, at
   // +1.4 % time (115.2 -> 116.8 us at config 4, A bit-identical).
   const int64_t BNT = tiles / H;
-  auto tok_of = [&](int64_t tile, int64_t& h) {
-    const TileCoord tc = tile_coord(hl::xcd_tile_order((uint32_t)tile, H, BNT), H, NT, T);
-    h = tc.hh;
-    return tc.tok0;
-  };
+  auto coord = [&](int64_t tile) { return tile_coord(hl::xcd_tile_order((uint32_t)tile, H, BNT), H, NT, T); };
   u32x4 kr[kLoads];
   float br = 0.f, gr = 0.f;
   const uint32_t k_off = hl::o_blk_lane(tid, K, H * K);
   auto prefetch = [&](int64_t tile) {
-    int64_t h;
-    const int64_t tok0 = tok_of(tile, h);
+    const TileCoord tc = coord(tile);
+    const int64_t h = tc.hh, tok0 = tc.tok0;
     const char* const kb = reinterpret_cast<const char*>(k + (tok0 * H + h) * K);
 #pragma unroll
     for (int it = 0; it < kLoads; ++it) kr[it] = ldg16_nt(kb + hl::o_blk_step(it, K, H * K) + k_off);
     if (tid < kBT) {
       const int64_t row = (tok0 + tid) * H + h;
       br = beta[row];
-      gr = g ? g[row] : 0.f;
+      gr = load_gate(g, gate_mode, row);
     }
   };
   auto stage = [&]() {
@@ -196,7 +237,7 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
     }
     if (tid < kBT) {
       sb[tid] = br;
-      sg[tid] = gr;
+      sg[tid] = form_gate(gr, gate_mode);
     }
   };
 
@@ -213,13 +254,13 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
   for (;;) {
     const int64_t tn = t + gridDim.x;
     if (tn < tiles) prefetch(tn);  // in flight while tile t computes
-    int64_t h;
-    const int64_t tok0 = tok_of(t, h);
+    const TileCoord tc = coord(t);
     wy::form_L_lds<SIGN, KS>([&](int tb, int s) { return load8(ks + (16 * tb + li) * kPitch + 32 * s + 8 * grp); },
                              sb, sg, Lb, wv);
     lds_barrier();  // every wave's k fragment reads are done: X may overwrite ks
     wy::invert_L(Lb, Xb, role);  // ends with a barrier
-    store_A(Xb, A + (tok0 * H + h) * kBT, H);
+    if constexpr (REC) store_rec(Xb, sb, sg, reinterpret_cast<char*>(out) + rec::offset(tc.b * H + tc.hh, tc.c, NT), wv);
+    else store_A(Xb, reinterpret_cast<float*>(out) + (tc.tok0 * H + tc.hh) * kBT, H);
 
     if (tn >= tiles) break;
     lds_barrier();  // every wave is done with tile t's LDS
@@ -229,34 +270,41 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
   }
 }
 
-template <typename IT, int K>
-hipError_t launch_A(const void* k, const void* beta, const void* g, void* A, int64_t B, int64_t T,
-                    int64_t H, int sign, hipStream_t s) {
+template <typename IT, int K, int SIGN, bool REC>
+hipError_t launch_A(const void* k, const void* beta, const void* g, int gate_mode, void* out, int64_t B,
+                    int64_t T, int64_t H, hipStream_t s) {
   const int64_t NT = T / kBT;
   const int64_t tiles = B * NT * H;
   if constexpr (std::is_same<IT, bf16>::value) {
     const int64_t pgrid = (int64_t)device_cu_count() * ab_pipe_wgs_per_cu<K>();
     if (pgrid > 0 && tiles >= 2 * pgrid) {
-      if (sign < 0)
-        hipLaunchKernelGGL((wy_build_A_pipe_kernel<K, -1>), dim3((unsigned)pgrid), dim3(kABThreads), 0, s,
-                           (const bf16*)k, (const float*)beta, (const float*)g, (float*)A, T, H, NT, tiles);
-      else
-        hipLaunchKernelGGL((wy_build_A_pipe_kernel<K, 1>), dim3((unsigned)pgrid), dim3(kABThreads), 0, s,
-                           (const bf16*)k, (const float*)beta, (const float*)g, (float*)A, T, H, NT, tiles);
+      hipLaunchKernelGGL((wy_build_A_pipe_kernel<K, SIGN, REC>), dim3((unsigned)pgrid), dim3(kABThreads), 0, s,
+                         (const bf16*)k, (const float*)beta, g, gate_mode, out, T, H, NT, tiles);
       return hipGetLastError();
     }
   }
-  const dim3 grid((unsigned)tiles);
-  if (sign < 0)
-    hipLaunchKernelGGL((wy_build_A_kernel<IT, K, -1>), grid, dim3(kABThreads), 0, s, (const IT*)k,
-                       (const float*)beta, (const float*)g, (float*)A, T, H, NT);
-  else
-    hipLaunchKernelGGL((wy_build_A_kernel<IT, K, 1>), grid, dim3(kABThreads), 0, s, (const IT*)k,
-                       (const float*)beta, (const float*)g, (float*)A, T, H, NT);
+  hipLaunchKernelGGL((wy_build_A_kernel<IT, K, SIGN, REC>), dim3((unsigned)tiles), dim3(kABThreads), 0, s,
+                     (const IT*)k, (const float*)beta, g, gate_mode, out, T, H, NT);
   return hipGetLastError();
 }
 
+template <typename IT, int K>
+hipError_t launch_A_sign(const void* k, const void* beta, const void* g, void* A, int64_t B, int64_t T, int64_t H,
+                         int sign, hipStream_t s) {
+  const int mode = g ? rec::kGateCumulative : rec::kGateNone;
+  return sign < 0 ? launch_A<IT, K, -1, false>(k, beta, g, mode, A, B, T, H, s)
+                  : launch_A<IT, K, 1, false>(k, beta, g, mode, A, B, T, H, s);
+}
+
 }  // namespace
+
+__attribute__((visibility("hidden"))) hipError_t build_records(int64_t K, const void* k, const void* beta,
+                                                               const void* gate, int gate_mode, void* records,
+                                                               int64_t B, int64_t T, int64_t H, hipStream_t s) {
+  return K == 64 ? launch_A<bf16, 64, 1, true>(k, beta, gate, gate_mode, records, B, T, H, s)
+                 : launch_A<bf16, 128, 1, true>(k, beta, gate, gate_mode, records, B, T, H, s);
+}
+
 }  // namespace thm
 
 extern "C" int thm_wy_build_A(const void* k, const void* beta, const void* g, void* A, int64_t B,
@@ -279,10 +327,10 @@ extern "C" int thm_wy_build_A(const void* k, const void* beta, const void* g, vo
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (k_dtype == THM_DTYPE_F32)
-    e = (K == 64) ? launch_A<float, 64>(k, beta, g, A, B, T, H, sign, s)
-                  : launch_A<float, 128>(k, beta, g, A, B, T, H, sign, s);
+    e = (K == 64) ? launch_A_sign<float, 64>(k, beta, g, A, B, T, H, sign, s)
+                  : launch_A_sign<float, 128>(k, beta, g, A, B, T, H, sign, s);
   else
-    e = (K == 64) ? launch_A<bf16, 64>(k, beta, g, A, B, T, H, sign, s)
-                  : launch_A<bf16, 128>(k, beta, g, A, B, T, H, sign, s);
+    e = (K == 64) ? launch_A_sign<bf16, 64>(k, beta, g, A, B, T, H, sign, s)
+                  : launch_A_sign<bf16, 128>(k, beta, g, A, B, T, H, sign, s);
   return (int)e;
 }

@@ -24,6 +24,9 @@ THM_DTYPE = {torch.float32: 0, torch.bfloat16: 1}
 THM_ACT_NONE = 0
 THM_ACT_SILU = 1
 THM_H_DELTA = 1
+THM_GATE_IDENTITY = 0
+THM_GATE_LOGSIGMOID = 1
+THM_GATE_CUMULATIVE = 2
 
 _c_vp = ctypes.c_void_p
 _c_i64 = ctypes.c_int64
@@ -47,12 +50,14 @@ SIGNATURES = {
                         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_vp],
     "thm_chunk_gated_delta_fwd": [_c_vp] * 9 + [ctypes.c_float] + [_c_i64] * 5 + [_c_i32, _c_i32, _c_vp],
     "thm_chunk_gated_delta_fwd_a": [_c_vp] * 10 + [ctypes.c_float] + [_c_i64] * 5 + [_c_i32, _c_i32, _c_vp],
+    "thm_chunk_gated_delta_rule_workspace": [_c_i64] * 5,
+    "thm_chunk_gated_delta_rule_fwd": [_c_vp] * 9 + [_c_i64, ctypes.c_float] + [_c_i64] * 5 + [_c_i32] * 4 + [_c_vp],
     "thm_wy_build_A": [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64,
                        _c_i32, _c_i32, _c_i32, _c_vp],
     "thm_chunk_local_cumsum": [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_vp],
     "thm_wy_fwd": [_c_vp] * 6 + [_c_i64] * 5 + [_c_i32, _c_i32, _c_i32, _c_vp],
 }
-_RESTYPES = {"thm_status_string": ctypes.c_char_p}
+_RESTYPES = {"thm_status_string": ctypes.c_char_p, "thm_chunk_gated_delta_rule_workspace": _c_i64}
 
 _lib = None
 _lock = threading.Lock()
