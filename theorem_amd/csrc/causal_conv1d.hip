@@ -15,8 +15,19 @@
 //     registers: they are passed with a DPP whole-wave shift (wave_shr:1), and
 //     lane 0 takes lane 63's value of the previous group (v_readlane).  Only the
 //     W-1 elements before each segment are re-read (wave-uniform loads).
+//   * Rows whose length is no multiple of VEC (RAGGED) start anywhere in a
+//     16-byte vector.  x and out share that offset, so a segment still walks
+//     whole aligned vectors, from `off` elements before the row:
+//     only the vectors at the two ends of a row hold elements of its
+//     neighbours, which are read as zero and not written.  [4, 4096, 4003] bf16
+//     with SiLU: element by element (2-byte lanes) 157 us, in whole vectors
+//     from the row's first 16 bytes 63, from its first 128-byte line (no split
+//     line between a segment's stores) 59, with silu()'s reciprocal 49;
+//     [8, 4096, 8191] 173, as 8192.
 //   * Weights and bias are wave-uniform; accumulation is fp32 FMA.
 //   * Stores are non-temporal: the output is not re-read by this kernel.
+#include <type_traits>
+
 #include "common.h"
 
 namespace thm {
@@ -50,7 +61,7 @@ __device__ __forceinline__ float load_param(const void* p, int64_t i) {
   return to_f32(reinterpret_cast<const WT*>(p)[i]);
 }
 
-template <typename XT, typename WT, int VEC, int W, int NV>
+template <typename XT, typename WT, int VEC, int W, int NV, bool RAGGED>
 __global__ void __launch_bounds__(kConvWaves * kWave)
 causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
                      const void* __restrict__ bias, XT* __restrict__ out, int64_t n_rows,
@@ -66,11 +77,22 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
   const int64_t seg = (int64_t)blockIdx.x * kConvWaves + wave;
   if (seg >= n_rows * segs_per_row) return;  // wave-uniform exit
   const int64_t row = seg / segs_per_row;
-  const int64_t s0 = (seg - row * segs_per_row) * SEG;
+  // First position of the segment in its row (RAGGED: the row's first 128-byte
+  // line starts `off` elements before it, so the segments cover whole lines).
+  constexpr int kLine = 128 / (int)sizeof(XT);
+  const int64_t off = RAGGED ? (row * seqlen) & (kLine - 1) : 0;
+  const int64_t s0 = (seg - row * segs_per_row) * SEG - off;
+  if (RAGGED && s0 >= seqlen) return;  // past this row's end (wave-uniform)
   const int64_t d = row % dim;
 
   const XT* __restrict__ xr = x + row * seqlen;
   XT* __restrict__ orow = out + row * seqlen;
+
+  // RAGGED: whether the segment holds an end of the row, and the row's
+  // elements [first_in, end_in) of the vector at e0.
+  const bool ends = s0 < 0 || s0 + SEG > seqlen;
+  auto first_in = [&](int64_t e0) { return e0 < 0 ? (int)-e0 : 0; };  // VEC or more: none
+  auto end_in = [&](int64_t e0) { return seqlen - e0 >= VEC ? VEC : seqlen > e0 ? (int)(seqlen - e0) : 0; };
 
   float cur[NV][VEC];   // this lane's vectors
   float halo[PA][VEC];  // vectors just left of the segment (stream index -1-q), wave-uniform
@@ -80,10 +102,15 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
     // the P vectors left of the segment (uniform; none for the row's first
     // segment, where they are the causal zero padding).
     u32x4 raw[NV], hraw[PA];
+    // RAGGED, last row: the vector that holds the row's end may reach past the
+    // tensor; that lane loads its elements one by one.  (A vector holds one end
+    // of a row at most: rows are longer than a vector.)
+    const bool past = RAGGED && row == n_rows - 1 && ((row + 1) * seqlen & (VEC - 1)) != 0;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int64_t e0 = s0 + (int64_t)(j * kWave + lane) * VEC;
-      raw[j] = ldg16_nt(xr + (e0 < seqlen ? e0 : 0));
+      const int64_t end = past ? seqlen - VEC + 1 : seqlen;
+      raw[j] = ldg16_nt(xr + (e0 < end && e0 > -VEC ? e0 : -(off & (VEC - 1))));
     }
 #pragma unroll
     for (int q = 0; q < PA; ++q) {
@@ -94,7 +121,18 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
     for (int j = 0; j < NV; ++j) {
       const int64_t e0 = s0 + (int64_t)(j * kWave + lane) * VEC;
       unpack16(raw[j], cur[j], XT{});
-      if (e0 >= seqlen) {
+      if constexpr (RAGGED) {
+        if (ends) {
+          const int lo = first_in(e0), hi = end_in(e0);
+          if (past && lo == 0 && hi > 0 && hi < VEC) {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) cur[j][i] = i < hi ? to_f32(xr[e0 + i]) : 0.f;
+          }
+#pragma unroll
+          for (int i = 0; i < VEC; ++i)
+            if (i < lo || i >= hi) cur[j][i] = 0.f;
+        }
+      } else if (e0 >= seqlen) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) cur[j][i] = 0.f;
       }
@@ -169,35 +207,47 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
         }
         acc = __builtin_fmaf(wk[k], xv, acc);
       }
-      if (act == THM_ACT_SILU) acc = acc / (1.f + fast_exp(-acc));
+      if (act == THM_ACT_SILU) acc = silu<XT>(acc);
       res[v] = acc;
     }
     const int64_t e0 = s0 + (int64_t)(j * kWave + lane) * VEC;
-    if (e0 < seqlen) store_vec<XT, VEC>(orow + e0, res);
+    if constexpr (RAGGED) {
+      const int lo = first_in(e0), hi = end_in(e0);
+      if (lo == 0 && hi == VEC) {
+        store_vec<XT, VEC>(orow + e0, res);
+      } else {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i)
+          if (i >= lo && i < hi) orow[e0 + i] = from_f32<XT>(res[i]);
+      }
+    } else if (e0 < seqlen) {
+      store_vec<XT, VEC>(orow + e0, res);
+    }
   }
 }
 
-template <typename XT, typename WT, int VEC, int W>
+template <typename XT, typename WT, int VEC, int W, bool RAGGED>
 hipError_t launch_conv(const void* x, const void* weight, const void* bias, void* out,
                        int64_t n_rows, int64_t dim, int64_t seqlen, int act, hipStream_t stream) {
   constexpr int SEG = kConvNV * kWave * VEC;
-  const int64_t segs_per_row = (seqlen + SEG - 1) / SEG;
+  // With the largest offset (a segment past a row's end does nothing).
+  const int64_t segs_per_row = (seqlen + (RAGGED ? 128 / (int)sizeof(XT) - 1 : 0) + SEG - 1) / SEG;
   const int64_t n_seg = n_rows * segs_per_row;
   const int64_t blocks = (n_seg + kConvWaves - 1) / kConvWaves;
-  hipLaunchKernelGGL((causal_conv1d_kernel<XT, WT, VEC, W, kConvNV>), dim3((unsigned)blocks),
+  hipLaunchKernelGGL((causal_conv1d_kernel<XT, WT, VEC, W, kConvNV, RAGGED>), dim3((unsigned)blocks),
                      dim3(kConvWaves * kWave), 0, stream, (const XT*)x, weight, bias, (XT*)out,
                      n_rows, dim, seqlen, segs_per_row, act);
   return hipGetLastError();
 }
 
-template <typename XT, int VEC, typename WT>
+template <typename XT, int VEC, bool RAGGED, typename WT>
 hipError_t dispatch_width_w(int width, const void* x, const void* weight, const void* bias,
                             void* out, int64_t n_rows, int64_t dim, int64_t seqlen, int act,
                             hipStream_t s) {
   switch (width) {
 #define THM_CONV_W(WV)                                                                           \
   case WV:                                                                                       \
-    return launch_conv<XT, WT, VEC, WV>(x, weight, bias, out, n_rows, dim, seqlen, act, s);
+    return launch_conv<XT, WT, VEC, WV, RAGGED>(x, weight, bias, out, n_rows, dim, seqlen, act, s);
     THM_CONV_W(1)
     THM_CONV_W(2)
     THM_CONV_W(3)
@@ -212,12 +262,12 @@ hipError_t dispatch_width_w(int width, const void* x, const void* weight, const 
   }
 }
 
-template <typename XT, int VEC>
+template <typename XT, int VEC, bool RAGGED>
 hipError_t dispatch_width(int width, const void* x, const void* weight, const void* bias,
                           void* out, int64_t n_rows, int64_t dim, int64_t seqlen, int w_is_bf16,
                           int act, hipStream_t s) {
-  return w_is_bf16 ? dispatch_width_w<XT, VEC, bf16>(width, x, weight, bias, out, n_rows, dim, seqlen, act, s)
-                   : dispatch_width_w<XT, VEC, float>(width, x, weight, bias, out, n_rows, dim, seqlen, act, s);
+  return w_is_bf16 ? dispatch_width_w<XT, VEC, RAGGED, bf16>(width, x, weight, bias, out, n_rows, dim, seqlen, act, s)
+                   : dispatch_width_w<XT, VEC, RAGGED, float>(width, x, weight, bias, out, n_rows, dim, seqlen, act, s);
 }
 
 }  // namespace
@@ -247,21 +297,22 @@ extern "C" int thm_causal_conv1d_fwd(const void* x, const void* weight, const vo
   if (!launch_fits((n_rows * ((seqlen + 255) / 256) + kConvWaves - 1) / kConvWaves, kConvWaves * kWave))
     return THM_ERR_BAD_SHAPE;
   const int vec = (int)(16 / xe);
-  // 16-byte vectors need every row start 16-byte aligned.
-  const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && (seqlen % vec == 0);
+  // 16-byte vectors need x and out 16-byte aligned; rows that are no multiple
+  // of a vector take the ragged form of the same kernel, which needs rows longer
+  // than a vector (from 64 elements on; below that a row is one wave of scalar
+  // lanes anyway).
+  const bool whole = seqlen % vec == 0;
+  const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && (whole || seqlen >= 64);
   const int wb = (w_dtype == THM_DTYPE_BF16);
   hipStream_t s = (hipStream_t)stream;
-  hipError_t e;
-  if (x_dtype == THM_DTYPE_F32) {
-    e = vec_ok ? dispatch_width<float, 4>(width, x, weight, bias, out, n_rows, dim, seqlen, wb,
-                                          activation, s)
-               : dispatch_width<float, 1>(width, x, weight, bias, out, n_rows, dim, seqlen, wb,
-                                          activation, s);
-  } else {
-    e = vec_ok ? dispatch_width<bf16, 8>(width, x, weight, bias, out, n_rows, dim, seqlen, wb,
-                                         activation, s)
-               : dispatch_width<bf16, 1>(width, x, weight, bias, out, n_rows, dim, seqlen, wb,
-                                         activation, s);
-  }
+  auto run = [&](auto xt, auto vec_c) {
+    using XT = decltype(xt);
+    constexpr int VEC = decltype(vec_c)::value;
+    if (!vec_ok) return dispatch_width<XT, 1, false>(width, x, weight, bias, out, n_rows, dim, seqlen, wb, activation, s);
+    return whole ? dispatch_width<XT, VEC, false>(width, x, weight, bias, out, n_rows, dim, seqlen, wb, activation, s)
+                 : dispatch_width<XT, VEC, true>(width, x, weight, bias, out, n_rows, dim, seqlen, wb, activation, s);
+  };
+  const hipError_t e = x_dtype == THM_DTYPE_F32 ? run(float{}, std::integral_constant<int, 4>{})
+                                                : run(bf16{}, std::integral_constant<int, 8>{});
   return (int)e;
 }

@@ -5,10 +5,13 @@
 // 1. Channels-last layout: x, out [B, S, D] with D contiguous (the layout of a
 //    [B, D, S] tensor that is a transposed view of [B, S, D]).  Vectors run
 //    along D: a lane owns VEC channels (one 16-byte vector) and walks a segment
-//    of kClSeg timesteps, keeping the last W-1 input vectors of its channels in
+//    of timesteps, keeping the last W-1 input vectors of its channels in
 //    registers; only the W-1 rows before each segment are read twice.  A
 //    wavefront reads and writes 1 KiB of one row per step, and x and out are
-//    streamed once.
+//    streamed once.  Bound by memory at large sizes (5.6 TB/s) and by the
+//    steps' arithmetic at smaller ones: [2, 5001, 4352] bf16 with SiLU 47.7 ->
+//    37.4 us (whole lanes, whole segments, no IEEE division; 64-step segments
+//    throughout and a step-by-step tail before).
 //
 // 2. Decode step (rolling state): for each (b, d), with state s[0..L_s) and
 //    the new samples x[0..L):  window = s ++ x,
@@ -16,15 +19,21 @@
 //    and the state becomes the last L_s samples of the window (in place).
 //    One lane per (b, d); a decode step moves a few bytes per channel, so this
 //    is latency-, not bandwidth-, bound.
+#include <algorithm>
+
 #include "common.h"
 
 namespace thm {
 namespace {
 
 constexpr int kClThreads = 256;
-constexpr int kClSeg = 64;  // timesteps per lane
+constexpr int kClSeg = 64;  // timesteps per lane, at most
 
-constexpr int kClDepth = 16;  // time steps whose loads are in flight ahead of use
+// Time steps whose loads are in flight ahead of use (16 KiB or less per wave;
+// 16 steps of bf16 lanes take 193 VGPRs against 134, 38.5 against 37.4 us at
+// [2, 5001, 4352], and 8 steps of fp32 lanes 94 against 84 at [4, 2500, 5120]).
+template <typename XT>
+constexpr int cl_depth() { return sizeof(XT) == 2 ? 8 : 16; }
 
 __device__ __forceinline__ float conv_param(const void* p, int64_t i, int is_bf16) {
   return is_bf16 ? (float)reinterpret_cast<const bf16*>(p)[i] : reinterpret_cast<const float*>(p)[i];
@@ -55,33 +64,34 @@ __device__ __forceinline__ void cl_store(XT* p, const float* v) {
   }
 }
 
-template <typename XT, typename WT, int VEC, int W, bool SILU>
+// One lane per (b, segment, channel group), channel group fastest, so a
+// wavefront's lanes stay full whatever the channel count.  BLOCKS: segments of
+// `seg` steps, a multiple of cl_depth, in blocks of cl_depth steps whose loads
+// are in flight a block ahead of use.  The last segment of a sequence starts early enough to be
+// whole and writes only the steps that are its own, so a ragged length costs
+// no step-by-step tail (whose loads each wait for memory).  Otherwise: steps
+// one by one (scalar lanes, and sequences shorter than a block).
+template <typename XT, typename WT, int VEC, int W, bool SILU, bool BLOCKS>
 __global__ void __launch_bounds__(kClThreads)
 causal_conv1d_cl_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
                         const void* __restrict__ bias, XT* __restrict__ out, int64_t seqlen,
-                        int64_t dim, int64_t groups, int64_t blocks_per_seg, int64_t segs) {
-  const int64_t blk = blockIdx.x;
-  const int64_t cb = blk % blocks_per_seg;
-  const int64_t bs = blk / blocks_per_seg;
-  const int64_t seg = bs % segs, b = bs / segs;
-  const int64_t cg = cb * kClThreads + threadIdx.x;  // channel group
-  if (cg >= groups) return;                           // no barriers follow
-  const int64_t d0 = cg * VEC;
-  const int64_t t0 = seg * kClSeg;
-  const int64_t tend = (t0 + kClSeg < seqlen) ? t0 + kClSeg : seqlen;
+                        int64_t dim, int seg, uint32_t groups, uint32_t segs, uint32_t items) {
+  const uint32_t item = blockIdx.x * kClThreads + threadIdx.x;
+  if (item >= items) return;  // no barriers follow
+  const uint32_t bs = item / groups, cg = item - bs * groups;
+  const uint32_t b = bs / segs;
+  const int64_t d0 = (int64_t)cg * VEC;
+  const int64_t own = (int64_t)(bs - b * segs) * seg;  // first step this lane writes
+  const int64_t tend = (own + seg < seqlen) ? own + seg : seqlen;
+  const int64_t t0 = BLOCKS ? tend - seg : own;
 
   const XT* __restrict__ xb = x + b * seqlen * dim + d0;
   XT* __restrict__ ob = out + b * seqlen * dim + d0;
-  // A whole segment of 16-byte vectors runs as straight-line code with
-  // kClDepth loads in flight ahead of use (no loop, so the compiler's wait
-  // counts stay exact); a partial last segment, or scalar lanes, loop.
-  const bool pipelined = VEC * sizeof(XT) == 16 && tend - t0 == kClSeg;
-  u32x4 pf[kClDepth];
-  if constexpr (VEC * sizeof(XT) == 16) {
-    if (pipelined) {
+  constexpr int kDepth = cl_depth<XT>();
+  u32x4 pf[kDepth];
+  if constexpr (BLOCKS) {
 #pragma unroll
-      for (int i = 0; i < kClDepth; ++i) pf[i] = ldg16_nt(xb + (t0 + i) * dim);
-    }
+    for (int i = 0; i < kDepth; ++i) pf[i] = ldg16_nt(xb + (t0 + i) * dim);
   }
   // win[k] = input at t - (W-1) + k for k < W-1 (zero before t = 0): loaded
   // from a clamped row, then zeroed, so every load is issued before any use.
@@ -110,7 +120,9 @@ causal_conv1d_cl_kernel(const XT* __restrict__ x, const void* __restrict__ weigh
     for (int v = 0; v < VEC; ++v) bv[v] = 0.f;
   }
 
-  auto step = [&](int64_t t, const float* cur) {
+  const int skip = (int)(own - t0);  // steps of the previous segment's lane
+  XT* op = ob + t0 * dim;
+  auto step = [&](int j, const float* cur) {
     float res[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
@@ -118,10 +130,11 @@ causal_conv1d_cl_kernel(const XT* __restrict__ x, const void* __restrict__ weigh
 #pragma unroll
       for (int k = 0; k < W - 1; ++k) acc = __builtin_fmaf(wk[k][v], win[k][v], acc);
       acc = __builtin_fmaf(wk[W - 1][v], cur[v], acc);
-      if constexpr (SILU) acc = acc / (1.f + fast_exp(-acc));
+      if constexpr (SILU) acc = silu<XT>(acc);
       res[v] = acc;
     }
-    cl_store<XT, VEC>(ob + t * dim, res);
+    if (!BLOCKS || j >= skip) cl_store<XT, VEC>(op, res);
+    op += dim;
 #pragma unroll
     for (int k = 0; k + 1 < W - 1; ++k)
 #pragma unroll
@@ -132,43 +145,50 @@ causal_conv1d_cl_kernel(const XT* __restrict__ x, const void* __restrict__ weigh
     }
   };
 
-  if constexpr (VEC * sizeof(XT) == 16) {
-    if (pipelined) {
+  if constexpr (BLOCKS) {
+    const XT* xp = xb + (t0 + kDepth) * dim;
+    int j = 0;
+    for (; j + kDepth < seg; j += kDepth) {
 #pragma unroll
-      for (int i = 0; i < kClSeg; ++i) {
+      for (int i = 0; i < kDepth; ++i) {
         float cur[VEC];
-        unpack16(pf[i % kClDepth], cur, XT{});
-        if (i + kClDepth < kClSeg) pf[i % kClDepth] = ldg16_nt(xb + (t0 + i + kClDepth) * dim);
-        step(t0 + i, cur);
+        unpack16(pf[i], cur, XT{});
+        pf[i] = ldg16_nt(xp);
+        xp += dim;
+        step(j + i, cur);
       }
-      return;
     }
-  }
-  for (int64_t t = t0; t < tend; ++t) {
-    float cur[VEC];
-    cl_load<XT, VEC>(xb + t * dim, cur);
-    step(t, cur);
+#pragma unroll
+    for (int i = 0; i < kDepth; ++i) {
+      float cur[VEC];
+      unpack16(pf[i], cur, XT{});
+      step(j + i, cur);
+    }
+  } else {
+    const int n = (int)(tend - t0);
+    for (int j = 0; j < n; ++j) {
+      float cur[VEC];
+      cl_load<XT, VEC>(xb + (t0 + j) * dim, cur);
+      step(j, cur);
+    }
   }
 }
 
-template <typename XT, typename WT, int VEC>
-hipError_t launch_cl_w(int width, const void* x, const void* weight, const void* bias, void* out,
+template <typename XT, typename WT, int VEC, bool BLOCKS>
+hipError_t launch_cl_w(int width, int seg, const void* x, const void* weight, const void* bias, void* out,
                        int64_t batch, int64_t seqlen, int64_t dim, int act, hipStream_t s) {
-  const int64_t groups = dim / VEC;
-  const int64_t blocks_per_seg = (groups + kClThreads - 1) / kClThreads;
-  const int64_t segs = (seqlen + kClSeg - 1) / kClSeg;
-  const dim3 grid((unsigned)(batch * segs * blocks_per_seg));
+  const int64_t groups = dim / VEC, segs = (seqlen + seg - 1) / seg;
+  const int64_t items = batch * segs * groups;
+  const dim3 grid((unsigned)((items + kClThreads - 1) / kClThreads));
+#define THM_CL_LAUNCH(WV, SL)                                                                             \
+  hipLaunchKernelGGL((causal_conv1d_cl_kernel<XT, WT, VEC, WV, SL, BLOCKS>), grid, dim3(kClThreads), 0, s,   \
+                     (const XT*)x, weight, bias, (XT*)out, seqlen, dim, seg, (uint32_t)groups,             \
+                     (uint32_t)segs, (uint32_t)items)
   switch (width) {
-#define THM_CL_W(WV)                                                                          \
-  case WV:                                                                                    \
-    if (act == THM_ACT_SILU)                                                                       \
-      hipLaunchKernelGGL((causal_conv1d_cl_kernel<XT, WT, VEC, WV, true>), grid, dim3(kClThreads), 0, \
-                         s, (const XT*)x, weight, bias, (XT*)out, seqlen, dim, groups,             \
-                         blocks_per_seg, segs);                                                    \
-    else                                                                                           \
-      hipLaunchKernelGGL((causal_conv1d_cl_kernel<XT, WT, VEC, WV, false>), grid, dim3(kClThreads), 0,\
-                         s, (const XT*)x, weight, bias, (XT*)out, seqlen, dim, groups,             \
-                         blocks_per_seg, segs);                                                    \
+#define THM_CL_W(WV)                                     \
+  case WV:                                               \
+    if (act == THM_ACT_SILU) THM_CL_LAUNCH(WV, true);    \
+    else THM_CL_LAUNCH(WV, false);                       \
     break;
     THM_CL_W(1)
     THM_CL_W(2)
@@ -179,17 +199,30 @@ hipError_t launch_cl_w(int width, const void* x, const void* weight, const void*
     THM_CL_W(7)
     THM_CL_W(8)
 #undef THM_CL_W
+#undef THM_CL_LAUNCH
     default:
       return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-template <typename XT, int VEC>
-hipError_t launch_cl(int width, const void* x, const void* weight, const void* bias, void* out,
-                     int64_t batch, int64_t seqlen, int64_t dim, int wb, int act, hipStream_t s) {
-  return wb ? launch_cl_w<XT, bf16, VEC>(width, x, weight, bias, out, batch, seqlen, dim, act, s)
-            : launch_cl_w<XT, float, VEC>(width, x, weight, bias, out, batch, seqlen, dim, act, s);
+template <typename XT, typename WT>
+hipError_t launch_cl(bool vec_ok, int width, const void* x, const void* weight, const void* bias, void* out,
+                     int64_t batch, int64_t seqlen, int64_t dim, int act, hipStream_t s) {
+  constexpr int VEC = 16 / (int)sizeof(XT);
+  if (!vec_ok) return launch_cl_w<XT, WT, 1, false>(width, kClSeg, x, weight, bias, out, batch, seqlen, dim, act, s);
+  constexpr int kDepth = cl_depth<XT>();
+  if (seqlen < kDepth) return launch_cl_w<XT, WT, VEC, false>(width, kClSeg, x, weight, bias, out, batch, seqlen, dim, act, s);
+  // Longest segments that leave every SIMD a few waves (each segment re-reads
+  // W - 1 steps; a lane's steps run one after another): 2 for bf16, 4 for fp32,
+  // whose lanes hold half the channels.  us at segments of 8 / 16 / 32 / 64:
+  // bf16 [8, 8192, 4096] 209 / 214 / 196 / 190, [2, 5001, 4352] 42 / 39 / 37 /
+  // 44, [1, 1000, 4352] 8.7 / 8.4 / 11.8 / 19.6; fp32 [4, 2500, 5120] - / 88 /
+  // 84 / 90.
+  const int64_t waves = (int64_t)std::max(device_cu_count(), 1) * 4 * (sizeof(XT) == 2 ? 2 : 4);
+  int seg = kClSeg;
+  while (seg > kDepth && (seg > seqlen || batch * ((seqlen + seg - 1) / seg) * (dim / VEC) < waves * kWave)) seg /= 2;
+  return launch_cl_w<XT, WT, VEC, true>(width, seg, x, weight, bias, out, batch, seqlen, dim, act, s);
 }
 
 template <typename XT>
@@ -214,7 +247,7 @@ causal_conv1d_update_kernel(const XT* __restrict__ x, XT* __restrict__ state,
     float acc = b0;
     const int64_t base = state_len - (width - 1) + t;
     for (int k = 0; k < width; ++k) acc = __builtin_fmaf(wk[k], at(base + k), acc);
-    if (act == THM_ACT_SILU) acc = acc / (1.f + fast_exp(-acc));
+    if (act == THM_ACT_SILU) acc = silu<XT>(acc);
     orow[t] = from_f32<XT>(acc);
   }
   // New state: the last L_s window samples, written front to back (the
@@ -259,17 +292,18 @@ extern "C" int thm_causal_conv1d_fwd_channels_last(const void* x, const void* we
   const int vec = (int)(16 / xe);
   const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && (dim % vec == 0);
   const int64_t groups = vec_ok ? dim / vec : dim;
+  // (Below 2^32 lanes, so the kernel's 32-bit indices hold; segments shorter
+  // than kClSeg are taken for small grids only.)
   if (!launch_fits(batch * ((seqlen + kClSeg - 1) / kClSeg) * ((groups + kClThreads - 1) / kClThreads), kClThreads))
     return THM_ERR_BAD_SHAPE;
   const int wb = (w_dtype == THM_DTYPE_BF16);
   hipStream_t s = (hipStream_t)stream;
-  hipError_t e;
-  if (x_dtype == THM_DTYPE_F32)
-    e = vec_ok ? launch_cl<float, 4>(width, x, weight, bias, out, batch, seqlen, dim, wb, activation, s)
-               : launch_cl<float, 1>(width, x, weight, bias, out, batch, seqlen, dim, wb, activation, s);
-  else
-    e = vec_ok ? launch_cl<bf16, 8>(width, x, weight, bias, out, batch, seqlen, dim, wb, activation, s)
-               : launch_cl<bf16, 1>(width, x, weight, bias, out, batch, seqlen, dim, wb, activation, s);
+  auto run = [&](auto xt) {
+    using XT = decltype(xt);
+    return wb ? launch_cl<XT, bf16>(vec_ok, width, x, weight, bias, out, batch, seqlen, dim, activation, s)
+              : launch_cl<XT, float>(vec_ok, width, x, weight, bias, out, batch, seqlen, dim, activation, s);
+  };
+  const hipError_t e = x_dtype == THM_DTYPE_F32 ? run(float{}) : run(bf16{});
   return (int)e;
 }
 

@@ -35,6 +35,21 @@ constexpr float kLog2e = 1.4426950408889634f;
 // exp(x) through the hardware base-2 exponential (v_exp_f32).
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
+// x sigmoid(x) = x (x >= 0 ? 1 : e) / (1 + e) with e = e^{-|x|} <= 1, rounded
+// afterwards to XT.  For bf16 the quotient is a multiplication by the hardware
+// reciprocal (1 + e in [1, 2], where it is good to an ulp of fp32): an IEEE
+// division is ten instructions per element, and the convolutions with SiLU
+// spent more time on it than on memory.
+template <typename XT>
+__device__ __forceinline__ float silu(float x) {
+  if constexpr (sizeof(XT) == 2) {
+    const float e = fast_exp(-fabsf(x));
+    return x * (x >= 0.f ? 1.f : e) * __builtin_amdgcn_rcpf(1.f + e);
+  } else {
+    return x / (1.f + fast_exp(-x));
+  }
+}
+
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
 // Wave-uniform value of lane `src` (v_readlane).
