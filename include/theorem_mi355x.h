@@ -149,6 +149,23 @@ int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, const void* g,
                     int32_t chunk_size, int32_t kv_dtype, int32_t flags, void* stream);
 
 /*
+ * thm_chunk_fwd_h with device scratch: where a delta-form call's sequences
+ * alone leave the GPU idle, they are cut into segments that run side by side
+ * (chosen from the shape, the dtype and the device's CU count only, so results
+ * are deterministic per shape; they agree with thm_chunk_fwd_h's to the
+ * rounding of the state).  workspace: at least thm_chunk_fwd_h_workspace bytes
+ * (0: none needed), 16-byte aligned, owned by the call until it has run on
+ * `stream`; otherwise as thm_chunk_fwd_h.
+ */
+int64_t thm_chunk_fwd_h_workspace(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V,
+                                  int32_t kv_dtype, int32_t flags);
+int thm_chunk_fwd_h_ws(const void* k, const void* w, const void* vu, const void* g,
+                       const void* h0, void* h, void* v_new, void* ht, void* workspace,
+                       int64_t workspace_bytes, int64_t B, int64_t T, int64_t H, int64_t K,
+                       int64_t V, int32_t chunk_size, int32_t kv_dtype, int32_t flags,
+                       void* stream);
+
+/*
  * Gated DeltaNet chunkwise output, per chunk c and token i of the chunk:
  *   o[i] = scale * ( sum_{j<=i in chunk} (q_i . k_j) exp(g_i - g_j) v_j
  *                    + exp(g_i) q_i . h[c] )

@@ -9,18 +9,20 @@
 // Replaces kernels/chunk_fwd_h/kernel.py:61-138 (Triton) and its launcher
 // kernel.py:141-191.
 //
-// Two kernels:
-//   * the register-prefetch kernel (chunk_fwd_h_reg.h): every fp32 call (its
-//     instantiations are in chunk_fwd_h_f32.hip) and bf16 on grids under
-//     kHDmaMinGrid workgroups;
-//   * the DMA pipeline below: bf16 on grids that fill the GPU.
+// Kernels:
+//   * fp32: the register-prefetch kernel (chunk_fwd_h_reg.h, instantiated in
+//     chunk_fwd_h_f32.hip), and the role-split kernel on small grids;
+//   * bf16: the DMA pipeline below on grids that fill the GPU, the role-split
+//     kernel (chunk_fwd_h_small.h) on smaller ones;
+//   * delta form on grids that do not fill the GPU, with scratch memory
+//     (thm_chunk_fwd_h_ws): long sequences cut into segments (segments.h).
 // This unit is compiled with MFMA accumulators forced into VGPRs
-// (theorem_amd/build.py): the bf16 register kernel at config 3 takes 24.4
-// against 25.5 us with them in AGPRs, and the DMA kernel uses no AGPRs either way.
+// (theorem_amd/build.py).
 #include "chunk_fwd_h_reg.h"
 #include "chunk_fwd_h_small.h"
 
 #include "pipe_cfg.h"
+#include "segments.h"
 
 namespace thm {
 namespace {
@@ -51,6 +53,8 @@ namespace {
 // issued through vmem.h, so the wait at the top of the loop is an exact count:
 // after this wave's DMA of chunk c it has issued NS - 1 chunks of stores and
 // NS - 2 chunks of DMA.
+// Cut into segments (segments.h), a workgroup walks the `len` chunks of its
+// segment from the state the combine kernel left in sbuf.
 using pipe::PCfg;
 static_assert(pipe::kBT == kBT && pipe::kTileV == kHBV, "one chunk length and V-tile width");
 
@@ -59,15 +63,16 @@ __global__ void __launch_bounds__(256 * KS)
 chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
                        const bf16* __restrict__ vu, const float* __restrict__ g,
                        const float* __restrict__ h0, float* __restrict__ hout,
-                       bf16* __restrict__ vnew, float* __restrict__ ht, int64_t T, int64_t H,
-                       int64_t NT, int64_t BH) {
+                       bf16* __restrict__ vnew, float* __restrict__ ht, const char* __restrict__ sbuf,
+                       int64_t T, int64_t H, int64_t NT, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
   using C = PCfg<K, KS, NS, DELTA, HAS_G, STORE_VN>;
   constexpr int NVT = V / kHBV;
   __shared__ __attribute__((aligned(1024))) char lds[C::kLds];
 
-  const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH, NVT);
-  const int64_t bh = bt.bh;
+  const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH * nseg, NVT);
+  const int64_t sg = bt.bh / BH, bh = bt.bh - sg * BH;
   const int64_t b = bh / H, hh = bh % H;
+  const seg::Span sp = seg::span_of(sg, len, NT);
   const int v0 = (int)bt.vt * kHBV;
 
   const int tid = threadIdx.x;
@@ -86,9 +91,10 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
 
   // Global geometry in bytes.  Token t of chunk c, head hh: ((b T + 64 c + t) H + hh) D.
   const int64_t tsk = H * K * 2, tsv = H * V * 2;
-  const int64_t kc0 = ((b * T) * H + hh) * K * 2;
-  const int64_t uc0 = ((b * T) * H + hh) * V * 2 + v0 * 2;
-  const int64_t gc0 = ((b * T) * H + hh) * 4;
+  const int64_t tok0 = b * T + sp.c0 * kBT;  // the segment's first token
+  const int64_t kc0 = (tok0 * H + hh) * K * 2;
+  const int64_t uc0 = (tok0 * H + hh) * V * 2 + v0 * 2;
+  const int64_t gc0 = (tok0 * H + hh) * 4;
   const int64_t kcs = kBT * tsk, ucs = kBT * tsv, gcs = kBT * H * 4;
 
   // Per-lane DMA source offsets within a chunk (fixed for the sequence).
@@ -134,12 +140,18 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   f32x4 S[C::KBH];
   const int ncol = v0 + 16 * wq + li;
   const int64_t st_base = bh * (int64_t)(K * V);
+  if (sg > 0) {
+    const char* sp0 = sbuf + rec::s_off(sg * per - 1, bh, BH, K, V) + ((v0 / 16 + wq) * (K / 16) + kap0 / 16) * 1024 + 16 * lane;
 #pragma unroll
-  for (int kb = 0; kb < C::KBH; ++kb)
+    for (int kb = 0; kb < C::KBH; ++kb) S[kb] = *reinterpret_cast<const f32x4*>(sp0 + kb * 1024);
+  } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      S[kb][r] = h0 ? h0[st_base + (int64_t)(kap0 + 16 * kb + 4 * grp + r) * V + ncol] : 0.f;
-  // Retire the h0 loads here: a load still pending at the loop entry would
+    for (int kb = 0; kb < C::KBH; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        S[kb][r] = h0 ? h0[st_base + (int64_t)(kap0 + 16 * kb + 4 * grp + r) * V + ncol] : 0.f;
+  }
+  // Retire the state loads here: a load still pending at the loop entry would
   // make the compiler wait for every outstanding operation inside the loop.
   wait_vmcnt<0>();
 
@@ -152,15 +164,15 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   // it, instead of as a burst after the chunk's DMA issue: 441 against 483 us
   // at config 4, the stores no longer queue ahead of the next chunk's loads.
   auto store_h_tile = [&](int64_t c, int kb) {
-    float* hb = hout + ((b * NT + c) * H + hh) * (int64_t)(K * V);
+    float* hb = hout + ((b * NT + sp.c0 + c) * H + hh) * (int64_t)(K * V);
     st_b128(hb, hoff0 + (uint32_t)(kb * 16 * V * 4), __builtin_bit_cast(u32x4, acc_to_row_quads(S[kb])));
   };
 
-  if (NT > 0) {
+  if (sp.n > 0) {
 #pragma unroll
-    for (int i = 0; i < NS - 1; ++i) issue(i < NT ? i : NT - 1, i);
+    for (int i = 0; i < NS - 1; ++i) issue(i < sp.n ? i : sp.n - 1, i);
   }
-  for (int64_t c = 0; c < NT; ++c) {
+  for (int64_t c = 0; c < sp.n; ++c) {
     const int s = (int)(c % NS);
     if (wi == 0) {
       if (c < NS - 1) wait_vmcnt<C::kWaitFirst0>();
@@ -172,7 +184,7 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
     lds_barrier();  // A: chunk c is in LDS; every wave is done with chunk c - 1
     {
       const int64_t cn = c + NS - 1;
-      issue(cn < NT ? cn : NT - 1, (int)(cn % NS));
+      issue(cn < sp.n ? cn : sp.n - 1, (int)(cn % NS));
     }
 
     const char* tk = stage_k(s);
@@ -261,7 +273,7 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
         for (int jb = 0; jb < 4; ++jb) vn[jb] -= part[jb];
       }
       if constexpr (STORE_VN) {
-        bf16* vb = vnew + ((b * T + c * kBT) * H + hh) * V;
+        bf16* vb = vnew + ((tok0 + c * kBT) * H + hh) * V;
         // Row tiles kJbStore kh .. + kJbStore - 1.  One branch per K half
         // (kh is wave-uniform) keeps the register indices static: indexing
         // vn by kh itself compiled to relative register moves.
@@ -312,7 +324,7 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   // Drain: no DMA may still target this workgroup's LDS when it exits.
   wait_vmcnt<0>();
 
-  if (ht) {
+  if (ht && sg == nseg - 1) {
 #pragma unroll
     for (int kb = 0; kb < C::KBH; ++kb)
 #pragma unroll
@@ -329,16 +341,18 @@ using pipe::kHStages;  // DMA ring depth of the bf16 pipeline
 
 template <int K, int V, bool DELTA>
 hipError_t launch_h_dma(const void* k, const void* w, const void* vu, const void* g, const void* h0,
-                        void* h, void* vnew, void* ht, int64_t B, int64_t T, int64_t H, hipStream_t s) {
+                        void* h, void* vnew, void* ht, const void* sbuf, const seg::Plan& p, int64_t B, int64_t T,
+                        int64_t H, hipStream_t s) {
   const int64_t NT = T / kBT;
   const int64_t BH = B * H;
-  const dim3 grid((unsigned)(BH * (V / kHBV)));
+  const dim3 grid((unsigned)(BH * (V / kHBV) * p.out));
   constexpr int KS = kHKSplit, NS = kHStages;
 #define THM_H_DMA_LAUNCH(HG, SV)                                                               \
   hipLaunchKernelGGL((chunk_fwd_h_dma_kernel<K, V, KS, NS, DELTA, HG, SV>), grid,              \
                      dim3(PCfg<K, KS, NS, DELTA, HG, SV>::kThreads), 0, s, (const bf16*)k,     \
                      (const bf16*)w, (const bf16*)vu, (const float*)g, (const float*)h0,       \
-                     (float*)h, (bf16*)vnew, (float*)ht, T, H, NT, BH)
+                     (float*)h, (bf16*)vnew, (float*)ht, (const char*)sbuf, T, H, NT, BH, p.out,      \
+                     p.len * p.per, p.per)
   const bool sv = DELTA && vnew != nullptr;
   if (g) {
     if (sv) THM_H_DMA_LAUNCH(true, DELTA);
@@ -351,35 +365,72 @@ hipError_t launch_h_dma(const void* k, const void* w, const void* vu, const void
   return hipGetLastError();
 }
 
-template <typename IT, bool DELTA, int K, int V>
-hipError_t launch_kv(const void* k, const void* w, const void* vu, const void* g, const void* h0,
-                     void* h, void* vnew, void* ht, int64_t B, int64_t T, int64_t H, hipStream_t s) {
-  if constexpr (std::is_same<IT, bf16>::value) {
-    if (B * H * (V / kHBV) >= kHDmaMinGrid)
-      return launch_h_dma<K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
-    return launch_h_small<bf16, K, V, kHSmallNW, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
+// bf16, delta form: the state at every segment's start (segments.h), then the
+// DMA kernel on all segments.
+template <int K, int V>
+hipError_t launch_h_segments(const void* k, const void* w, const void* u, const void* g, const void* h0, void* h,
+                             void* vnew, void* ht, char* ws, const seg::Plan& p, int64_t B, int64_t T, int64_t H,
+                             hipStream_t s) {
+  const int64_t NT = T / kBT, BH = B * H, nt = p.segs(NT);
+  char* const pbuf = ws;
+  char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
+#define THM_H_TRANS_LAUNCH(HG)                                                                                     \
+  hipLaunchKernelGGL((seg::chunk_transition_kernel<K, V, true, HG>), dim3((unsigned)(BH * (nt - 1))),              \
+                     dim3(rec::TCfg<K, V, true>::kThreads), 0, s, (const bf16*)k, (const bf16*)w, (const bf16*)u,  \
+                     (const float*)g, (const char*)nullptr, (const float*)h0, pbuf, sbuf, T, H, NT, BH, p.len)
+  if (g) THM_H_TRANS_LAUNCH(true);
+  else THM_H_TRANS_LAUNCH(false);
+#undef THM_H_TRANS_LAUNCH
+  hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, false>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, pbuf,
+                     sbuf, BH, nt);
+  return launch_h_dma<K, V, true>(k, w, u, g, h0, h, vnew, ht, sbuf, p, B, T, H, s);
+}
+
+template <bool DELTA, int K, int V>
+hipError_t launch_kv(const void* k, const void* w, const void* vu, const void* g, const void* h0, void* h,
+                     void* vnew, void* ht, char* ws, const seg::Plan& p, int64_t B, int64_t T, int64_t H,
+                     hipStream_t s) {
+  if constexpr (DELTA) {
+    if (p.out > 1) return launch_h_segments<K, V>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
   }
-  return launch_h<IT, K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
+  if (B * H * (V / kHBV) >= kHDmaMinGrid)
+    return launch_h_dma<K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, nullptr, p, B, T, H, s);
+  return launch_h_small<bf16, K, V, kHSmallNW, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
 }
 
-template <typename IT, bool DELTA>
+template <bool DELTA>
 hipError_t dispatch_kv(int64_t K, int64_t V, const void* k, const void* w, const void* vu,
-                       const void* g, const void* h0, void* h, void* vnew, void* ht, int64_t B,
-                       int64_t T, int64_t H, hipStream_t s) {
-  if (K == 64 && V == 64) return launch_kv<IT, DELTA, 64, 64>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
-  if (K == 64 && V == 128) return launch_kv<IT, DELTA, 64, 128>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
-  if (K == 128 && V == 64) return launch_kv<IT, DELTA, 128, 64>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
-  return launch_kv<IT, DELTA, 128, 128>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
+                       const void* g, const void* h0, void* h, void* vnew, void* ht, char* ws, const seg::Plan& p,
+                       int64_t B, int64_t T, int64_t H, hipStream_t s) {
+  if (K == 64 && V == 64) return launch_kv<DELTA, 64, 64>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
+  if (K == 64 && V == 128) return launch_kv<DELTA, 64, 128>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
+  if (K == 128 && V == 64) return launch_kv<DELTA, 128, 64>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
+  return launch_kv<DELTA, 128, 128>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
 }
 
-}  // namespace
-}  // namespace thm
+// Segments of a call (segments.h plan_segments); one piece for the reference
+// form and on grids that fill the GPU without them.  Periods in us per chunk,
+// from MI355X timings (in one piece -> best of nine plans -> this rule):
+//   bf16, small-grid kernel against transitions and the DMA kernel: B = 1,
+//     H = 16, K = V = 128, 128 chunks 141 -> 104 -> 101 us (with other inputs
+//     every pass 200 -> 111), 32 chunks 38 -> 42 -> 38; H = 4, 64 chunks 71 ->
+//     50 -> 50; K = V = 64, 64 chunks 46 -> 32 -> 32;
+//   fp32, register kernel (at K = 64 the small-grid kernel in one piece): 16
+//     heads of K = V = 128, 32 chunks 137 -> 81 -> 80, 4 heads, 64 chunks 268
+//     -> 74 -> 74; 16 heads of K = V = 64, 64 chunks 97 -> 50 -> 50.
+inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, bool delta, bool f32) {
+  const int64_t NT = T / kBT, BH = B * H, nvt = V / kHBV;
+  if (!delta || BH * nvt >= kHDmaMinGrid) return {1, 1, std::max<int64_t>(NT, 1)};
+  if (f32) {
+    const double period = K == 128 ? 4.7 : 2.5;
+    return seg::plan_segments(BH, NT, {nvt, (K + V) / kHBV, nvt, K == 128 ? period : 1.7, period, 1.2, period});
+  }
+  return seg::plan_segments(BH, NT, {V / 32, 1, nvt, 1.2, 2.2, 0.9, 2.6});
+}
 
-extern "C" int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, const void* g,
-                               const void* h0, void* h, void* v_new, void* ht, int64_t B,
-                               int64_t T, int64_t H, int64_t K, int64_t V, int32_t chunk_size,
-                               int32_t kv_dtype, int32_t flags, void* stream) {
-  using namespace thm;
+int h_entry(const void* k, const void* w, const void* vu, const void* g, const void* h0, void* h, void* v_new,
+            void* ht, void* workspace, int64_t workspace_bytes, bool segments, int64_t B, int64_t T, int64_t H,
+            int64_t K, int64_t V, int32_t chunk_size, int32_t kv_dtype, int32_t flags, void* stream) {
   if (flags & ~THM_H_DELTA) return THM_ERR_BAD_ARGUMENT;
   const bool delta = (flags & THM_H_DELTA) != 0;
   if (!delta && v_new) return THM_ERR_BAD_ARGUMENT;  // v_new exists only in the delta form
@@ -403,13 +454,49 @@ extern "C" int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, con
   // Per-lane offsets within one chunk's token block are 32-bit.
   if (64 * H * (K > V ? K : V) * (kv_dtype == THM_DTYPE_F32 ? 4 : 2) > (INT64_C(1) << 31))
     return THM_ERR_UNSUPPORTED;
+  const bool f32 = kv_dtype == THM_DTYPE_F32;
+  seg::Plan p = {1, 1, std::max<int64_t>(T / kBT, 1)};
+  if (segments) {
+    p = plan_of(B, T, H, K, V, delta, f32);
+    const int64_t need = seg::p_bytes(p, B * H, T / kBT, K) + seg::s_bytes(p, B * H, T / kBT, K, V);
+    if (workspace_bytes < need) return THM_ERR_BAD_ARGUMENT;
+    if (need > 0 && !workspace) return THM_ERR_NULL_POINTER;
+    if ((uintptr_t)workspace % 16) return THM_ERR_MISALIGNED;
+  }
+  char* const ws = (char*)workspace;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
-  if (kv_dtype == THM_DTYPE_F32) {
-    e = chunk_fwd_h_f32(delta, K, V, k, w, vu, g, h0, h, v_new, ht, B, T, H, s);
-  } else {
-    e = delta ? dispatch_kv<bf16, true>(K, V, k, w, vu, g, h0, h, v_new, ht, B, T, H, s)
-              : dispatch_kv<bf16, false>(K, V, k, w, vu, g, h0, h, v_new, ht, B, T, H, s);
-  }
+  if (f32) e = chunk_fwd_h_f32(delta, K, V, k, w, vu, g, h0, h, v_new, ht, ws, p.out, p.per, p.len, B, T, H, s);
+  else if (delta) e = dispatch_kv<true>(K, V, k, w, vu, g, h0, h, v_new, ht, ws, p, B, T, H, s);
+  else e = dispatch_kv<false>(K, V, k, w, vu, g, h0, h, v_new, ht, ws, p, B, T, H, s);
   return (int)e;
+}
+
+}  // namespace
+}  // namespace thm
+
+extern "C" int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, const void* g,
+                               const void* h0, void* h, void* v_new, void* ht, int64_t B,
+                               int64_t T, int64_t H, int64_t K, int64_t V, int32_t chunk_size,
+                               int32_t kv_dtype, int32_t flags, void* stream) {
+  return thm::h_entry(k, w, vu, g, h0, h, v_new, ht, nullptr, 0, false, B, T, H, K, V, chunk_size, kv_dtype, flags,
+                      stream);
+}
+
+extern "C" int thm_chunk_fwd_h_ws(const void* k, const void* w, const void* vu, const void* g, const void* h0,
+                                  void* h, void* v_new, void* ht, void* workspace, int64_t workspace_bytes, int64_t B,
+                                  int64_t T, int64_t H, int64_t K, int64_t V, int32_t chunk_size, int32_t kv_dtype,
+                                  int32_t flags, void* stream) {
+  return thm::h_entry(k, w, vu, g, h0, h, v_new, ht, workspace, workspace_bytes, true, B, T, H, K, V, chunk_size,
+                      kv_dtype, flags, stream);
+}
+
+extern "C" int64_t thm_chunk_fwd_h_workspace(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int32_t kv_dtype,
+                                             int32_t flags) {
+  using namespace thm;
+  if (B <= 0 || T <= 0 || H <= 0 || T % kBT || (K != 64 && K != 128) || (V != 64 && V != 128) ||
+      B > (INT64_C(1) << 31) / H)
+    return 0;  // nothing to compute, or a call thm_chunk_fwd_h_ws refuses
+  const seg::Plan p = plan_of(B, T, H, K, V, (flags & THM_H_DELTA) != 0, kv_dtype == THM_DTYPE_F32);
+  return seg::p_bytes(p, B * H, T / kBT, K) + seg::s_bytes(p, B * H, T / kBT, K, V);
 }

@@ -38,6 +38,7 @@
 
 #include "h_layout.h"
 #include "mfma.h"
+#include "segments.h"
 #include "vmem.h"
 
 namespace thm {
@@ -97,36 +98,38 @@ __device__ __forceinline__ const char* cptr(const void* p, int64_t byte_off) {
 }
 
 // DEEP: two register sets, two chunks ahead (see the chunk loop below).
-template <typename IT, int K, int V, bool DELTA, bool HAS_G, bool DEEP>
+// Segments (segments.h): a workgroup walks the `len` chunks of its segment,
+// from the combine kernel's state in sbuf.  TRANS: the transition kernel of
+// this form, over column tiles of [P | Q]; only the final state is written, P
+// in A-operand blocks and Q in accumulator blocks, both fp32.
+template <typename IT, int K, int V, bool DELTA, bool HAS_G, bool DEEP, bool TRANS>
 __global__ void __launch_bounds__(kHThreads)
 chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT* __restrict__ vu,
                    const float* __restrict__ g, const float* __restrict__ h0,
                    float* __restrict__ hout, IT* __restrict__ vnew, float* __restrict__ ht,
-                   int64_t T, int64_t H, int64_t NT, int64_t BH) {
+                   char* __restrict__ pbuf, char* __restrict__ sbuf, int64_t T, int64_t H,
+                   int64_t NTotal, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
   using C = HCfg<IT, K, V, DELTA>;
   using St = HStage<IT>;
   using Pf = HPrefetch<IT, K, V, DELTA>;
   constexpr int KB = K / 16;
-  constexpr int NVT = V / kHBV;
+  constexpr int NPT = TRANS ? K / kHBV : 0;  // column tiles of P, ahead of the V-tiles
+  constexpr int NVT = NPT + V / kHBV;
   constexpr int EB = C::kEB;
   __shared__ __attribute__((aligned(16))) bf16 lds_b[C::kStages * C::kBf16PerStage];
   __shared__ __attribute__((aligned(16))) IT lds_u[C::kStages * C::kUTile];
   __shared__ __attribute__((aligned(16))) float lds_g[C::kStages * kBT];
 
-  // XCD-aware block mapping: block i runs on XCD i % 8; give all V-tiles of a
-  // (b, head) the same i % 8 when the grid allows it.
-  const int64_t blk = blockIdx.x;
-  int64_t bh, vt;
-  if (BH % 8 == 0) {
-    const int64_t xcd = blk % 8, slot = blk / 8;
-    bh = (slot / NVT) * 8 + xcd;
-    vt = slot % NVT;
-  } else {
-    bh = blk / NVT;
-    vt = blk % NVT;
-  }
+  // XCD-aware block mapping: the column tiles of one (b, head, segment) share an XCD.
+  const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH * nseg, NVT);
+  const int64_t sg = bt.bh / BH, bh = bt.bh - sg * BH;
   const int64_t b = bh / H, hh = bh % H;
-  const int v0 = (int)vt * kHBV;
+  const bool is_p = TRANS && bt.vt < NPT;
+  if (is_p && sg == 0) return;  // segment 0 starts from a known state (whole workgroup)
+  const int v0 = (int)(is_p ? bt.vt : bt.vt - NPT) * kHBV;  // first column, of P or of V
+  const int uv0 = is_p ? 0 : v0;                            // P reads any column of u and drops it
+  const seg::Span sp = seg::span_of(sg, len, NTotal);
+  const int64_t NT = sp.n;
 
   auto stage = [&](int i) {
     St st;
@@ -156,13 +159,14 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   const int uj0 = tid / C::kUCPR, ucol0 = (tid % C::kUCPR) * C::kVE;
   const uint32_t koff0 = (uint32_t)(kj0 * tok_stride_k + kcol * EB);
   const uint32_t kstep = (uint32_t)((kHThreads / C::kKCPR) * tok_stride_k);
-  const uint32_t uoff0 = (uint32_t)(uj0 * tok_stride_v + (v0 + ucol0) * EB);
+  const uint32_t uoff0 = (uint32_t)(uj0 * tok_stride_v + (uv0 + ucol0) * EB);
   const uint32_t ustep = (uint32_t)((kHThreads / C::kUCPR) * tok_stride_v);
   const uint32_t goff = (uint32_t)(lane * H * 4);  // every wave: token `lane` of the chunk
   // chunk bases (bytes from the tensor start), advanced per chunk
-  const int64_t kc0 = ((b * T) * H + hh) * K * EB;
-  const int64_t uc0 = ((b * T) * H + hh) * V * EB;
-  const int64_t gc0 = ((b * T) * H + hh) * 4;
+  const int64_t tok0 = b * T + sp.c0 * kBT;  // the segment's first token
+  const int64_t kc0 = (tok0 * H + hh) * K * EB;
+  const int64_t uc0 = (tok0 * H + hh) * V * EB;
+  const int64_t gc0 = (tok0 * H + hh) * 4;
   const int64_t kcs = kBT * tok_stride_k, ucs = kBT * tok_stride_v, gcs = kBT * H * 4;
 
   auto prefetch = [&](Pf& pf, int64_t c) {
@@ -212,11 +216,22 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   f32x4 S[KB];
   const uint32_t s_off = (uint32_t)((4 * grp * V + vcol) * 4);  // + (16 kb + r) * V * 4
   const int64_t st_base = bh * (int64_t)(K * V) * 4;             // h0 / ht (bytes)
+  if (is_p) {
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      S[kb][r] = h0 ? *reinterpret_cast<const float*>(cptr(h0, st_base) + s_off + (16 * kb + r) * V * 4) : 0.f;
+      for (int r = 0; r < 4; ++r) S[kb][r] = 16 * kb + 4 * grp + r == vcol ? 1.f : 0.f;
+  } else if (sg > 0) {
+    const char* sp0 = sbuf + rec::s_off(sg * per - 1, bh, BH, K, V) + (v0 / 16 + wv) * KB * 1024 + 16 * lane;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) S[kb] = TRANS ? zero4() : *reinterpret_cast<const f32x4*>(sp0 + kb * 1024);
+  } else {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        S[kb][r] = h0 ? *reinterpret_cast<const float*>(cptr(h0, st_base) + s_off + (16 * kb + r) * V * 4) : 0.f;
+  }
 
   // v_new rows j = 16 jb + 4 grp + r of this lane's column, relative to the chunk base.
   // (h and v_new are stored one element per lane: 16 consecutive lanes cover
@@ -224,7 +239,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   // kernel below is slower here: 31.0 against 25.6 us at config 3.)
   const uint32_t vn_off = (uint32_t)(4 * grp * tok_stride_v + vcol * EB);
   auto store_state = [&](int64_t c) {
-    char* hb = reinterpret_cast<char*>(hout) + ((b * NT + c) * H + hh) * (int64_t)(K * V) * 4;
+    char* hb = reinterpret_cast<char*>(hout) + ((b * NTotal + sp.c0 + c) * H + hh) * (int64_t)(K * V) * 4;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -252,14 +267,17 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
       const int64_t pc = DEEP ? c + 2 : c + 1;
       if (pc < NT) prefetch(nxt, pc);
     }
-    if constexpr (DELTA) store_state(c);  // state before chunk c
+    if constexpr (DELTA && !TRANS) store_state(c);  // state before chunk c
 
     // v_new (or v) for rows j = 16 jb + 4 grp + r of this lane's column.
     f32x4 vn[4];
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vn[jb][r] = to_f32(cs.u[(16 * jb + 4 * grp + r) * C::kUPitch + ucol]);
+      for (int r = 0; r < 4; ++r) {
+        const float x = to_f32(cs.u[(16 * jb + 4 * grp + r) * C::kUPitch + ucol]);
+        vn[jb][r] = is_p ? 0.f : x;
+      }
 
     if constexpr (DELTA) {
       // P1: B operand = S pairs (kappa blocks 2s, 2s+1) in paired order.
@@ -329,9 +347,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
     lds_barrier();
     // v_new after the commit: stores queued behind the prefetch would make its
     // wait cover them too (loads and stores share one in-order counter).
-    if constexpr (DELTA) {
+    if constexpr (DELTA && !TRANS) {
       if (vnew) {
-        char* vb = reinterpret_cast<char*>(vnew) + (((b * T + c * kBT) * H + hh) * V) * EB;
+        char* vb = reinterpret_cast<char*>(vnew) + (((tok0 + c * kBT) * H + hh) * V) * EB;
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
@@ -349,7 +367,17 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
     for (int64_t c = 0; c < NT; ++c) chunk(c, pa, pa);
   }
 
-  if (ht) {
+  if constexpr (TRANS) {
+    const int slot = 16 * (li & 3) + 4 * grp + (li >> 2);  // of row 4 grp + li / 4 (acc_to_row_quads)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (is_p)
+        *reinterpret_cast<f32x4*>(pbuf + rec::p_off(sg, bh, BH, K) + (kb * KB + v0 / 16 + wv) * 1024 + 16 * slot) =
+            acc_to_row_quads(S[kb]);
+      else
+        *reinterpret_cast<f32x4*>(sbuf + rec::s_off(sg, bh, BH, K, V) + ((v0 / 16 + wv) * KB + kb) * 1024 + 16 * lane) = S[kb];
+    }
+  } else if (ht && sg == nseg - 1) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -365,30 +393,41 @@ constexpr int64_t kHDmaMinGrid = 256;
 
 template <typename IT, int K, int V, bool DELTA>
 hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g, const void* h0,
-                    void* h, void* vnew, void* ht, int64_t B, int64_t T, int64_t H, hipStream_t s) {
+                    void* h, void* vnew, void* ht, char* ws, const seg::Plan& p, int64_t B, int64_t T,
+                    int64_t H, hipStream_t s) {
   const int64_t NT = T / kBT;
   const int64_t BH = B * H;
-  const dim3 grid((unsigned)(BH * (V / kHBV)));
-  const bool deep = BH * (V / kHBV) >= kHDmaMinGrid;  // bandwidth-bound regime
-#define THM_H_LAUNCH(HG, DP)                                                                      \
-  hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP>), grid, dim3(kHThreads), 0, s,  \
-                     (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g, (const float*)h0, \
-                     (float*)h, (IT*)vnew, (float*)ht, T, H, NT, BH)
+  const int64_t wgs = BH * (V / kHBV) * p.out;
+  char* const pbuf = ws;
+  char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
+#define THM_H_LAUNCH(HG, DP, TR, GRID, NSEG, LEN)                                                           \
+  hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP, TR>), dim3((unsigned)(GRID)),             \
+                     dim3(kHThreads), 0, s, (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g,     \
+                     (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, T, H, NT, BH, NSEG, LEN, p.per)
+  if constexpr (DELTA) {
+    if (p.out > 1) {
+      const int64_t nt = p.segs(NT), grid = BH * (nt - 1) * ((K + V) / kHBV);
+      if (g) THM_H_LAUNCH(true, false, true, grid, nt - 1, p.len);
+      else THM_H_LAUNCH(false, false, true, grid, nt - 1, p.len);
+      hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, true>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
+                         pbuf, sbuf, BH, nt);
+    }
+  }
+  const bool deep = p.out == 1 && wgs >= kHDmaMinGrid;  // bandwidth-bound regime
   if (g) {
-    if (deep) THM_H_LAUNCH(true, true);
-    else THM_H_LAUNCH(true, false);
+    if (deep) THM_H_LAUNCH(true, true, false, wgs, p.out, p.len * p.per);
+    else THM_H_LAUNCH(true, false, false, wgs, p.out, p.len * p.per);
   } else {
-    if (deep) THM_H_LAUNCH(false, true);
-    else THM_H_LAUNCH(false, false);
+    if (deep) THM_H_LAUNCH(false, true, false, wgs, p.out, p.len * p.per);
+    else THM_H_LAUNCH(false, false, false, wgs, p.out, p.len * p.per);
   }
 #undef THM_H_LAUNCH
   return hipGetLastError();
 }
 
-// fp32 inputs, defined in chunk_fwd_h_f32.hip: the register kernel for every
-// (K, V) and form.
+// fp32 inputs, defined in chunk_fwd_h_f32.hip (out, per, len: seg::Plan).
 }  // namespace
 __attribute__((visibility("hidden"))) hipError_t chunk_fwd_h_f32(bool delta, int64_t K, int64_t V, const void* k, const void* w, const void* vu,
-                           const void* g, const void* h0, void* h, void* vnew, void* ht, int64_t B, int64_t T,
-                           int64_t H, hipStream_t s);
+                           const void* g, const void* h0, void* h, void* vnew, void* ht, char* ws, int64_t out, int64_t per,
+                           int64_t len, int64_t B, int64_t T, int64_t H, hipStream_t s);
 }  // namespace thm

@@ -105,9 +105,14 @@ py::object h(const at::Tensor& k, const c10::optional<at::Tensor>& w, const at::
   c10::optional<at::Tensor> vn, ht;
   if (delta && want_vn) vn = at::empty_like(vu);
   if (want_ht) ht = at::empty({B, H, K, V}, f32);
-  const int st = thm_chunk_fwd_h(k.data_ptr(), ptr(w), vu.data_ptr(), ptr(g), ptr(h0), hs.data_ptr(),
-                                 vn.has_value() ? vn->data_ptr() : nullptr, ht.has_value() ? ht->data_ptr() : nullptr,
-                                 B, T, H, K, V, (int32_t)kBT, code, delta ? THM_H_DELTA : 0, stream_of(dev));
+  const int32_t flags = delta ? THM_H_DELTA : 0;
+  const int64_t nws = thm_chunk_fwd_h_workspace(B, T, H, K, V, code, flags);
+  at::Tensor ws;
+  if (nws > 0) ws = at::empty({nws}, k.options().dtype(at::kByte));
+  const int st = thm_chunk_fwd_h_ws(k.data_ptr(), ptr(w), vu.data_ptr(), ptr(g), ptr(h0), hs.data_ptr(),
+                                    vn.has_value() ? vn->data_ptr() : nullptr,
+                                    ht.has_value() ? ht->data_ptr() : nullptr, nws > 0 ? ws.data_ptr() : nullptr, nws,
+                                    B, T, H, K, V, (int32_t)kBT, code, flags, stream_of(dev));
   if (st != THM_OK) return py::int_(st);
   return py::make_tuple(hs, vn.has_value() ? py::cast(*vn) : py::none(), ht.has_value() ? py::cast(*ht) : py::none());
 }

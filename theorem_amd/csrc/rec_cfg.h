@@ -1,5 +1,5 @@
 // Chunk records of the chunked Gated DeltaNet forward, and the layout of the
-// kernels that read them (chunk_fwd_rec.hip).  Plain constants and index
+// kernels that read them (chunk_fwd_rec.hip, segments.h).  Plain constants and index
 // maps, also compiled on the host.
 //
 // A record holds what the recurrence of one (b, head, chunk) needs besides
@@ -72,7 +72,8 @@ struct OCfg {
 };
 
 // Transition kernel: one wavefront per 16 kCT columns of [P | Q], K + V in all.
-template <int K, int V>
+// Stage: the k tile, the v tiles and the record; WU: k, u, w tiles and the gates.
+template <int K, int V, bool WU>
 struct TCfg {
   static constexpr int kCT = 2;  // 16-column tiles per wave
   static constexpr int kWaves = (K + V) / (16 * kCT), kThreads = 64 * kWaves;
@@ -80,13 +81,13 @@ struct TCfg {
   static constexpr int kRowK = K * 2, kTileK = kBT * kRowK;
   static constexpr int kRowV = kTileV * 2, kTileVB = kBT * kRowV;
   static constexpr int kNVT = V / kTileV;
-  static constexpr int kStage = kTileK + kNVT * kTileVB + kBytes;  // k, v tiles, record
+  static constexpr int kStage = kTileK + kNVT * kTileVB + (WU ? kTileK + 1024 : kBytes);
   static constexpr int kStages = 3;
   static constexpr int kLds = kStages * kStage;
   // 1 KiB DMA instructions of a chunk, in the order of the stage, spread over
   // the waves round by round: every wave issues kDma, or one fewer where the
   // last round does not reach it.
-  static constexpr int kKInstr = kTileK / 1024, kRInstr = kBytes / 1024, kVInstr = kNVT * kTileVB / 1024;
+  static constexpr int kKInstr = kTileK / 1024, kRInstr = (WU ? kTileK : kBytes) / 1024, kVInstr = kNVT * kTileVB / 1024;
   static constexpr int kInstr = kKInstr + kVInstr + kRInstr;
   static constexpr int kDma = (kInstr + kWaves - 1) / kWaves;
   static constexpr int kWait = (kStages - 2) * kDma;

@@ -46,6 +46,8 @@ SIGNATURES = {
                               _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_vp],
     "thm_chunk_fwd_h": [_c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp,
                         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_vp],
+    "thm_chunk_fwd_h_workspace": [_c_i64] * 5 + [_c_i32, _c_i32],
+    "thm_chunk_fwd_h_ws": [_c_vp] * 9 + [_c_i64] * 6 + [_c_i32, _c_i32, _c_i32, _c_vp],
     "thm_chunk_fwd_o": [_c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, ctypes.c_float,
                         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_vp],
     "thm_chunk_gated_delta_fwd": [_c_vp] * 9 + [ctypes.c_float] + [_c_i64] * 5 + [_c_i32, _c_i32, _c_vp],
@@ -57,7 +59,8 @@ SIGNATURES = {
     "thm_chunk_local_cumsum": [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_vp],
     "thm_wy_fwd": [_c_vp] * 6 + [_c_i64] * 5 + [_c_i32, _c_i32, _c_i32, _c_vp],
 }
-_RESTYPES = {"thm_status_string": ctypes.c_char_p, "thm_chunk_gated_delta_rule_workspace": _c_i64}
+_RESTYPES = {"thm_status_string": ctypes.c_char_p, "thm_chunk_gated_delta_rule_workspace": _c_i64,
+             "thm_chunk_fwd_h_workspace": _c_i64}
 
 _lib = None
 _lock = threading.Lock()

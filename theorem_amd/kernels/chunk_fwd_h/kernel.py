@@ -65,10 +65,12 @@ def custom_kernel(data):
     h = torch.empty((B, NT, H, K, V), dtype=f32, device=dev)
     v_new = (torch.empty_like(vu) if vu.is_contiguous() else vu.new_empty(vu.shape)) if want_vn else None
     ht = torch.empty((B, H, K, V), dtype=f32, device=dev) if want_ht else None
-    status = _capi.load_library().thm_chunk_fwd_h(
+    lib, flags = _capi.load_library(), _capi.THM_H_DELTA if delta else 0
+    ws = torch.empty(lib.thm_chunk_fwd_h_workspace(B, T, H, K, V, code, flags), dtype=torch.uint8, device=dev)
+    status = lib.thm_chunk_fwd_h_ws(
         pk, pw, pu, pg, ph0, h.data_ptr(), None if v_new is None else v_new.data_ptr(),
-        None if ht is None else ht.data_ptr(),
-        B, T, H, K, V, CHUNK_SIZE, code, _capi.THM_H_DELTA if delta else 0, _capi.stream_of(k))
+        None if ht is None else ht.data_ptr(), ws.data_ptr(), ws.numel(),
+        B, T, H, K, V, CHUNK_SIZE, code, flags, _capi.stream_of(k))
     _capi.check(status, "thm_chunk_fwd_h")
     if delta:
         return h, v_new, ht
