@@ -18,7 +18,8 @@
 //      out[t] = act(bias + sum_k w[k] window[L_s - (W-1) + t + k]),  t < L,
 //    and the state becomes the last L_s samples of the window (in place).
 //    One lane per (b, d); a decode step moves a few bytes per channel, so this
-//    is latency-, not bandwidth-, bound.
+//    is latency-, not bandwidth-, bound: one sample per sequence has a kernel
+//    of its own (causal_conv1d_step_kernel).
 #include <algorithm>
 
 #include "common.h"
@@ -255,11 +256,68 @@ causal_conv1d_update_kernel(const XT* __restrict__ x, XT* __restrict__ state,
   for (int64_t i = 0; i < state_len; ++i) st[i] = i + seqlen < state_len ? st[i + seqlen] : xr[i + seqlen - state_len];
 }
 
+// One new sample per row and a state of W - 1 + OFF samples (OFF 0 or 1: what a
+// decode loop keeps): the state, the taps and the sample are loaded whole and
+// all at once, where the general kernel's loop waits for each tap in turn.
+// [64, 4096] bf16, W = 4, kernel trace: 5.6 -> 2.5 us.
+template <typename XT, typename WT, int W, int OFF>
+__global__ void __launch_bounds__(256)
+causal_conv1d_step_kernel(const XT* __restrict__ x, XT* __restrict__ state, const void* __restrict__ weight,
+                          const void* __restrict__ bias, XT* __restrict__ out, uint32_t rows, uint32_t dim, int act) {
+  constexpr int L = W - 1 + OFF;
+  const uint32_t row = blockIdx.x * 256 + threadIdx.x;  // b * dim + d
+  if (row >= rows) return;
+  const uint32_t d = row % dim;
+  XT win[L + 1];  // the state, then the new sample
+  WT wk[W];
+  XT* const st = state + (int64_t)row * L;
+  if constexpr (L > 0) __builtin_memcpy(win, st, L * sizeof(XT));
+  __builtin_memcpy(wk, reinterpret_cast<const WT*>(weight) + (int64_t)d * W, W * sizeof(WT));
+  win[L] = x[row];
+  float acc = bias ? to_f32(reinterpret_cast<const WT*>(bias)[d]) : 0.f;
+#pragma unroll
+  for (int k = 0; k < W; ++k) acc = __builtin_fmaf(to_f32(wk[k]), to_f32(win[OFF + k]), acc);
+  if (act == THM_ACT_SILU) acc = silu<XT>(acc);
+  out[row] = from_f32<XT>(acc);
+  if constexpr (L > 0) __builtin_memcpy(st, win + 1, L * sizeof(XT));
+}
+
+template <typename XT, typename WT, int OFF>
+hipError_t launch_step(int width, const void* x, void* state, const void* weight, const void* bias, void* out,
+                       int64_t rows, int64_t dim, int act, hipStream_t s) {
+  const dim3 grid((unsigned)((rows + 255) / 256));
+  switch (width) {
+#define THM_STEP_W(WV)                                                                                              \
+  case WV:                                                                                                          \
+    hipLaunchKernelGGL((causal_conv1d_step_kernel<XT, WT, WV, OFF>), grid, dim3(256), 0, s, (const XT*)x, (XT*)state, \
+                       weight, bias, (XT*)out, (uint32_t)rows, (uint32_t)dim, act);                                 \
+    break;
+    THM_STEP_W(1)
+    THM_STEP_W(2)
+    THM_STEP_W(3)
+    THM_STEP_W(4)
+    THM_STEP_W(5)
+    THM_STEP_W(6)
+    THM_STEP_W(7)
+    THM_STEP_W(8)
+#undef THM_STEP_W
+    default:
+      return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <typename XT>
 hipError_t launch_update(const void* x, void* state, const void* weight, const void* bias, void* out,
                          int64_t batch, int64_t dim, int64_t seqlen, int64_t state_len, int width,
                          int wb, int act, hipStream_t s) {
   const int64_t rows = batch * dim;
+  if (seqlen == 1 && state_len == width - 1)
+    return wb ? launch_step<XT, bf16, 0>(width, x, state, weight, bias, out, rows, dim, act, s)
+              : launch_step<XT, float, 0>(width, x, state, weight, bias, out, rows, dim, act, s);
+  if (seqlen == 1 && state_len == width)
+    return wb ? launch_step<XT, bf16, 1>(width, x, state, weight, bias, out, rows, dim, act, s)
+              : launch_step<XT, float, 1>(width, x, state, weight, bias, out, rows, dim, act, s);
   const dim3 grid((unsigned)((rows + 255) / 256));
   hipLaunchKernelGGL((causal_conv1d_update_kernel<XT>), grid, dim3(256), 0, s, (const XT*)x,
                      (XT*)state, weight, bias, (XT*)out, rows, dim, seqlen, state_len, width, wb, act);
