@@ -125,6 +125,12 @@ def chunk_fwd_fused_a(q, k, v, beta, A, g, scale: float, initial_state=None, out
 def _fwd_records(q, k, v, beta, gate, gate_kind: int, scale: float, initial_state, output_final_state: bool):
     """The bf16 forward from (q, k, v, beta, gate) in one C call
     (thm_chunk_gated_delta_rule_fwd): (o, ht or None)."""
+    fp = _capi.fastpath()
+    if fp is not None:
+        r = _capi.fast_result(fp.gated_delta_rule(q, k, v, beta, gate, gate_kind, initial_state, float(scale),
+                                                  bool(output_final_state)), "thm_chunk_gated_delta_rule_fwd")
+        if r is not None:
+            return r
     B, T, H, K = k.shape
     V = v.shape[-1]
     assert T % BT == 0, f"T={T} must be a multiple of {BT}"

@@ -1,4 +1,5 @@
-// Host fast path of the four custom_kernel wrappers (theorem_amd.kernels.*):
+// Host fast path of the custom_kernel wrappers (theorem_amd.kernels.*), the conv
+// decode step and the chunked forward (theorem_amd.chain):
 // the argument checks, the output allocation and the C-ABI launch of one call
 // in C++ (pybind11 over torch tensors), instead of Python attribute queries,
 // torch.empty calls from Python and a ctypes call with 17 arguments.
@@ -40,23 +41,90 @@ bool is_f32(const c10::optional<at::Tensor>& t) { return !t.has_value() || t->sc
 
 void* stream_of(int dev) { return c10::hip::getCurrentHIPStream(dev).stream(); }
 
-// causal_conv1d.custom_kernel((x, weight, bias), activation) for x [B, D, S] contiguous.
-py::object conv1d(const at::Tensor& x, const at::Tensor& weight, const c10::optional<at::Tensor>& bias,
-                  int32_t activation) {
-  if (!x.is_cuda() || x.dim() != 3 || weight.dim() != 2) return py::none();
+bool aligned16(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+// weight [D, W] and bias [D] (or none) of one dtype on `dev`.
+bool conv_params_ok(const at::Tensor& weight, const c10::optional<at::Tensor>& bias, int64_t D, int dev) {
+  return weight.dim() == 2 && ok(weight, dev) && ok_opt(bias, dev) && weight.size(0) == D && weight.size(1) <= INT32_MAX &&
+         dtype_code(weight) >= 0 &&
+         (!bias.has_value() || (bias->dim() == 1 && bias->size(0) == D && bias->scalar_type() == weight.scalar_type()));
+}
+
+// causal_conv1d.custom_kernel((x, weight, bias), activation) for x [B, D, S]
+// contiguous, and for a channels-last x (`rows` false).
+py::object conv1d_any(const at::Tensor& x, const at::Tensor& weight, const c10::optional<at::Tensor>& bias,
+                      int32_t activation, bool rows) {
+  if (!x.is_cuda() || x.dim() != 3 || x.is_contiguous() != rows) return py::none();
   const int dev = x.get_device();
-  if (!ok(x, dev) || !ok(weight, dev) || !ok_opt(bias, dev)) return py::none();
-  const int64_t B = x.size(0), D = x.size(1), S = x.size(2), W = weight.size(1);
-  if (weight.size(0) != D || (bias.has_value() && (bias->dim() != 1 || bias->size(0) != D ||
-                                                   bias->scalar_type() != weight.scalar_type())))
-    return py::none();
-  const int32_t xd = dtype_code(x), wd = dtype_code(weight);
-  if (xd < 0 || wd < 0 || W > INT32_MAX) return py::none();
-  at::Tensor out = at::empty_like(x);
-  const int st = thm_causal_conv1d_fwd(x.data_ptr(), weight.data_ptr(), ptr(bias), out.data_ptr(), B, D, S,
-                                       (int32_t)W, xd, wd, activation, stream_of(dev));
+  const int64_t B = x.size(0), D = x.size(1), S = x.size(2);
+  if (!aligned16(x) || !conv_params_ok(weight, bias, D, dev)) return py::none();
+  if (!rows && !(D > 1 && x.stride(1) == 1 && x.stride(2) == D && x.stride(0) == D * S)) return py::none();
+  const int32_t xd = dtype_code(x), wd = dtype_code(weight), W = (int32_t)weight.size(1);
+  if (xd < 0) return py::none();
+  at::Tensor out = at::empty_like(x);  // x's layout
+  const int st = rows ? thm_causal_conv1d_fwd(x.data_ptr(), weight.data_ptr(), ptr(bias), out.data_ptr(), B, D, S, W, xd,
+                                              wd, activation, stream_of(dev))
+                      : thm_causal_conv1d_fwd_channels_last(x.data_ptr(), weight.data_ptr(), ptr(bias), out.data_ptr(), B,
+                                                            S, D, W, xd, wd, activation, stream_of(dev));
   if (st != THM_OK) return py::int_(st);
   return py::cast(out);
+}
+py::object conv1d(const at::Tensor& x, const at::Tensor& weight, const c10::optional<at::Tensor>& bias, int32_t activation) {
+  return conv1d_any(x, weight, bias, activation, true);
+}
+py::object conv1d_channels_last(const at::Tensor& x, const at::Tensor& weight, const c10::optional<at::Tensor>& bias,
+                                int32_t activation) {
+  return conv1d_any(x, weight, bias, activation, false);
+}
+
+// causal_conv1d.causal_conv1d_update: x [B, D] or [B, D, L], conv_state [B, D, state_len] updated in place.
+py::object conv1d_update(const at::Tensor& x, const at::Tensor& conv_state, const at::Tensor& weight,
+                         const c10::optional<at::Tensor>& bias, int32_t activation) {
+  if (!x.is_cuda() || (x.dim() != 2 && x.dim() != 3) || conv_state.dim() != 3) return py::none();
+  const int dev = x.get_device();
+  const int64_t B = x.size(0), D = x.size(1), L = x.dim() == 3 ? x.size(2) : 1;
+  if (!ok(x, dev) || !ok(conv_state, dev) || !conv_params_ok(weight, bias, D, dev) || conv_state.size(0) != B ||
+      conv_state.size(1) != D || conv_state.scalar_type() != x.scalar_type())
+    return py::none();
+  const int32_t xd = dtype_code(x), wd = dtype_code(weight);
+  if (xd < 0) return py::none();
+  at::Tensor out = at::empty_like(x);
+  const int st = thm_causal_conv1d_update(x.data_ptr(), conv_state.data_ptr(), weight.data_ptr(), ptr(bias),
+                                          out.data_ptr(), B, D, L, conv_state.size(2), (int32_t)weight.size(1), xd, wd,
+                                          activation, stream_of(dev));
+  if (st != THM_OK) return py::int_(st);
+  return py::cast(out);
+}
+
+// chain: (o, final state or None) of the whole bf16 forward from q, k, v, beta and the gate.
+py::object gated_delta_rule(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& beta,
+                            const c10::optional<at::Tensor>& gate, int32_t gate_kind,
+                            const c10::optional<at::Tensor>& h0, double scale, bool want_ht) {
+  if (!k.is_cuda() || k.dim() != 4 || v.dim() != 4) return py::none();
+  const int dev = k.get_device();
+  if (!ok(q, dev) || !ok(k, dev) || !ok(v, dev) || !ok(beta, dev) || !ok_opt(gate, dev) || !ok_opt(h0, dev))
+    return py::none();
+  const int64_t B = k.size(0), T = k.size(1), H = k.size(2), K = k.size(3), V = v.size(3);
+  const at::IntArrayRef bth = k.sizes().slice(0, 3);
+  if (T % kBT || q.sizes() != k.sizes() || v.sizes().slice(0, 3) != bth || beta.sizes() != bth ||
+      (gate.has_value() && gate->sizes() != bth) || (h0.has_value() && h0->sizes() != at::IntArrayRef({B, H, K, V})))
+    return py::none();
+  if (q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || v.scalar_type() != at::kBFloat16 ||
+      beta.scalar_type() != at::kFloat || !is_f32(h0) || (gate_kind == THM_GATE_CUMULATIVE && !is_f32(gate)))
+    return py::none();
+  const int32_t gd = gate.has_value() ? dtype_code(*gate) : THM_DTYPE_F32;
+  if (gd < 0) return py::none();
+  const int64_t nws = thm_chunk_gated_delta_rule_workspace(B, T, H, K, V);
+  if (nws < 0) return py::none();
+  at::Tensor ws = at::empty({nws}, k.options().dtype(at::kByte)), out = at::empty_like(v);
+  c10::optional<at::Tensor> ht;
+  if (want_ht) ht = at::empty({B, H, K, V}, k.options().dtype(at::kFloat));
+  const int st = thm_chunk_gated_delta_rule_fwd(
+      q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(), ptr(gate), ptr(h0), out.data_ptr(),
+      ht.has_value() ? ht->data_ptr() : nullptr, ws.data_ptr(), nws, (float)scale, B, T, H, K, V, (int32_t)kBT,
+      THM_DTYPE_BF16, gd, gate_kind, stream_of(dev));
+  if (st != THM_OK) return py::int_(st);
+  return py::make_tuple(out, ht.has_value() ? py::cast(*ht) : py::none());
 }
 
 // recompute_w_u: (w, u) from k, v [B, T, H, K / V], beta [B, T, H], A [B, T, H, 64], g.
@@ -145,6 +213,12 @@ py::object o(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, cons
 PYBIND11_MODULE(_fastpath, m) {
   m.doc() = "Host fast path of the custom_kernel wrappers (None: use the Python path; int: C status to raise)";
   m.def("conv1d", &conv1d, py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("activation"));
+  m.def("conv1d_channels_last", &conv1d_channels_last, py::arg("x"), py::arg("weight"), py::arg("bias"),
+        py::arg("activation"));
+  m.def("conv1d_update", &conv1d_update, py::arg("x"), py::arg("conv_state"), py::arg("weight"), py::arg("bias"),
+        py::arg("activation"));
+  m.def("gated_delta_rule", &gated_delta_rule, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("beta"),
+        py::arg("gate"), py::arg("gate_kind"), py::arg("h0"), py::arg("scale"), py::arg("want_ht"));
   m.def("wu", &wu, py::arg("k"), py::arg("v"), py::arg("beta"), py::arg("A"), py::arg("g"));
   m.def("h", &h, py::arg("k"), py::arg("w"), py::arg("vu"), py::arg("g"), py::arg("h0"), py::arg("delta"),
         py::arg("want_vn"), py::arg("want_ht"));

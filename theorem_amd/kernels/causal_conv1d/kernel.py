@@ -61,6 +61,8 @@ def custom_kernel(data: tuple, activation: str | None = None) -> torch.Tensor:
     fp = _capi.fastpath() if act is not None else None
     if fp is not None:
         out = _capi.fast_result(fp.conv1d(x, weight, bias, act), "thm_causal_conv1d_fwd")
+        if out is None:
+            out = _capi.fast_result(fp.conv1d_channels_last(x, weight, bias, act), "thm_causal_conv1d_fwd_channels_last")
         if out is not None:
             return out
     B, D, S = x.shape
@@ -92,6 +94,11 @@ def causal_conv1d_update(x: torch.Tensor, conv_state: torch.Tensor, weight: torc
     (state_len >= W - 1, dtype of x) updated in place to the last state_len
     samples of conv_state ++ x.  Returns out like x:
         out[..., t] = act(bias + sum_k weight[:, k] * (conv_state ++ x)[..., state_len - W + 1 + t + k])."""
+    fp = _capi.fastpath() if activation in _ACT else None
+    if fp is not None:
+        out = _capi.fast_result(fp.conv1d_update(x, conv_state, weight, bias, _ACT[activation]), "thm_causal_conv1d_update")
+        if out is not None:
+            return out
     squeeze = x.dim() == 2
     if squeeze:
         x = x.unsqueeze(-1)
