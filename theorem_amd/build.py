@@ -31,6 +31,7 @@ SOURCES = [
     "recompute_w_u.hip",
     "chunk_fwd_h.hip",
     "chunk_fwd_h_f32.hip",
+    "chunk_fwd_h_scan.hip",
     "chunk_fwd_o.hip",
     "chunk_fwd_fused.hip",
     "chunk_fwd_rec.hip",
@@ -46,6 +47,7 @@ SOURCES = [
 # fp32 chunk_fwd_o (775 -> 884 and 883 -> 927 us), so it is not global.
 MFMA_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 UNIT_FLAGS = {
+    "chunk_fwd_h_scan.hip": MFMA_VGPR_FORM,
     "recompute_w_u.hip": MFMA_VGPR_FORM,
     "chunk_fwd_h.hip": MFMA_VGPR_FORM,
 }

@@ -14,6 +14,8 @@
 //     chunk_fwd_h_f32.hip), and the role-split kernel on small grids;
 //   * bf16: the DMA pipeline below on grids that fill the GPU, the role-split
 //     kernel (chunk_fwd_h_small.h) on smaller ones;
+//   * reference form on grids that do not fill the GPU: the chunks of a batch
+//     side by side and a scan over them (chunk_fwd_h_scan.hip);
 //   * delta form on grids that do not fill the GPU, with scratch memory
 //     (thm_chunk_fwd_h_ws): long sequences cut into segments (segments.h).
 // This unit is compiled with MFMA accumulators forced into VGPRs
@@ -25,6 +27,12 @@
 #include "segments.h"
 
 namespace thm {
+
+// chunk_fwd_h_scan.hip
+int h_scan_tile(int64_t BH, int64_t NT, int64_t K, int64_t V);
+hipError_t chunk_fwd_h_scan(bool f32, int tile, const void* k, const void* v, const void* g, const void* h0, void* h,
+                            void* ht, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, hipStream_t s);
+
 namespace {
 
 // ---------------------------------------------------------------------------
@@ -466,7 +474,9 @@ int h_entry(const void* k, const void* w, const void* vu, const void* g, const v
   char* const ws = (char*)workspace;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
-  if (f32) e = chunk_fwd_h_f32(delta, K, V, k, w, vu, g, h0, h, v_new, ht, ws, p.out, p.per, p.len, B, T, H, s);
+  if (const int tile = delta ? 0 : h_scan_tile(B * H, T / kBT, K, V))
+    e = chunk_fwd_h_scan(f32, tile, k, vu, g, h0, h, ht, B, T, H, K, V, s);
+  else if (f32) e = chunk_fwd_h_f32(delta, K, V, k, w, vu, g, h0, h, v_new, ht, ws, p.out, p.per, p.len, B, T, H, s);
   else if (delta) e = dispatch_kv<true>(K, V, k, w, vu, g, h0, h, v_new, ht, ws, p, B, T, H, s);
   else e = dispatch_kv<false>(K, V, k, w, vu, g, h0, h, v_new, ht, ws, p, B, T, H, s);
   return (int)e;
