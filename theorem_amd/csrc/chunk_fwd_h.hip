@@ -430,6 +430,7 @@ inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, 
   const int64_t NT = T / kBT, BH = B * H, nvt = V / kHBV;
   if (!delta || BH * nvt >= kHDmaMinGrid) return {1, 1, std::max<int64_t>(NT, 1)};
   if (f32) {
+    if (h_seg_cols(K, V) == 128) return seg::plan_segments(BH, NT, {nvt, (K + V) / 128, V / 128, 4.7, 5.3, 1.65, 6.4});
     const double period = K == 128 ? 4.7 : 2.5;
     return seg::plan_segments(BH, NT, {nvt, (K + V) / kHBV, nvt, K == 128 ? period : 1.7, period, 1.2, period});
   }

@@ -11,7 +11,8 @@
 // Replaces kernels/chunk_fwd_h/kernel.py:61-138 (Triton) and its launcher
 // kernel.py:141-191.
 //
-// One workgroup per (b, head, V-tile of 64 columns), 4 wavefronts; wave wv
+// One workgroup per (b, head, V-tile of 64 columns; 128 in some segment
+// launches), a wavefront for every 16; wave wv
 // owns state columns 16 wv .. 16 wv + 15 of the tile for the whole sequence,
 // held in MFMA accumulators (K/16 tiles of 16x16 fp32).  Per chunk:
 //   P1 (delta)  v_new^[j][n] = sum_kappa w[j][kappa] S[kappa][n]: the S
@@ -45,27 +46,35 @@ namespace thm {
 namespace {
 
 constexpr int kBT = 64;
-constexpr int kHBV = 64;        // V-tile width
-constexpr int kHThreads = 256;  // 4 wavefronts x 16 state columns
+constexpr int kHBV = 64;  // V-tile width
+// V-tile width of the segment launches (fp32 inputs).  Staging a chunk of k and
+// w (an fp32 -> bf16 hi + lo split of each) and its barriers take a large part
+// of a period and the LDS stage leaves one workgroup per CU: where P and V both
+// make whole tiles of 128, twice the waves share them (period 4.7 us for 64
+// columns -> 5.3 for 128).  B = 2, T = 2048, H = 8: transitions 42.4 -> 27.7 us,
+// outputs 37.2 -> 30.5, combine 8.4 -> 13.3 (8 segments instead of 5).
+constexpr int h_seg_cols(int64_t K, int64_t V) { return K == 128 && V == 128 ? 128 : kHBV; }
 
-template <typename IT, int K, int V, bool DELTA>
+// BV columns per workgroup, a wavefront for every 16.
+template <typename IT, int K, int V, bool DELTA, int BV>
 struct HCfg {
+  static constexpr int kThreads = 4 * BV;
   static constexpr bool kSplit = std::is_same<IT, float>::value;
   static constexpr int kEB = (int)sizeof(IT);
   static constexpr int kVE = 16 / kEB;               // elements per 16-byte load
   static constexpr int kKPitch = K + 8;              // bf16 elements (16-byte pad)
-  static constexpr int kUPitch = kHBV + kVE;         // IT elements (16-byte pad)
+  static constexpr int kUPitch = BV + kVE;         // IT elements (16-byte pad)
   static constexpr int kKTile = kBT * kKPitch;       // bf16 elements
   static constexpr int kUTile = kBT * kUPitch;       // IT elements
   // bf16 elements of one stage: k (hi[, lo]), w (hi[, lo]) when DELTA
   static constexpr int kBf16PerStage = (kSplit ? 2 : 1) * (DELTA ? 2 : 1) * kKTile;
   // per-thread 16-byte load slots of one chunk
   static constexpr int kKCPR = K / kVE;              // 16-byte chunks per k / w row
-  static constexpr int kKLoads = kBT * kKCPR / kHThreads;
-  static constexpr int kUCPR = kHBV / kVE;           // 16-byte chunks per u row of the tile
-  static constexpr int kULoads = kBT * kUCPR / kHThreads;
-  static_assert(kHThreads % kKCPR == 0 && kHThreads % kUCPR == 0, "slot mapping");
-  static_assert(kBT * kKCPR % kHThreads == 0 && kBT * kUCPR % kHThreads == 0, "slot count");
+  static constexpr int kKLoads = kBT * kKCPR / kThreads;
+  static constexpr int kUCPR = BV / kVE;           // 16-byte chunks per u row of the tile
+  static constexpr int kULoads = kBT * kUCPR / kThreads;
+  static_assert(kThreads % kKCPR == 0 && kThreads % kUCPR == 0, "slot mapping");
+  static_assert(kBT * kKCPR % kThreads == 0 && kBT * kUCPR % kThreads == 0, "slot count");
   static constexpr int kStageBytes =
       kBf16PerStage * 2 + kUTile * kEB + kBT * (int)sizeof(float);
   // Double-buffer the stage when two fit in 128 KiB of LDS; otherwise one stage
@@ -84,9 +93,9 @@ struct HStage {
 };
 
 // One chunk's loads, in registers.
-template <typename IT, int K, int V, bool DELTA>
+template <typename IT, int K, int V, bool DELTA, int BV>
 struct HPrefetch {
-  using C = HCfg<IT, K, V, DELTA>;
+  using C = HCfg<IT, K, V, DELTA, BV>;
   u32x4 k[C::kKLoads];
   u32x4 w[DELTA ? C::kKLoads : 1];
   u32x4 u[C::kULoads];
@@ -102,19 +111,19 @@ __device__ __forceinline__ const char* cptr(const void* p, int64_t byte_off) {
 // from the combine kernel's state in sbuf.  TRANS: the transition kernel of
 // this form, over column tiles of [P | Q]; only the final state is written, P
 // in A-operand blocks and Q in accumulator blocks, both fp32.
-template <typename IT, int K, int V, bool DELTA, bool HAS_G, bool DEEP, bool TRANS>
-__global__ void __launch_bounds__(kHThreads)
+template <typename IT, int K, int V, bool DELTA, bool HAS_G, bool DEEP, bool TRANS, int BV>
+__global__ void __launch_bounds__(4 * BV)
 chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT* __restrict__ vu,
                    const float* __restrict__ g, const float* __restrict__ h0,
                    float* __restrict__ hout, IT* __restrict__ vnew, float* __restrict__ ht,
                    char* __restrict__ pbuf, char* __restrict__ sbuf, int64_t T, int64_t H,
                    int64_t NTotal, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
-  using C = HCfg<IT, K, V, DELTA>;
+  using C = HCfg<IT, K, V, DELTA, BV>;
   using St = HStage<IT>;
-  using Pf = HPrefetch<IT, K, V, DELTA>;
+  using Pf = HPrefetch<IT, K, V, DELTA, BV>;
   constexpr int KB = K / 16;
-  constexpr int NPT = TRANS ? K / kHBV : 0;  // column tiles of P, ahead of the V-tiles
-  constexpr int NVT = NPT + V / kHBV;
+  constexpr int NPT = TRANS ? K / BV : 0;  // column tiles of P, ahead of the V-tiles
+  constexpr int NVT = NPT + V / BV;
   constexpr int EB = C::kEB;
   __shared__ __attribute__((aligned(16))) bf16 lds_b[C::kStages * C::kBf16PerStage];
   __shared__ __attribute__((aligned(16))) IT lds_u[C::kStages * C::kUTile];
@@ -126,7 +135,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   const int64_t b = bh / H, hh = bh % H;
   const bool is_p = TRANS && bt.vt < NPT;
   if (is_p && sg == 0) return;  // segment 0 starts from a known state (whole workgroup)
-  const int v0 = (int)(is_p ? bt.vt : bt.vt - NPT) * kHBV;  // first column, of P or of V
+  const int v0 = (int)(is_p ? bt.vt : bt.vt - NPT) * BV;  // first column, of P or of V
   const int uv0 = is_p ? 0 : v0;                            // P reads any column of u and drops it
   const seg::Span sp = seg::span_of(sg, len, NTotal);
   const int64_t NT = sp.n;
@@ -158,9 +167,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   const int kj0 = tid / C::kKCPR, kcol = (tid % C::kKCPR) * C::kVE;
   const int uj0 = tid / C::kUCPR, ucol0 = (tid % C::kUCPR) * C::kVE;
   const uint32_t koff0 = (uint32_t)(kj0 * tok_stride_k + kcol * EB);
-  const uint32_t kstep = (uint32_t)((kHThreads / C::kKCPR) * tok_stride_k);
+  const uint32_t kstep = (uint32_t)((C::kThreads / C::kKCPR) * tok_stride_k);
   const uint32_t uoff0 = (uint32_t)(uj0 * tok_stride_v + (uv0 + ucol0) * EB);
-  const uint32_t ustep = (uint32_t)((kHThreads / C::kUCPR) * tok_stride_v);
+  const uint32_t ustep = (uint32_t)((C::kThreads / C::kUCPR) * tok_stride_v);
   const uint32_t goff = (uint32_t)(lane * H * 4);  // every wave: token `lane` of the chunk
   // chunk bases (bytes from the tensor start), advanced per chunk
   const int64_t tok0 = b * T + sp.c0 * kBT;  // the segment's first token
@@ -190,7 +199,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   auto commit = [&](const Pf& pf, const St& st) {
 #pragma unroll
     for (int it = 0; it < C::kKLoads; ++it) {
-      const int off = (kj0 + it * (kHThreads / C::kKCPR)) * C::kKPitch + kcol;
+      const int off = (kj0 + it * (C::kThreads / C::kKCPR)) * C::kKPitch + kcol;
       if constexpr (C::kSplit) {
         float vals[4];
         unpack16(pf.k[it], vals, 0.f);
@@ -206,7 +215,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
     }
 #pragma unroll
     for (int it = 0; it < C::kULoads; ++it) {
-      const int off = (uj0 + it * (kHThreads / C::kUCPR)) * C::kUPitch + ucol0;
+      const int off = (uj0 + it * (C::kThreads / C::kUCPR)) * C::kUPitch + ucol0;
       *reinterpret_cast<u32x4*>(st.u + off) = pf.u[it];
     }
     if (wv == 0) st.g[lane] = pf.g;
@@ -397,29 +406,33 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
                     int64_t H, hipStream_t s) {
   const int64_t NT = T / kBT;
   const int64_t BH = B * H;
-  const int64_t wgs = BH * (V / kHBV) * p.out;
   char* const pbuf = ws;
   char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
-#define THM_H_LAUNCH(HG, DP, TR, GRID, NSEG, LEN)                                                           \
-  hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP, TR>), dim3((unsigned)(GRID)),             \
-                     dim3(kHThreads), 0, s, (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g,     \
+#define THM_H_LAUNCH(HG, DP, TR, BV, GRID, NSEG, LEN)                                                       \
+  hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP, TR, BV>), dim3((unsigned)(GRID)),         \
+                     dim3(4 * BV), 0, s, (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g,        \
                      (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, T, H, NT, BH, NSEG, LEN, p.per)
   if constexpr (DELTA) {
     if (p.out > 1) {
-      const int64_t nt = p.segs(NT), grid = BH * (nt - 1) * ((K + V) / kHBV);
-      if (g) THM_H_LAUNCH(true, false, true, grid, nt - 1, p.len);
-      else THM_H_LAUNCH(false, false, true, grid, nt - 1, p.len);
+      constexpr int BV = h_seg_cols(K, V);
+      const int64_t nt = p.segs(NT), grid = BH * (nt - 1) * ((K + V) / BV);
+      if (g) THM_H_LAUNCH(true, false, true, BV, grid, nt - 1, p.len);
+      else THM_H_LAUNCH(false, false, true, BV, grid, nt - 1, p.len);
       hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, true>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
                          pbuf, sbuf, BH, nt);
+      if (g) THM_H_LAUNCH(true, false, false, BV, BH * (V / BV) * p.out, p.out, p.len * p.per);
+      else THM_H_LAUNCH(false, false, false, BV, BH * (V / BV) * p.out, p.out, p.len * p.per);
+      return hipGetLastError();
     }
   }
-  const bool deep = p.out == 1 && wgs >= kHDmaMinGrid;  // bandwidth-bound regime
+  const int64_t wgs = BH * (V / kHBV);
+  const bool deep = wgs >= kHDmaMinGrid;  // bandwidth-bound regime
   if (g) {
-    if (deep) THM_H_LAUNCH(true, true, false, wgs, p.out, p.len * p.per);
-    else THM_H_LAUNCH(true, false, false, wgs, p.out, p.len * p.per);
+    if (deep) THM_H_LAUNCH(true, true, false, kHBV, wgs, 1, NT);
+    else THM_H_LAUNCH(true, false, false, kHBV, wgs, 1, NT);
   } else {
-    if (deep) THM_H_LAUNCH(false, true, false, wgs, p.out, p.len * p.per);
-    else THM_H_LAUNCH(false, false, false, wgs, p.out, p.len * p.per);
+    if (deep) THM_H_LAUNCH(false, true, false, kHBV, wgs, 1, NT);
+    else THM_H_LAUNCH(false, false, false, kHBV, wgs, 1, NT);
   }
 #undef THM_H_LAUNCH
   return hipGetLastError();
