@@ -425,7 +425,10 @@ hipError_t dispatch_kv(int64_t K, int64_t V, const void* k, const void* w, const
 //     50 -> 50; K = V = 64, 64 chunks 46 -> 32 -> 32;
 //   fp32, register kernel (at K = 64 the small-grid kernel in one piece): 16
 //     heads of K = V = 128, 32 chunks 137 -> 81 -> 80, 4 heads, 64 chunks 268
-//     -> 74 -> 74; 16 heads of K = V = 64, 64 chunks 97 -> 50 -> 50.
+//     -> 74 -> 74; 16 heads of K = V = 64, 64 chunks 97 -> 50 -> 50.  With 128
+//     columns a workgroup (h_seg_cols; kernel trace, sums of the three
+//     launches): 16 heads, 32 chunks 71, 4 heads, 64 chunks 77, 8 heads, 128
+//     chunks 126 (530 in one piece), 32 heads, 16 chunks 60 (72).
 inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, bool delta, bool f32) {
   const int64_t NT = T / kBT, BH = B * H, nvt = V / kHBV;
   if (!delta || BH * nvt >= kHDmaMinGrid) return {1, 1, std::max<int64_t>(NT, 1)};

@@ -420,8 +420,16 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
       else THM_H_LAUNCH(false, false, true, BV, grid, nt - 1, p.len);
       hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, true>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
                          pbuf, sbuf, BH, nt);
-      if (g) THM_H_LAUNCH(true, false, false, BV, BH * (V / BV) * p.out, p.out, p.len * p.per);
-      else THM_H_LAUNCH(false, false, false, BV, BH * (V / BV) * p.out, p.out, p.len * p.per);
+      // Outputs: tiles of 64 where they all run at once anyway (8 segments of 16
+      // heads 30.8 -> 28.6 us, 22 of 4 heads 21.6 -> 19.6, 13 of 8 57 -> 49).
+      const int64_t narrow = BH * (V / kHBV) * p.out, wide = BH * (V / BV) * p.out;
+      if (narrow <= device_cu_count()) {
+        if (g) THM_H_LAUNCH(true, false, false, kHBV, narrow, p.out, p.len * p.per);
+        else THM_H_LAUNCH(false, false, false, kHBV, narrow, p.out, p.len * p.per);
+      } else {
+        if (g) THM_H_LAUNCH(true, false, false, BV, wide, p.out, p.len * p.per);
+        else THM_H_LAUNCH(false, false, false, BV, wide, p.out, p.len * p.per);
+      }
       return hipGetLastError();
     }
   }
