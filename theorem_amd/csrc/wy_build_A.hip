@@ -16,12 +16,12 @@
 //      (fp32 k: bf16 hi + lo, three products).  The 10 lower blocks are spread
 //      over the 4 waves; every wave loads the tile's k (the repeats hit L2).
 //   2. L blocks (scaled by beta_i e^{g_i - g_j}, strict lower part) go to LDS.
-//   3. Wave w inverts the diagonal block w: lane c (< 16) owns column c and runs
-//      the 16-row substitution.
-//   4. The 6 off-diagonal blocks, 3 levels of independent blocks (3, 2, 1
-//      waves), each two fp32 MFMA products (v_mfma_f32_16x16x4_f32, exact fp32
-//      multiplies): T = sum L_im X_mj, then X_ij = -X_ii T, T passing through
-//      LDS to change from the accumulator to the operand layout.
+//   3. One wave inverts the four diagonal blocks: lane (d, c) owns column c of
+//      block d and runs the 16-row substitution.
+//   4. The other three waves take a block column of X each, its two to nine
+//      16x16 products on v_mfma_f32_16x16x4_f32 (exact fp32 multiplies): T = sum
+//      L_im X_mj, then X_ij = -X_ii T, each product's accumulators being the
+//      next one's B operand (wy_blocks.h invert_L).
 //   5. All 256 threads write A_c: 16-byte stores, 4 full 256-byte rows per
 //      wavefront instruction.
 // HBM traffic per tile: k, beta, g read once, A written once.
