@@ -274,6 +274,18 @@ int thm_wy_build_A(const void* k, const void* beta, const void* g, void* A,
                    int32_t chunk_size, int32_t k_dtype, int32_t sign, void* stream);
 
 /*
+ * thm_wy_build_A from per-token log decays: also writes their chunk-local
+ * cumulative sums g [B, T, H] fp32 (thm_chunk_local_cumsum), which A is formed
+ * with.
+ *   a [B, T, H] F32 or BF16 (a_dtype); gate_kind THM_GATE_IDENTITY or
+ *   THM_GATE_LOGSIGMOID.  k fp32 only (k_dtype = THM_DTYPE_F32).
+ */
+int thm_wy_build_A_gates(const void* k, const void* beta, const void* a, void* A, void* g,
+                         int64_t B, int64_t T, int64_t H, int64_t K, int32_t chunk_size,
+                         int32_t k_dtype, int32_t a_dtype, int32_t gate_kind, int32_t sign,
+                         void* stream);
+
+/*
  * Fused WY forward: the WY matrix A_c of thm_wy_build_A (same sign convention)
  * and the recompute_w_u products with it, in one pass, per chunk c:
  *   w_c = A_c (k_c * beta_c exp(g_c)),   u_c = A_c (v_c * beta_c)

@@ -158,6 +158,28 @@ def _fwd_records(q, k, v, beta, gate, gate_kind: int, scale: float, initial_stat
     return o, ht
 
 
+def _gates_with_A(k, beta, a) -> bool:
+    """Whether thm_wy_build_A_gates takes these; otherwise chunk_local_cumsum and
+    build_A do, with their checks."""
+    B, T, H, K = k.shape
+    return (k.is_cuda and beta.device == k.device and a.device == k.device and k.dtype == beta.dtype == torch.float32
+            and a.dtype in _capi.THM_DTYPE and T % BT == 0 and beta.shape == (B, T, H) and a.shape == (B, T, H))
+
+
+def _build_A_gates(k, beta, a, logsigmoid: bool):
+    """(A, g): build_A(k, beta, g) with g = chunk_local_cumsum(a), in one launch."""
+    B, T, H, K = k.shape
+    k, beta, a = (_capi.prep(t, n) for t, n in ((k, "k"), (beta, "beta"), (a, "a")))
+    A = torch.empty(B, T, H, BT, dtype=torch.float32, device=k.device)
+    g = torch.empty(B, T, H, dtype=torch.float32, device=k.device)
+    status = _capi.load_library().thm_wy_build_A_gates(
+        _capi.ptr(k), _capi.ptr(beta), _capi.ptr(a), _capi.ptr(A), _capi.ptr(g), B, T, H, K, BT,
+        _capi.THM_DTYPE[k.dtype], _capi.THM_DTYPE[a.dtype],
+        _capi.THM_GATE_LOGSIGMOID if logsigmoid else _capi.THM_GATE_IDENTITY, +1, _capi.stream_of(k))
+    _capi.check(status, "thm_wy_build_A_gates")
+    return A, g
+
+
 def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=None,
                                output_final_state: bool = False, A: torch.Tensor | None = None,
                                return_intermediates: bool = False, a: torch.Tensor | None = None,
@@ -189,7 +211,9 @@ def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=Non
             return _fwd_records(q, k, v, beta, g, _capi.THM_GATE_CUMULATIVE, scale, initial_state, output_final_state)
         kind = _capi.THM_GATE_LOGSIGMOID if a_logsigmoid else _capi.THM_GATE_IDENTITY
         return _fwd_records(q, k, v, beta, a, kind, scale, initial_state, output_final_state)
-    if a is not None:
+    if a is not None and A is None and not fused and not return_intermediates and _gates_with_A(k, beta, a):
+        A, g = _build_A_gates(k, beta, a, a_logsigmoid)
+    elif a is not None:
         g = chunk_local_cumsum(a, logsigmoid=a_logsigmoid)
     if fused and fused_form == "A":
         o, _, ht = chunk_fwd_fused_a(q, k, v, beta, A, g, scale, initial_state, output_final_state)

@@ -24,6 +24,9 @@
 //      next one's B operand (wy_blocks.h invert_L).
 //   5. All 256 threads write A_c: 16-byte stores, 4 full 256-byte rows per
 //      wavefront instruction.
+// With per-token log decays (thm_wy_build_A_gates) the tile's first wave also
+// forms and writes their cumulative sums, which it needs anyway: no launch of
+// their own (4.9 us at B = 2, T = 2048, H = 8).
 // HBM traffic per tile: k, beta, g read once, A written once.
 //
 // The record form (REC, bf16 k, sign +1; thm_chunk_gated_delta_rule_fwd) takes
@@ -105,8 +108,8 @@ __device__ __forceinline__ float form_gate(float x, int mode) {
 template <typename IT, int K, int SIGN, bool REC>
 __global__ void __launch_bounds__(kABThreads)
 wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
-                  const void* __restrict__ g, int gate_mode, void* __restrict__ out, int64_t T, int64_t H,
-                  int64_t NT) {
+                  const void* __restrict__ g, int gate_mode, void* __restrict__ out, float* __restrict__ g_out,
+                  int64_t T, int64_t H, int64_t NT) {
   constexpr bool kSplit = std::is_same<IT, float>::value;
   constexpr int KS = K / 32;  // contraction steps
   __shared__ __attribute__((aligned(16))) float Lb[10 * kBlk];  // L = sign M, lower blocks (diagonal blocks: strict lower part)
@@ -140,8 +143,11 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
     }
   }
   if (tid < kBT) {
-    sb[tid] = beta[(tok0 + tid) * H + h];
-    sg[tid] = form_gate(load_gate(g, gate_mode, (tok0 + tid) * H + h), gate_mode);
+    const int64_t row = (tok0 + tid) * H + h;
+    sb[tid] = beta[row];
+    const float gc = form_gate(load_gate(g, gate_mode, row), gate_mode);
+    sg[tid] = gc;
+    if (g_out) g_out[row] = gc;
   }
   lds_barrier();
 
@@ -272,7 +278,7 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
 
 template <typename IT, int K, int SIGN, bool REC>
 hipError_t launch_A(const void* k, const void* beta, const void* g, int gate_mode, void* out, int64_t B,
-                    int64_t T, int64_t H, hipStream_t s) {
+                    int64_t T, int64_t H, hipStream_t s, float* g_out = nullptr) {
   const int64_t NT = T / kBT;
   const int64_t tiles = B * NT * H;
   if constexpr (std::is_same<IT, bf16>::value) {
@@ -284,7 +290,7 @@ hipError_t launch_A(const void* k, const void* beta, const void* g, int gate_mod
     }
   }
   hipLaunchKernelGGL((wy_build_A_kernel<IT, K, SIGN, REC>), dim3((unsigned)tiles), dim3(kABThreads), 0, s,
-                     (const IT*)k, (const float*)beta, g, gate_mode, out, T, H, NT);
+                     (const IT*)k, (const float*)beta, g, gate_mode, out, g_out, T, H, NT);
   return hipGetLastError();
 }
 
@@ -332,5 +338,38 @@ extern "C" int thm_wy_build_A(const void* k, const void* beta, const void* g, vo
   else
     e = (K == 64) ? launch_A_sign<bf16, 64>(k, beta, g, A, B, T, H, sign, s)
                   : launch_A_sign<bf16, 128>(k, beta, g, A, B, T, H, sign, s);
+  return (int)e;
+}
+
+extern "C" int thm_wy_build_A_gates(const void* k, const void* beta, const void* a, void* A, void* g, int64_t B,
+                                    int64_t T, int64_t H, int64_t K, int32_t chunk_size, int32_t k_dtype,
+                                    int32_t a_dtype, int32_t gate_kind, int32_t sign, void* stream) {
+  using namespace thm;
+  if (chunk_size != kBT) return THM_ERR_BAD_ARGUMENT;
+  if (sign != 1 && sign != -1) return THM_ERR_BAD_ARGUMENT;
+  if (gate_kind != THM_GATE_IDENTITY && gate_kind != THM_GATE_LOGSIGMOID) return THM_ERR_BAD_ARGUMENT;
+  if (B < 0 || T < 0 || H <= 0 || K <= 0 || T % kBT) return THM_ERR_BAD_SHAPE;
+  if (k_dtype != THM_DTYPE_F32) return THM_ERR_BAD_DTYPE;  // fp32 k only: the one-tile kernel
+  if (a_dtype != THM_DTYPE_F32 && a_dtype != THM_DTYPE_BF16) return THM_ERR_BAD_DTYPE;
+  if (K != 64 && K != 128) return THM_ERR_UNSUPPORTED;
+  if (B == 0 || T == 0) return THM_OK;
+  if (!k || !beta || !a || !A || !g) return THM_ERR_NULL_POINTER;
+  if (((uintptr_t)k % 16) || ((uintptr_t)A % 16)) return THM_ERR_MISALIGNED;
+  if (((uintptr_t)beta % 4) || ((uintptr_t)g % 4) || ((uintptr_t)a % (a_dtype == THM_DTYPE_F32 ? 4 : 2)))
+    return THM_ERR_MISALIGNED;
+  if (B * (T / kBT) > (INT64_C(1) << 31) / H) return THM_ERR_BAD_SHAPE;
+  if (!launch_fits(B * (T / kBT) * H, kABThreads)) return THM_ERR_BAD_SHAPE;
+  if (kBT * H * K * 2 >= (INT64_C(1) << 32)) return THM_ERR_BAD_SHAPE;  // as thm_wy_build_A
+  const int mode = rec::kGatePerToken | (gate_kind == THM_GATE_LOGSIGMOID ? rec::kGateLogsigmoid : 0) |
+                   (a_dtype == THM_DTYPE_BF16 ? rec::kGateBf16 : 0);
+  hipStream_t s = (hipStream_t)stream;
+  float* const go = (float*)g;
+  hipError_t e;
+  if (K == 64)
+    e = sign < 0 ? launch_A<float, 64, -1, false>(k, beta, a, mode, A, B, T, H, s, go)
+                 : launch_A<float, 64, 1, false>(k, beta, a, mode, A, B, T, H, s, go);
+  else
+    e = sign < 0 ? launch_A<float, 128, -1, false>(k, beta, a, mode, A, B, T, H, s, go)
+                 : launch_A<float, 128, 1, false>(k, beta, a, mode, A, B, T, H, s, go);
   return (int)e;
 }

@@ -56,6 +56,7 @@ SIGNATURES = {
     "thm_chunk_gated_delta_rule_fwd": [_c_vp] * 9 + [_c_i64, ctypes.c_float] + [_c_i64] * 5 + [_c_i32] * 4 + [_c_vp],
     "thm_wy_build_A": [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64,
                        _c_i32, _c_i32, _c_i32, _c_vp],
+    "thm_wy_build_A_gates": [_c_vp] * 5 + [_c_i64] * 4 + [_c_i32] * 5 + [_c_vp],
     "thm_chunk_local_cumsum": [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_vp],
     "thm_wy_fwd": [_c_vp] * 6 + [_c_i64] * 5 + [_c_i32, _c_i32, _c_i32, _c_vp],
 }
