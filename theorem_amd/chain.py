@@ -46,6 +46,12 @@ def build_A(k: torch.Tensor, beta: torch.Tensor, g: torch.Tensor | None) -> torc
     return recompute_w_u.build_A(k, beta, g, sign=+1)
 
 
+def _check_state(initial_state, B: int, H: int, K: int, V: int) -> None:
+    """The kernels read B H K V floats from initial_state, whatever its shape."""
+    assert initial_state is None or initial_state.shape == (B, H, K, V), (
+        f"initial_state {tuple(initial_state.shape)} must be {(B, H, K, V)}")
+
+
 def wy_fwd(k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, g: torch.Tensor | None,
            sign: int = +1) -> tuple[torch.Tensor, torch.Tensor]:
     """(w, u) = recompute_w_u(k, v, beta, A, g) with A = build_A(k, beta, g, sign)
@@ -76,7 +82,8 @@ def chunk_fwd_fused(q, k, w, u, g, scale: float, initial_state=None, output_fina
     B, T, H, K = k.shape
     V = u.shape[-1]
     assert T % BT == 0, f"T={T} must be a multiple of {BT}"
-    assert q.shape == k.shape == w.shape and u.shape[:3] == (B, T, H)
+    assert q.shape == k.shape == w.shape and u.shape[:3] == (B, T, H) and (g is None or g.shape == (B, T, H))
+    _check_state(initial_state, B, H, K, V)
     assert q.dtype == k.dtype == w.dtype == u.dtype == torch.bfloat16, "the fused path is bf16-only"
     _capi.require_device(q, k, w, u, g, initial_state)
     for name, t in (("g", g), ("initial_state", initial_state)):
@@ -105,6 +112,7 @@ def chunk_fwd_fused_a(q, k, v, beta, A, g, scale: float, initial_state=None, out
     assert T % BT == 0, f"T={T} must be a multiple of {BT}"
     assert q.shape == k.shape and v.shape[:3] == (B, T, H) and beta.shape == (B, T, H)
     assert A.shape == (B, T, H, BT) and (g is None or g.shape == (B, T, H))
+    _check_state(initial_state, B, H, K, V)
     assert q.dtype == k.dtype == v.dtype == torch.bfloat16, "the fused path is bf16-only"
     _capi.require_device(q, k, v, beta, A, g, initial_state)
     for name, t in (("beta", beta), ("A", A), ("g", g), ("initial_state", initial_state)):
@@ -136,6 +144,7 @@ def _fwd_records(q, k, v, beta, gate, gate_kind: int, scale: float, initial_stat
     assert T % BT == 0, f"T={T} must be a multiple of {BT}"
     assert q.shape == k.shape and v.shape[:3] == (B, T, H) and beta.shape == (B, T, H)
     assert gate is None or gate.shape == (B, T, H)
+    _check_state(initial_state, B, H, K, V)
     assert q.dtype == k.dtype == v.dtype == torch.bfloat16, "the fused path is bf16-only"
     _capi.require_device(q, k, v, beta, gate, initial_state)
     for name, t in (("beta", beta), ("initial_state", initial_state)):
