@@ -5,8 +5,8 @@ bf16 default): chunk records, segment transitions and the output kernel.
 Against the float64 oracle (oracle/deltanet.py), rtol = atol = 1e-2 as the
 other bf16 paths, and against chunk_fwd_fused_a on the same inputs (A from the
 A-builder, the recurrence in one piece), whose error it may not exceed by more
-than half: the segments round P S + Q to ~2^-16, below the bf16 rounding of S
-inside every chunk.
+than half: both round S to bf16 inside every chunk, the segments also the columns
+of P; P S + Q itself is formed in fp32.
 """
 from __future__ import annotations
 

@@ -1,8 +1,8 @@
 """GPU parity of chunk_fwd_h's segmented delta form (thm_chunk_fwd_h_ws): every
 output against the float64 oracle and against thm_chunk_fwd_h (one piece) on
 the same inputs.  rtol = atol = 1e-2 (bf16) and 1e-3 (fp32, whose products
-carry ~2^-16); the error may not exceed the one-piece form's by half: P S + Q
-is formed to ~2^-16 (bf16 inputs) or in exact fp32 products (fp32 inputs)."""
+carry ~2^-16); the error may not exceed the one-piece form's by half (P S + Q
+is formed in exact fp32 products)."""
 from __future__ import annotations
 
 import pytest

@@ -389,7 +389,7 @@ hipError_t launch_h_segments(const void* k, const void* w, const void* u, const 
   if (g) THM_H_TRANS_LAUNCH(true);
   else THM_H_TRANS_LAUNCH(false);
 #undef THM_H_TRANS_LAUNCH
-  hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, false>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, pbuf,
+  hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, pbuf,
                      sbuf, BH, nt);
   return launch_h_dma<K, V, true>(k, w, u, g, h0, h, vnew, ht, sbuf, p, B, T, H, s);
 }
@@ -437,7 +437,7 @@ inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, 
     const double period = K == 128 ? 4.7 : 2.5;
     return seg::plan_segments(BH, NT, {nvt, (K + V) / kHBV, nvt, K == 128 ? period : 1.7, period, 1.2, period});
   }
-  return seg::plan_segments(BH, NT, {V / 32, 1, nvt, 1.2, 2.2, 0.9, 2.6});
+  return seg::plan_segments(BH, NT, {V / 32, 1, nvt, 1.2, 2.2, K == 128 ? 1.65 : 0.9, 2.6});
 }
 
 int h_entry(const void* k, const void* w, const void* vu, const void* g, const void* h0, void* h, void* v_new,

@@ -418,7 +418,7 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
       const int64_t nt = p.segs(NT), grid = BH * (nt - 1) * ((K + V) / BV);
       if (g) THM_H_LAUNCH(true, false, true, BV, grid, nt - 1, p.len);
       else THM_H_LAUNCH(false, false, true, BV, grid, nt - 1, p.len);
-      hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V, true>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
+      hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
                          pbuf, sbuf, BH, nt);
       // Outputs: tiles of 64 where they all run at once anyway (8 segments of 16
       // heads 30.8 -> 28.6 us, 22 of 4 heads 21.6 -> 19.6, 13 of 8 57 -> 49).

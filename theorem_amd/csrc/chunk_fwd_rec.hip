@@ -308,14 +308,14 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
 }
 
 // Measured at K = V = 128: period 2.0-2.1 us (outputs), 2.3-2.4 (transitions),
-// 0.9 per combine step; whole forwards, unsegmented -> best of ten plans ->
+// 1.65 per combine step; whole forwards, unsegmented -> best of ten plans ->
 // this rule's choice: 16 heads: 16 chunks 42 -> 36 -> 36 us, 32 chunks 77 ->
 // 48 -> 48, 128 chunks 276 -> 107 -> 107; 32 heads, 32 chunks 84 -> 66; 4
 // heads, 64 chunks 140 -> 55.  128 workgroups or more without segments do not
 // gain (64 heads, 32 chunks: 86 unsegmented, 96 at best).
-inline Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t V) {
+inline Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t nvt = V / kTileV;
-  return plan_segments(B * H, T / kBT, {nvt, 1, nvt, 2.02, 2.4, 0.9, 2.1});
+  return plan_segments(B * H, T / kBT, {nvt, 1, nvt, 2.02, 2.4, K == 128 ? 1.65 : 0.9, 2.1});
 }
 
 struct Workspace {
@@ -347,7 +347,7 @@ hipError_t launch_rec(const void* q, const void* k, const void* v, const void* b
                        dim3(rec::TCfg<K, V, false>::kThreads), 0, s, (const bf16*)k, (const bf16*)nullptr, (const bf16*)v,
                        (const float*)nullptr, ws + w.records, (const float*)h0, ws + w.pbuf, ws + w.sbuf, T, H, NT, BH,
                        p.len);
-    hipLaunchKernelGGL((chunk_combine_kernel<K, V, false>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, ws + w.pbuf,
+    hipLaunchKernelGGL((chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, ws + w.pbuf,
                        ws + w.sbuf, BH, nt);
   }
   hipLaunchKernelGGL((chunk_output_kernel<K, V>), dim3((unsigned)(BH * (V / kTileV) * p.out)), dim3(rec::kOThreads), 0,
@@ -364,7 +364,7 @@ extern "C" int64_t thm_chunk_gated_delta_rule_workspace(int64_t B, int64_t T, in
   if (B < 0 || T < 0 || H <= 0 || T % kBT || (K != 64 && K != 128) || (V != 64 && V != 128)) return THM_ERR_BAD_SHAPE;
   if (B == 0 || T == 0) return 0;
   if (B > (INT64_C(1) << 31) / H || B * (T / kBT) > (INT64_C(1) << 31) / H) return THM_ERR_BAD_SHAPE;
-  return workspace_of(B, T, H, K, V, plan_of(B, T, H, V)).bytes;
+  return workspace_of(B, T, H, K, V, plan_of(B, T, H, K, V)).bytes;
 }
 
 extern "C" int thm_chunk_gated_delta_rule_fwd(const void* q, const void* k, const void* v, const void* beta,
@@ -394,7 +394,7 @@ extern "C" int thm_chunk_gated_delta_rule_fwd(const void* q, const void* k, cons
   if (((uintptr_t)gate % (gate_dtype == THM_DTYPE_F32 ? 4 : 2)) || ((uintptr_t)o % 8)) return THM_ERR_MISALIGNED;
   if (B > (INT64_C(1) << 31) / H) return THM_ERR_BAD_SHAPE;
   if (T > 0 && B * (T / kBT) > (INT64_C(1) << 31) / H) return THM_ERR_BAD_SHAPE;
-  const Plan plan = plan_of(B, T, H, V);
+  const Plan plan = plan_of(B, T, H, K, V);
   // The largest grids: records (one tile per workgroup), transitions, outputs.
   if (!launch_fits(B * (T / kBT) * H, 256) || !launch_fits(B * H * (V / kTileV) * plan.out * plan.per, 512))
     return THM_ERR_BAD_SHAPE;

@@ -306,11 +306,10 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
   wait_vmcnt<0>();  // no DMA may still target this workgroup's LDS when it exits
   if (!active) return;
 
-  // P in 16 x 16 blocks (row block, column block) of A-operand lanes, as the
-  // record's A blocks: lane (grp, li) holds P[16 kb + li][16 nb + 4 grp .. + 3]
-  // as 4 bf16 hi then 4 lo; after acc_to_row_quads lane (g, 4 a + b) holds row
-  // 4 g + a, columns 4 b .. + 3.  Q in blocks (column block, row block) of fp32
-  // accumulator lanes.
+  // P in 16 x 16 blocks (row block, column block) of A-operand lanes: lane
+  // (grp, li) holds P[16 kb + li][16 nb + 4 grp .. + 3]; after acc_to_row_quads
+  // lane (g, 4 a + b) holds row 4 g + a, columns 4 b .. + 3.  Q in blocks
+  // (column block, row block) of accumulator lanes.
   if (is_p) {
     const int slot = 16 * (li & 3) + 4 * grp + (li >> 2);
     char* const pb = pbuf + rec::p_off(seg, bh, BH, K) + (n0 / 16) * 1024 + 16 * slot;
@@ -318,7 +317,7 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        *reinterpret_cast<u32x4*>(pb + (kb * KB + ct) * 1024) = hi_lo4(acc_to_row_quads(S[ct][kb]));
+        *reinterpret_cast<f32x4*>(pb + (kb * KB + ct) * 1024) = acc_to_row_quads(S[ct][kb]);
   } else {
     char* const sb = sbuf + rec::s_off(seg, bh, BH, K, V) + (n0 / 16) * KB * 1024 + 16 * lane;
 #pragma unroll
@@ -332,17 +331,16 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
 // Combine kernel: S_{s+1} = P_s S_s + Q_s for s = 1 .. nseg - 2, in place of
 // Q_s (S_1 = Q_0).  One workgroup of K / 16 wavefronts per (b, head, 16
 // columns); wave w forms row tile w of the new state and hands it to the
-// others through LDS.  P and S as bf16 hi + lo, three products (hi hi, hi lo,
-// lo hi): ~2^-16 relative; F32 (fp32 inputs): P and S as fp32 on
-// v_mfma_f32_16x16x4_f32, exact products.  A serial chain of small steps: P and Q of the
-// next two steps are in flight during one, and the three products run in
-// accumulators of their own.
-template <int K, int V, bool F32>
+// others through LDS.  P and S as fp32 on v_mfma_f32_16x16x4_f32, exact
+// products: the state is carried in fp32 from one end of a sequence to the
+// other, as in one piece.  A serial chain of small steps: P and Q of the next
+// two steps are in flight during one, and the products run in two accumulators.
+template <int K, int V>
 __global__ void __launch_bounds__(4 * K)
 chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int64_t BH, int64_t nseg) {
   constexpr int KB = K / 16, NVB = V / 16;
   constexpr int kAhead = 2;
-  __shared__ __attribute__((aligned(16))) u32x4 xs[2][KB][64];  // one row tile's 4 rows per lane: hi, lo, or fp32
+  __shared__ __attribute__((aligned(16))) f32x4 xs[2][KB][64];  // one row tile's 4 rows per lane
   const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH, NVB);  // one XCD reads one (b, head)'s P
   const int wi = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -351,12 +349,12 @@ chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int
     return reinterpret_cast<f32x4*>(sbuf + rec::s_off(s, bt.bh, BH, K, V) + (bt.vt * KB + wi) * 1024 + 16 * lane);
   };
   f32x4 qn[kAhead];
-  u32x4 pn[kAhead][KB];
+  f32x4 pn[kAhead][KB];
   auto load = [&](int64_t s, int i) {
     qn[i] = *q_at(s);
     const char* pb = pbuf + rec::p_off(s, bt.bh, BH, K) + wi * KB * 1024 + 16 * lane;
 #pragma unroll
-    for (int nb = 0; nb < KB; ++nb) pn[i][nb] = ldg16(pb + nb * 1024);
+    for (int nb = 0; nb < KB; ++nb) pn[i][nb] = *reinterpret_cast<const f32x4*>(pb + nb * 1024);
   };
   const int64_t last = nseg - 2;
   f32x4 S = *q_at(0);
@@ -364,35 +362,21 @@ chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int
   for (int i = 0; i < kAhead; ++i) load(1 + i < last ? 1 + i : last, i);
   auto step = [&](int64_t s, int i) {
     const int f = (int)(s & 1);
-    xs[f][wi][lane] = F32 ? __builtin_bit_cast(u32x4, S) : hi_lo4(S);
-    u32x4 p[KB];
+    xs[f][wi][lane] = S;
+    f32x4 p[KB];
 #pragma unroll
     for (int nb = 0; nb < KB; ++nb) p[nb] = pn[i][nb];
-    f32x4 hh = qn[i], hl = zero4(), lh = zero4();
+    f32x4 acc[2] = {qn[i], zero4()};
     load(s + kAhead < last ? s + kAhead : last, i);
     lds_barrier();  // S_s is in LDS (the other buffer's readers finished before this barrier)
-    if constexpr (F32) {
 #pragma unroll
-      for (int nb = 0; nb < KB; ++nb) {
-        const f32x4 a = __builtin_bit_cast(f32x4, p[nb]), x = __builtin_bit_cast(f32x4, xs[f][nb][lane]);
-        f32x4& acc = nb & 1 ? hl : hh;
+    for (int nb = 0; nb < KB; ++nb) {
+      const f32x4 x = xs[f][nb][lane];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], x[q], acc, 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int s2 = 0; s2 < KB / 2; ++s2) {
-        const u32x4 a = p[2 * s2], b = p[2 * s2 + 1], x = xs[f][2 * s2][lane], y = xs[f][2 * s2 + 1][lane];
-        const bf16x8 ph = __builtin_bit_cast(bf16x8, u32x4{a[0], a[1], b[0], b[1]});
-        const bf16x8 pl = __builtin_bit_cast(bf16x8, u32x4{a[2], a[3], b[2], b[3]});
-        const bf16x8 sh = __builtin_bit_cast(bf16x8, u32x4{x[0], x[1], y[0], y[1]});
-        const bf16x8 sl = __builtin_bit_cast(bf16x8, u32x4{x[2], x[3], y[2], y[3]});
-        hh = mfma16x16x32(ph, sh, hh);
-        hl = mfma16x16x32(ph, sl, hl);
-        lh = mfma16x16x32(pl, sh, lh);
-      }
+      for (int q = 0; q < 4; ++q)
+        acc[nb & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[nb][q], x[q], acc[nb & 1], 0, 0, 0);
     }
-    S = hh + (hl + lh);
+    S = acc[0] + acc[1];
     *q_at(s) = S;
   };
   for (int64_t s = 1; s <= last; s += kAhead) {
