@@ -153,7 +153,9 @@ int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, const void* g,
  * alone leave the GPU idle, they are cut into segments that run side by side
  * (chosen from the shape, the dtype and the device's CU count only, so results
  * are deterministic per shape; they agree with thm_chunk_fwd_h's to the
- * rounding of the state).  workspace: at least thm_chunk_fwd_h_workspace bytes
+ * rounding of the state).  The segments' maps are formed without the states
+ * and may overflow where those do not: columns whose states at the segments'
+ * starts are not all finite are walked in one piece instead.  workspace: at least thm_chunk_fwd_h_workspace bytes
  * (0: none needed), 16-byte aligned, owned by the call until it has run on
  * `stream`; otherwise as thm_chunk_fwd_h.
  */

@@ -72,7 +72,7 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
                        const bf16* __restrict__ vu, const float* __restrict__ g,
                        const float* __restrict__ h0, float* __restrict__ hout,
                        bf16* __restrict__ vnew, float* __restrict__ ht, const char* __restrict__ sbuf,
-                       int64_t T, int64_t H, int64_t NT, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
+                       const uint32_t* __restrict__ redo, int64_t T, int64_t H, int64_t NT, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
   using C = PCfg<K, KS, NS, DELTA, HAS_G, STORE_VN>;
   constexpr int NVT = V / kHBV;
   __shared__ __attribute__((aligned(1024))) char lds[C::kLds];
@@ -80,8 +80,9 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH * nseg, NVT);
   const int64_t sg = bt.bh / BH, bh = bt.bh - sg * BH;
   const int64_t b = bh / H, hh = bh % H;
-  const seg::Span sp = seg::span_of(sg, len, NT);
+  seg::Span sp = seg::span_of(sg, len, NT);
   const int v0 = (int)bt.vt * kHBV;
+  const bool whole = nseg > 1 && seg::redo_columns<V>(redo, bh, v0, kHBV);
 
   const int tid = threadIdx.x;
   const int wi = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -162,6 +163,10 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   // Retire the state loads here: a load still pending at the loop entry would
   // make the compiler wait for every outstanding operation inside the loop.
   wait_vmcnt<0>();
+  if (whole) {
+    if (sg > 0) return;  // (uniform over the workgroup)
+    sp.n = NT;
+  }
 
   // Store offsets of the row-quad layout (acc_to_row_quads) for this wave's
   // first 16-row tile of h and of v_new; later tiles add 16 rows.
@@ -332,7 +337,7 @@ chunk_fwd_h_dma_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w,
   // Drain: no DMA may still target this workgroup's LDS when it exits.
   wait_vmcnt<0>();
 
-  if (ht && sg == nseg - 1) {
+  if (ht && sp.c0 + sp.n == NT) {
 #pragma unroll
     for (int kb = 0; kb < C::KBH; ++kb)
 #pragma unroll
@@ -349,8 +354,8 @@ using pipe::kHStages;  // DMA ring depth of the bf16 pipeline
 
 template <int K, int V, bool DELTA>
 hipError_t launch_h_dma(const void* k, const void* w, const void* vu, const void* g, const void* h0,
-                        void* h, void* vnew, void* ht, const void* sbuf, const seg::Plan& p, int64_t B, int64_t T,
-                        int64_t H, hipStream_t s) {
+                        void* h, void* vnew, void* ht, const void* sbuf, const void* redo, const seg::Plan& p,
+                        int64_t B, int64_t T, int64_t H, hipStream_t s) {
   const int64_t NT = T / kBT;
   const int64_t BH = B * H;
   const dim3 grid((unsigned)(BH * (V / kHBV) * p.out));
@@ -359,8 +364,8 @@ hipError_t launch_h_dma(const void* k, const void* w, const void* vu, const void
   hipLaunchKernelGGL((chunk_fwd_h_dma_kernel<K, V, KS, NS, DELTA, HG, SV>), grid,              \
                      dim3(PCfg<K, KS, NS, DELTA, HG, SV>::kThreads), 0, s, (const bf16*)k,     \
                      (const bf16*)w, (const bf16*)vu, (const float*)g, (const float*)h0,       \
-                     (float*)h, (bf16*)vnew, (float*)ht, (const char*)sbuf, T, H, NT, BH, p.out,      \
-                     p.len * p.per, p.per)
+                     (float*)h, (bf16*)vnew, (float*)ht, (const char*)sbuf, (const uint32_t*)redo, T, \
+                     H, NT, BH, p.out, p.len * p.per, p.per)
   const bool sv = DELTA && vnew != nullptr;
   if (g) {
     if (sv) THM_H_DMA_LAUNCH(true, DELTA);
@@ -382,6 +387,7 @@ hipError_t launch_h_segments(const void* k, const void* w, const void* u, const 
   const int64_t NT = T / kBT, BH = B * H, nt = p.segs(NT);
   char* const pbuf = ws;
   char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
+  char* const redo = sbuf + seg::s_bytes(p, BH, NT, K, V);
 #define THM_H_TRANS_LAUNCH(HG)                                                                                     \
   hipLaunchKernelGGL((seg::chunk_transition_kernel<K, V, true, HG>), dim3((unsigned)(BH * (nt - 1))),              \
                      dim3(rec::TCfg<K, V, true>::kThreads), 0, s, (const bf16*)k, (const bf16*)w, (const bf16*)u,  \
@@ -390,8 +396,8 @@ hipError_t launch_h_segments(const void* k, const void* w, const void* u, const 
   else THM_H_TRANS_LAUNCH(false);
 #undef THM_H_TRANS_LAUNCH
   hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, pbuf,
-                     sbuf, BH, nt);
-  return launch_h_dma<K, V, true>(k, w, u, g, h0, h, vnew, ht, sbuf, p, B, T, H, s);
+                     sbuf, (uint32_t*)redo, BH, nt);
+  return launch_h_dma<K, V, true>(k, w, u, g, h0, h, vnew, ht, sbuf, redo, p, B, T, H, s);
 }
 
 template <bool DELTA, int K, int V>
@@ -402,7 +408,7 @@ hipError_t launch_kv(const void* k, const void* w, const void* vu, const void* g
     if (p.out > 1) return launch_h_segments<K, V>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
   }
   if (B * H * (V / kHBV) >= kHDmaMinGrid)
-    return launch_h_dma<K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, nullptr, p, B, T, H, s);
+    return launch_h_dma<K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, nullptr, nullptr, p, B, T, H, s);
   return launch_h_small<bf16, K, V, kHSmallNW, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
 }
 
@@ -440,6 +446,11 @@ inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, 
   return seg::plan_segments(BH, NT, {V / 32, 1, nvt, 1.2, 2.2, K == 128 ? 1.65 : 0.9, 2.6});
 }
 
+inline int64_t workspace_bytes_of(const seg::Plan& p, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
+  const int64_t BH = B * H, NT = T / kBT;
+  return seg::p_bytes(p, BH, NT, K) + seg::s_bytes(p, BH, NT, K, V) + seg::redo_bytes(p, BH, V);
+}
+
 int h_entry(const void* k, const void* w, const void* vu, const void* g, const void* h0, void* h, void* v_new,
             void* ht, void* workspace, int64_t workspace_bytes, bool segments, int64_t B, int64_t T, int64_t H,
             int64_t K, int64_t V, int32_t chunk_size, int32_t kv_dtype, int32_t flags, void* stream) {
@@ -470,7 +481,7 @@ int h_entry(const void* k, const void* w, const void* vu, const void* g, const v
   seg::Plan p = {1, 1, std::max<int64_t>(T / kBT, 1)};
   if (segments) {
     p = plan_of(B, T, H, K, V, delta, f32);
-    const int64_t need = seg::p_bytes(p, B * H, T / kBT, K) + seg::s_bytes(p, B * H, T / kBT, K, V);
+    const int64_t need = workspace_bytes_of(p, B, T, H, K, V);
     if (workspace_bytes < need) return THM_ERR_BAD_ARGUMENT;
     if (need > 0 && !workspace) return THM_ERR_NULL_POINTER;
     if ((uintptr_t)workspace % 16) return THM_ERR_MISALIGNED;
@@ -512,5 +523,5 @@ extern "C" int64_t thm_chunk_fwd_h_workspace(int64_t B, int64_t T, int64_t H, in
       B > (INT64_C(1) << 31) / H)
     return 0;  // nothing to compute, or a call thm_chunk_fwd_h_ws refuses
   const seg::Plan p = plan_of(B, T, H, K, V, (flags & THM_H_DELTA) != 0, kv_dtype == THM_DTYPE_F32);
-  return seg::p_bytes(p, B * H, T / kBT, K) + seg::s_bytes(p, B * H, T / kBT, K, V);
+  return workspace_bytes_of(p, B, T, H, K, V);
 }

@@ -116,7 +116,8 @@ __global__ void __launch_bounds__(4 * BV)
 chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT* __restrict__ vu,
                    const float* __restrict__ g, const float* __restrict__ h0,
                    float* __restrict__ hout, IT* __restrict__ vnew, float* __restrict__ ht,
-                   char* __restrict__ pbuf, char* __restrict__ sbuf, int64_t T, int64_t H,
+                   char* __restrict__ pbuf, char* __restrict__ sbuf, const uint32_t* __restrict__ redo,
+                   int64_t T, int64_t H,
                    int64_t NTotal, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
   using C = HCfg<IT, K, V, DELTA, BV>;
   using St = HStage<IT>;
@@ -138,7 +139,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   const int v0 = (int)(is_p ? bt.vt : bt.vt - NPT) * BV;  // first column, of P or of V
   const int uv0 = is_p ? 0 : v0;                            // P reads any column of u and drops it
   const seg::Span sp = seg::span_of(sg, len, NTotal);
-  const int64_t NT = sp.n;
+  int64_t NT = sp.n;
+  bool whole = false;
+  if constexpr (!TRANS) whole = nseg > 1 && seg::redo_columns<V>(redo, bh, v0, BV);
 
   auto stage = [&](int i) {
     St st;
@@ -263,6 +266,10 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   // and committed at its end.  DEEP is faster on large grids (fp32 at config
   // 4: 890 -> 779 us) and slower on small ones (fp32 config 3: 38.9 -> 46.7
   // us), where the chunk's own latency chain, not the loads, sets the period.
+  if (whole) {
+    if (sg > 0) return;  // (uniform over the workgroup)
+    NT = NTotal;
+  }
   Pf pa, pb;
   if (NT > 0) {
     prefetch(pa, 0);
@@ -386,7 +393,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
       else
         *reinterpret_cast<f32x4*>(sbuf + rec::s_off(sg, bh, BH, K, V) + ((v0 / 16 + wv) * KB + kb) * 1024 + 16 * lane) = S[kb];
     }
-  } else if (ht && sg == nseg - 1) {
+  } else if (ht && sp.c0 + NT == NTotal) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -408,10 +415,11 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
   const int64_t BH = B * H;
   char* const pbuf = ws;
   char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
+  uint32_t* const redo = (uint32_t*)(sbuf + seg::s_bytes(p, BH, NT, K, V));
 #define THM_H_LAUNCH(HG, DP, TR, BV, GRID, NSEG, LEN)                                                       \
   hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP, TR, BV>), dim3((unsigned)(GRID)),         \
                      dim3(4 * BV), 0, s, (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g,        \
-                     (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, T, H, NT, BH, NSEG, LEN, p.per)
+                     (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, redo, T, H, NT, BH, NSEG, LEN, p.per)
   if constexpr (DELTA) {
     if (p.out > 1) {
       constexpr int BV = h_seg_cols(K, V);
@@ -419,7 +427,7 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
       if (g) THM_H_LAUNCH(true, false, true, BV, grid, nt - 1, p.len);
       else THM_H_LAUNCH(false, false, true, BV, grid, nt - 1, p.len);
       hipLaunchKernelGGL((seg::chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s,
-                         pbuf, sbuf, BH, nt);
+                         pbuf, sbuf, redo, BH, nt);
       // Outputs: tiles of 64 where they all run at once anyway (8 segments of 16
       // heads 30.8 -> 28.6 us, 22 of 4 heads 21.6 -> 19.6, 13 of 8 57 -> 49).
       const int64_t narrow = BH * (V / kHBV) * p.out, wide = BH * (V / BV) * p.out;

@@ -60,8 +60,8 @@ template <int K, int V>
 __global__ void __launch_bounds__(rec::kOThreads)
 chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
                     const char* __restrict__ records, const float* __restrict__ h0,
-                    const char* __restrict__ sbuf, bf16* __restrict__ o, float* __restrict__ ht, float scale,
-                    int64_t T, int64_t H, int64_t NT, int64_t BH, int64_t nseg, int64_t len, int64_t t_per_seg) {
+                    const char* __restrict__ sbuf, const uint32_t* __restrict__ redo, bf16* __restrict__ o,
+                    float* __restrict__ ht, float scale, int64_t T, int64_t H, int64_t NT, int64_t BH, int64_t nseg, int64_t len, int64_t t_per_seg) {
   using C = rec::OCfg<K>;
   constexpr int NVT = V / kTileV, KB2 = C::KB / 2;
   __shared__ __attribute__((aligned(1024))) char lds[C::kLds];
@@ -70,7 +70,8 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
   const int64_t seg = bt.bh / BH, bh = bt.bh - seg * BH;
   const int64_t b = bh / H, hh = bh - b * H;
   const int v0 = (int)bt.vt * kTileV;
-  const Span sp = span_of(seg, len, NT);
+  Span sp = span_of(seg, len, NT);
+  const bool whole = nseg > 1 && redo_columns<V>(redo, bh, v0, kTileV);
 
   const int tid = threadIdx.x;
   const int wi = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -149,7 +150,7 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
     issue_av(0, 0);
 #pragma unroll
     for (int m = 0; m < 3; ++m) issue_part(0, 0, m);
-    issue_av(sp.n > 1 ? 1 : 0, 1);
+    issue_av(sp.c0 + 1 < NT ? 1 : 0, 1);  // (past a segment of one chunk, for `whole`)
   }
   // State S[kappa = 16 kb + 4 grp + r][n = v0 + 16 wq + li] in S[kb][r] (state waves).
   f32x4 S[C::KB];
@@ -170,6 +171,10 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
     }
   }
   wait_vmcnt<0>();  // the state and the first tiles; the loop counts from here
+  if (whole) {
+    if (seg > 0) return;  // (uniform over the workgroup)
+    sp.n = NT;
+  }
 
   for (int64_t c = 0; c < sp.n; ++c) {
     const int s = (int)(c & 1);
@@ -299,7 +304,7 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
   }
   wait_vmcnt<0>();  // no DMA may still target this workgroup's LDS when it exits
 
-  if (state_wave && ht && seg == nseg - 1) {
+  if (state_wave && ht && sp.c0 + sp.n == NT) {
 #pragma unroll
     for (int kb = 0; kb < C::KB; ++kb)
 #pragma unroll
@@ -319,7 +324,7 @@ inline Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
 }
 
 struct Workspace {
-  int64_t records, pbuf, sbuf, bytes;
+  int64_t records, pbuf, sbuf, redo, bytes;
 };
 inline Workspace workspace_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, const Plan& p) {
   const int64_t NT = T / kBT, BH = B * H;
@@ -327,7 +332,8 @@ inline Workspace workspace_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_
   w.records = 0;
   w.pbuf = BH * NT * rec::kBytes;
   w.sbuf = w.pbuf + p_bytes(p, BH, NT, K);
-  w.bytes = w.sbuf + s_bytes(p, BH, NT, K, V);
+  w.redo = w.sbuf + s_bytes(p, BH, NT, K, V);
+  w.bytes = w.redo + redo_bytes(p, BH, V);
   return w;
 }
 
@@ -348,11 +354,11 @@ hipError_t launch_rec(const void* q, const void* k, const void* v, const void* b
                        (const float*)nullptr, ws + w.records, (const float*)h0, ws + w.pbuf, ws + w.sbuf, T, H, NT, BH,
                        p.len);
     hipLaunchKernelGGL((chunk_combine_kernel<K, V>), dim3((unsigned)(BH * (V / 16))), dim3(4 * K), 0, s, ws + w.pbuf,
-                       ws + w.sbuf, BH, nt);
+                       ws + w.sbuf, (uint32_t*)(ws + w.redo), BH, nt);
   }
   hipLaunchKernelGGL((chunk_output_kernel<K, V>), dim3((unsigned)(BH * (V / kTileV) * p.out)), dim3(rec::kOThreads), 0,
                      s, (const bf16*)q, (const bf16*)k, (const bf16*)v, ws + w.records, (const float*)h0, ws + w.sbuf,
-                     (bf16*)o, (float*)ht, scale, T, H, NT, BH, p.out, p.len * p.per, p.per);
+                     (const uint32_t*)(ws + w.redo), (bf16*)o, (float*)ht, scale, T, H, NT, BH, p.out, p.len * p.per, p.per);
   return hipGetLastError();
 }
 

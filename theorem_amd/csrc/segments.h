@@ -335,12 +335,18 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
 // products: the state is carried in fp32 from one end of a sequence to the
 // other, as in one piece.  A serial chain of small steps: P and Q of the next
 // two steps are in flight during one, and the products run in two accumulators.
+// A segment's map can overflow where the states of the sequence do not (a
+// column that is zero stays zero whatever P is), and P S is then no number:
+// where any state of the 16 columns is not finite, redo[bh V / 16 + vt] says so
+// and the kernels that walk the segments take those columns in one piece.
 template <int K, int V>
 __global__ void __launch_bounds__(4 * K)
-chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int64_t BH, int64_t nseg) {
+chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, uint32_t* __restrict__ redo, int64_t BH,
+                     int64_t nseg) {
   constexpr int KB = K / 16, NVB = V / 16;
   constexpr int kAhead = 2;
   __shared__ __attribute__((aligned(16))) f32x4 xs[2][KB][64];  // one row tile's 4 rows per lane
+  __shared__ uint32_t over[KB];
   const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH, NVB);  // one XCD reads one (b, head)'s P
   const int wi = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -358,6 +364,7 @@ chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int
   };
   const int64_t last = nseg - 2;
   f32x4 S = *q_at(0);
+  uint32_t top = 0;  // the largest magnitude's bits: infinities and NaN lie above every finite one
 #pragma unroll
   for (int i = 0; i < kAhead; ++i) load(1 + i < last ? 1 + i : last, i);
   auto step = [&](int64_t s, int i) {
@@ -378,12 +385,34 @@ chunk_combine_kernel(const char* __restrict__ pbuf, char* __restrict__ sbuf, int
     }
     S = acc[0] + acc[1];
     *q_at(s) = S;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) top = max(top, __float_as_uint(S[r]) & 0x7fffffffu);
   };
   for (int64_t s = 1; s <= last; s += kAhead) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i)
       if (s + i <= last) step(s + i, i);  // uniform over the workgroup
   }
+  const bool any = __any(top >= 0x7f800000u);
+  if (lane == 0) over[wi] = any;
+  lds_barrier();
+  if (threadIdx.x == 0) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int i = 0; i < KB; ++i) o |= over[i];
+    redo[bt.bh * NVB + bt.vt] = o;
+  }
+}
+
+// Whether the columns [v0, v0 + cols) of sequence bh are walked in one piece
+// after all (segment 0 takes every chunk, the others none).
+template <int V>
+__device__ __forceinline__ bool redo_columns(const uint32_t* redo, int64_t bh, int v0, int cols) {
+  const uint32_t* p = redo + bh * (V / 16) + v0 / 16;
+  uint32_t o = 0;
+#pragma unroll
+  for (int i = 0; i < cols / 16; ++i) o |= p[i];
+  return o != 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -433,13 +462,15 @@ inline Plan plan_segments(int64_t BH, int64_t NT, const Costs& k) {
   return best;
 }
 
-// Workspace of a plan: P of segments 1 .. nt - 2 and the states, in bytes.
+// Workspace of a plan: P of segments 1 .. nt - 2, the states and the redo
+// flags, in bytes.
 inline int64_t p_bytes(const Plan& p, int64_t BH, int64_t NT, int64_t K) {
   return p.out > 1 ? (p.segs(NT) - 2) * BH * K * K * 4 : 0;
 }
 inline int64_t s_bytes(const Plan& p, int64_t BH, int64_t NT, int64_t K, int64_t V) {
   return p.out > 1 ? (p.segs(NT) - 1) * BH * K * V * 4 : 0;
 }
+inline int64_t redo_bytes(const Plan& p, int64_t BH, int64_t V) { return p.out > 1 ? BH * (V / 16) * 4 : 0; }
 
 }  // namespace seg
 }  // namespace
