@@ -3,8 +3,8 @@ rows that start anywhere in a 16-byte vector or a 128-byte line (the last
 row's end vector reaches past the tensor), and channels-last segments whose
 last one overlaps the one before.  Against float64 (torch, CPU): fp32 sums of
 W + 1 terms, W 2^-24 relative to the sum of the terms' magnitudes, and one
-rounding to the output type; with SiLU also the hardware exponential's and
-reciprocal's few ulp.  The elements around the output are left alone."""
+rounding to the output type; with SiLU also the hardware exponential's few
+ulp.  The elements around the output are left alone."""
 from __future__ import annotations
 
 import pytest

@@ -207,9 +207,9 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
         }
         acc = __builtin_fmaf(wk[k], xv, acc);
       }
-      if (act == THM_ACT_SILU) acc = silu<XT>(acc);
       res[v] = acc;
     }
+    if (act == THM_ACT_SILU) silu<XT, VEC>(res);
     const int64_t e0 = s0 + (int64_t)(j * kWave + lane) * VEC;
     if constexpr (RAGGED) {
       const int lo = first_in(e0), hi = end_in(e0);

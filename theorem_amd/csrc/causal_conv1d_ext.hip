@@ -131,9 +131,9 @@ causal_conv1d_cl_kernel(const XT* __restrict__ x, const void* __restrict__ weigh
 #pragma unroll
       for (int k = 0; k < W - 1; ++k) acc = __builtin_fmaf(wk[k][v], win[k][v], acc);
       acc = __builtin_fmaf(wk[W - 1][v], cur[v], acc);
-      if constexpr (SILU) acc = silu<XT>(acc);
       res[v] = acc;
     }
+    if constexpr (SILU) silu<XT, VEC>(res);
     if (!BLOCKS || j >= skip) cl_store<XT, VEC>(op, res);
     op += dim;
 #pragma unroll
@@ -248,7 +248,7 @@ causal_conv1d_update_kernel(const XT* __restrict__ x, XT* __restrict__ state,
     float acc = b0;
     const int64_t base = state_len - (width - 1) + t;
     for (int k = 0; k < width; ++k) acc = __builtin_fmaf(wk[k], at(base + k), acc);
-    if (act == THM_ACT_SILU) acc = silu<XT>(acc);
+    if (act == THM_ACT_SILU) silu<XT, 1>(&acc);
     orow[t] = from_f32<XT>(acc);
   }
   // New state: the last L_s window samples, written front to back (the
@@ -277,7 +277,7 @@ causal_conv1d_step_kernel(const XT* __restrict__ x, XT* __restrict__ state, cons
   float acc = bias ? to_f32(reinterpret_cast<const WT*>(bias)[d]) : 0.f;
 #pragma unroll
   for (int k = 0; k < W; ++k) acc = __builtin_fmaf(to_f32(wk[k]), to_f32(win[OFF + k]), acc);
-  if (act == THM_ACT_SILU) acc = silu<XT>(acc);
+  if (act == THM_ACT_SILU) silu<XT, 1>(&acc);
   out[row] = from_f32<XT>(acc);
   if constexpr (L > 0) __builtin_memcpy(st, win + 1, L * sizeof(XT));
 }

@@ -35,18 +35,32 @@ constexpr float kLog2e = 1.4426950408889634f;
 // exp(x) through the hardware base-2 exponential (v_exp_f32).
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
-// x sigmoid(x) = x (x >= 0 ? 1 : e) / (1 + e) with e = e^{-|x|} <= 1, rounded
-// afterwards to XT.  For bf16 the quotient is a multiplication by the hardware
-// reciprocal (1 + e in [1, 2], where it is good to an ulp of fp32): an IEEE
-// division is ten instructions per element, and the convolutions with SiLU
-// spent more time on it than on memory.
-template <typename XT>
-__device__ __forceinline__ float silu(float x) {
+// v[i] <- v[i] sigmoid(v[i]), rounded afterwards to XT.  An IEEE division is
+// ten instructions, and the bf16 convolutions with SiLU spent more time on it
+// than on memory: there the quotient is the hardware reciprocal's (1 ulp) and
+// one residual step, which gives the correctly rounded quotient (the residual
+// is exact and the reciprocal's error reaches its second order only) while
+// neither 1 / d nor the quotient leaves the normal range: |v| < 80.  A vector
+// with a larger element takes the division.
+template <typename XT, int N>
+__device__ __forceinline__ void silu(float* v) {
+  float d[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) d[i] = 1.f + fast_exp(-v[i]);
+  float top = sizeof(XT) == 2 ? 0.f : 80.f;
   if constexpr (sizeof(XT) == 2) {
-    const float e = fast_exp(-fabsf(x));
-    return x * (x >= 0.f ? 1.f : e) * __builtin_amdgcn_rcpf(1.f + e);
+#pragma unroll
+    for (int i = 0; i < N; ++i) top = fmaxf(top, fabsf(v[i]));
+  }
+  if (top >= 80.f) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] /= d[i];
   } else {
-    return x / (1.f + fast_exp(-x));
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float r = __builtin_amdgcn_rcpf(d[i]), q = v[i] * r;
+      v[i] = __builtin_fmaf(__builtin_fmaf(-d[i], q, v[i]), r, q);
+    }
   }
 }
 
