@@ -40,26 +40,32 @@ __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp
 // than on memory: there the quotient is the hardware reciprocal's (1 ulp) and
 // one residual step, which gives the correctly rounded quotient (the residual
 // is exact and the reciprocal's error reaches its second order only) while
-// neither 1 / d nor the quotient leaves the normal range: |v| < 80.  A vector
-// with a larger element takes the division.
+// neither 1 / d nor the quotient leaves the normal range: |v| < 80.  Four
+// elements (four: the denominators of a whole vector cost a wave of occupancy)
+// with a larger one among them take the division.
 template <typename XT, int N>
 __device__ __forceinline__ void silu(float* v) {
-  float d[N];
+  constexpr int M = N < 4 ? N : 4;
+  static_assert(N % M == 0, "whole groups");
 #pragma unroll
-  for (int i = 0; i < N; ++i) d[i] = 1.f + fast_exp(-v[i]);
-  float top = sizeof(XT) == 2 ? 0.f : 80.f;
-  if constexpr (sizeof(XT) == 2) {
+  for (int j = 0; j < N; j += M) {
+    float d[M];
 #pragma unroll
-    for (int i = 0; i < N; ++i) top = fmaxf(top, fabsf(v[i]));
-  }
-  if (top >= 80.f) {
+    for (int i = 0; i < M; ++i) d[i] = 1.f + fast_exp(-v[j + i]);
+    float top = sizeof(XT) == 2 ? 0.f : 80.f;
+    if constexpr (sizeof(XT) == 2) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] /= d[i];
-  } else {
+      for (int i = 0; i < M; ++i) top = fmaxf(top, fabsf(v[j + i]));
+    }
+    if (top >= 80.f) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const float r = __builtin_amdgcn_rcpf(d[i]), q = v[i] * r;
-      v[i] = __builtin_fmaf(__builtin_fmaf(-d[i], q, v[i]), r, q);
+      for (int i = 0; i < M; ++i) v[j + i] /= d[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        const float r = __builtin_amdgcn_rcpf(d[i]), q = v[j + i] * r;
+        v[j + i] = __builtin_fmaf(__builtin_fmaf(-d[i], q, v[j + i]), r, q);
+      }
     }
   }
 }
