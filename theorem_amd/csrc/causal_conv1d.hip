@@ -22,7 +22,7 @@
 //     neighbours, which are read as zero and not written.  [4, 4096, 4003] bf16
 //     with SiLU: element by element (2-byte lanes) 157 us, in whole vectors
 //     from the row's first 16 bytes 63, from its first 128-byte line (no split
-//     line between a segment's stores) 59, with silu()'s reciprocal 49;
+//     line between a segment's stores) 59, with silu()'s quotient 51;
 //     [8, 4096, 8191] 173, as 8192.
 //   * Weights and bias are wave-uniform; accumulation is fp32 FMA.
 //   * Stores are non-temporal: the output is not re-read by this kernel.
@@ -122,7 +122,7 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
       const int64_t e0 = s0 + (int64_t)(j * kWave + lane) * VEC;
       unpack16(raw[j], cur[j], XT{});
       if constexpr (RAGGED) {
-        if (ends) {
+        if (ends && s0 + j * kWave * VEC < seqlen) {
           const int lo = first_in(e0), hi = end_in(e0);
           if (past && lo == 0 && hi > 0 && hi < VEC) {
 #pragma unroll
@@ -190,6 +190,7 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
 
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (RAGGED && s0 + j * kWave * VEC >= seqlen) return;  // nothing of the row left (wave-uniform)
     float res[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
@@ -226,18 +227,62 @@ causal_conv1d_kernel(const XT* __restrict__ x, const void* __restrict__ weight,
   }
 }
 
-template <typename XT, typename WT, int VEC, int W, bool RAGGED>
-hipError_t launch_conv(const void* x, const void* weight, const void* bias, void* out,
+template <typename XT, typename WT, int VEC, int W, int NV, bool RAGGED>
+hipError_t launch_conv_nv(const void* x, const void* weight, const void* bias, void* out,
                        int64_t n_rows, int64_t dim, int64_t seqlen, int act, hipStream_t stream) {
-  constexpr int SEG = kConvNV * kWave * VEC;
+  constexpr int SEG = NV * kWave * VEC;
   // With the largest offset (a segment past a row's end does nothing).
   const int64_t segs_per_row = (seqlen + (RAGGED ? 128 / (int)sizeof(XT) - 1 : 0) + SEG - 1) / SEG;
   const int64_t n_seg = n_rows * segs_per_row;
   const int64_t blocks = (n_seg + kConvWaves - 1) / kConvWaves;
-  hipLaunchKernelGGL((causal_conv1d_kernel<XT, WT, VEC, W, kConvNV, RAGGED>), dim3((unsigned)blocks),
+  hipLaunchKernelGGL((causal_conv1d_kernel<XT, WT, VEC, W, NV, RAGGED>), dim3((unsigned)blocks),
                      dim3(kConvWaves * kWave), 0, stream, (const XT*)x, weight, bias, (XT*)out,
                      n_rows, dim, seqlen, segs_per_row, act);
   return hipGetLastError();
+}
+
+// Ragged bf16 rows take waves of two vector groups where one such wave holds
+// the row, or where four groups a wave would not fill the GPU's wave slots
+// once.  us, W = 4, SiLU, four groups -> two: [4, 4096, 700] 16.1 -> 14.9,
+// [4, 4096, 1003] 18.9 -> 21.3 (two waves a row, four: still one or two), [1,
+// 1024, 1793] 5.5 -> 4.9, [1, 1024, 3003] 6.0 -> 5.6.
+template <typename XT, typename WT, int VEC, int W, bool RAGGED>
+hipError_t launch_conv(const void* x, const void* weight, const void* bias, void* out, int64_t n_rows, int64_t dim,
+                       int64_t seqlen, int act, hipStream_t s) {
+  if constexpr (RAGGED && sizeof(XT) == 2) {
+    constexpr int kTwo = 2 * kWave * VEC;
+    const int64_t waves = n_rows * ((seqlen + kConvNV * kWave * VEC - 1) / (kConvNV * kWave * VEC));
+    if (seqlen + 128 / (int)sizeof(XT) - 1 <= kTwo || waves < (int64_t)16 * device_cu_count())
+      return launch_conv_nv<XT, WT, VEC, W, 2, RAGGED>(x, weight, bias, out, n_rows, dim, seqlen, act, s);
+  }
+  return launch_conv_nv<XT, WT, VEC, W, kConvNV, RAGGED>(x, weight, bias, out, n_rows, dim, seqlen, act, s);
+}
+
+// Whether rows that are no multiple of a vector take whole vectors (RAGGED)
+// rather than scalar lanes (four waves' worth of 64 elements a wave).  Both
+// compute whole waves: a ragged wave pays for its masked ends and for a last
+// group of up to 512 elements, a scalar one for narrow loads.  us, scalar ->
+// ragged:
+//   bf16, W = 4, SiLU, [4, 4096, S]: S = 100 6.6 -> 9.0, 255 8.2 -> 10.0, 500
+//     15.2 -> 13.8, 513 20.0 -> 14.6, 1003 31 -> 18.9, 4003 120 -> 48; [2,
+//     4096, 509] 7.9 -> 8.2, [1, 4352, 509] 5.7 -> 6.4;
+//   fp32, whose scalar lanes read 256 bytes a wave, as long as x and out stay
+//     in the 256 MiB memory-side cache: W = 4, [4, 4096, 1003] 21.6 -> 24.5,
+//     [4, 4096, 2001] (2 x 131 MB) 43.9 -> 44.6, [4, 4096, 2501] 61.5 -> 54.4,
+//     [8, 6144, 639] (2 x 126 MB) 41.3 -> 43.9, [8, 6144, 801] 64.6 -> 54.3;
+//     wide filters, W = 8, [4, 4096, S]: S = 509 15.3 -> 17.8, 513 21.3 ->
+//     18.0, 1501 40.3 -> 35.3, but 1021 (whose second wave is nearly empty)
+//     28.0 -> 29.7; W = 5: S = 801 21.8 -> 20.2, 1793 42.6 -> 39.9;
+//     few long rows, too few scalar waves in flight for their bytes: W = 4, [1,
+//     1024, S]: S = 2001 (8 MB) 5.1 -> 5.8, 3003 6.3 -> 6.2, 5001 8.7 -> 7.6,
+//     without SiLU 7001 (29 MB) 10.2 -> 11.0; [1, 2048, S]: S = 2001 7.6 ->
+//     7.2, 3003 (25 MB) 10.1 -> 9.0, 4501 13.5 -> 14.6; W = 2, 6001 8.4 -> 9.3.
+inline bool ragged_vectors(int64_t n_rows, int64_t seqlen, int width, bool f32) {
+  if (seqlen <= 512) return false;
+  if (!f32) return true;
+  const int64_t bytes = n_rows * seqlen * 4;
+  return 2 * bytes > (INT64_C(1) << 28) || (width >= 5 && (seqlen + 31) % 1024 > 256) ||
+         (width >= 4 && seqlen >= 2000 && bytes >= 12000000 && bytes <= 25000000);
 }
 
 template <typename XT, int VEC, bool RAGGED, typename WT>
@@ -298,11 +343,10 @@ extern "C" int thm_causal_conv1d_fwd(const void* x, const void* weight, const vo
     return THM_ERR_BAD_SHAPE;
   const int vec = (int)(16 / xe);
   // 16-byte vectors need x and out 16-byte aligned; rows that are no multiple
-  // of a vector take the ragged form of the same kernel, which needs rows longer
-  // than a vector (from 64 elements on; below that a row is one wave of scalar
-  // lanes anyway).
+  // of a vector take the ragged form of the same kernel where it pays.
   const bool whole = seqlen % vec == 0;
-  const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && (whole || seqlen >= 64);
+  const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) &&
+                      (whole || ragged_vectors(n_rows, seqlen, width, x_dtype == THM_DTYPE_F32));
   const int wb = (w_dtype == THM_DTYPE_BF16);
   hipStream_t s = (hipStream_t)stream;
   auto run = [&](auto xt, auto vec_c) {
