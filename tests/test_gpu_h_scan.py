@@ -51,3 +51,11 @@ def test_scan_vs_oracle(dev, dt, B, NT, H, K, V, plain):
     for name, x, e in (("h", h, eh), ("final state", ht, eht)):
         err = np.linalg.norm(np_(x) - e) / np.linalg.norm(e)
         assert err <= bound, f"{name}: relative error {err:.3e}, bound {bound:.3e}"
+
+
+# Heads rounded up to whole rounds of the XCDs: one workgroup per CU (45 heads of
+# 4 tiles, 15 of 16), two (45 of 8, 17 of 16).
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,NT,H,K,V", [(5, 17, 9, 64, 64), (1, 6, 15, 128, 128), (5, 32, 9, 128, 64), (1, 33, 17, 128, 128)])
+def test_heads_not_a_multiple_of_the_xcds(dev, dt, B, NT, H, K, V):
+    test_scan_vs_oracle(dev, dt, B, NT, H, K, V, False)

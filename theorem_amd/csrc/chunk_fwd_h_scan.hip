@@ -46,7 +46,7 @@ template <typename IT, int TB>
 __global__ void __launch_bounds__(kScanThreads)
 chunk_fwd_h_scan_kernel(const IT* __restrict__ k, const IT* __restrict__ v, const float* __restrict__ g,
                         const float* __restrict__ h0, float* __restrict__ h, float* __restrict__ ht, int64_t T,
-                        int64_t H, int64_t NT, int64_t BH, int K, int V) {
+                        int64_t H, int64_t NT, int64_t BH, int64_t heads, int K, int V) {
   constexpr int CPL = TB / 16;  // columns per lane
   constexpr int E = TB * TB;
   constexpr bool kF32 = std::is_same<IT, float>::value;
@@ -56,9 +56,12 @@ chunk_fwd_h_scan_kernel(const IT* __restrict__ k, const IT* __restrict__ v, cons
   __shared__ __attribute__((aligned(16))) float fac[kBatch][kBT];
 
   // The tiles of one (b, head) share an XCD, whose L2 then serves the columns
-  // of k and v that several tiles read.
+  // of k and v that several tiles read.  `heads`: BH rounded up to whole rounds
+  // of the XCDs (64 x 64, bf16, 48 chunks of 45 heads, us: walking 25.6, tiles
+  // of a head spread over the XCDs 28.1; 64 chunks 33.2, 36.7, together 20.8).
   const int nv = V / TB;
-  const hl::BhTile bt = hl::xcd_tile(blockIdx.x, BH, (K / TB) * nv);
+  const hl::BhTile bt = hl::xcd_tile(blockIdx.x, heads, (K / TB) * nv);
+  if (bt.bh >= BH) return;  // (uniform over the workgroup)
   const int64_t b = bt.bh / H, hh = bt.bh - b * H;
   const int kt = (int)bt.vt / nv, vt = (int)bt.vt - kt * nv;
   const int tid = threadIdx.x;
@@ -184,9 +187,12 @@ chunk_fwd_h_scan_kernel(const IT* __restrict__ k, const IT* __restrict__ v, cons
 template <typename IT, int TB>
 hipError_t launch_scan(const void* k, const void* v, const void* g, const void* h0, void* h, void* ht, int64_t B,
                        int64_t T, int64_t H, int64_t K, int64_t V, hipStream_t s) {
-  hipLaunchKernelGGL((chunk_fwd_h_scan_kernel<IT, TB>), dim3((unsigned)(B * H * (K / TB) * (V / TB))),
-                     dim3(kScanThreads), 0, s, (const IT*)k, (const IT*)v, (const float*)g, (const float*)h0, (float*)h,
-                     (float*)ht, T, H, T / kBT, B * H, (int)K, (int)V);
+  const int64_t BH = B * H, tiles = (K / TB) * (V / TB), whole = (BH + 7) / 8 * 8;
+  const int64_t slots = device_cu_count() * (int64_t)(BH * tiles <= device_cu_count() ? 1 : 2);
+  const int64_t heads = BH > 8 && whole * tiles <= slots ? whole : BH;  // (fewer heads would leave XCDs idle)
+  hipLaunchKernelGGL((chunk_fwd_h_scan_kernel<IT, TB>), dim3((unsigned)(heads * tiles)), dim3(kScanThreads), 0, s,
+                     (const IT*)k, (const IT*)v, (const float*)g, (const float*)h0, (float*)h, (float*)ht, T, H, T / kBT,
+                     BH, heads, (int)K, (int)V);
   return hipGetLastError();
 }
 
@@ -200,16 +206,21 @@ hipError_t launch_scan(const void* k, const void* v, const void* g, const void* 
 //   16 heads of 64 x 64, 128 chunks    58 -> 33 -> 40        (100 -> 35 -> 70)
 //   8 heads of 128 x 128, 128 chunks   84 -> 54 -> 35        (181 -> 66 -> 70)
 //   16 heads of 128 x 128, 128 chunks  83 -> 109 -> 42       (185 -> 128 -> 75)
-// Two 32 x 32 workgroups per CU gain on long sequences only, three nowhere:
-//   32 heads of 128 x 128, 32 chunks   25.2 -> 54 -> 23.5    (51 -> 62 -> 39)
-//   48 heads of 128 x 128, 32 chunks   26.6 -> 83 -> 33.7    (52 -> 91 -> 55)
+// Two 32 x 32 workgroups per CU gain on long sequences at K = 128 (a walking
+// workgroup takes all K rows of 64 columns, so its chunk costs more there),
+// three nowhere; walking -> 32, 64 chunks:
+//   128 x 128, 20 heads   44.6 -> 37.1    (100 -> 70)     32 heads  43.5 -> 41.7  (97 -> 74)
+//   128 x 64, 45 heads    43.8 -> 37.8    (93 -> 71)      64 heads  44.3 -> 44.9  (127 -> 98)
+//   64 x 128, 45 heads, tiles of a head apart, 43.6 -> 70.9; 64 heads 37.7 -> 43.9
+// (where h takes most of the memory-side cache, 22 and 25 heads of 128 x 128 at
+// 128 chunks, bf16, it loses: 85 -> 105 and 113 -> 136; 24 heads 149 -> 129).
 // Four chunks or fewer are walked in the time of one batch (2 chunks of 62
 // heads of 64 x 64: 3.4 -> 9.8 -> 4.1).
 __attribute__((visibility("hidden"))) int h_scan_tile(int64_t BH, int64_t NT, int64_t K, int64_t V) {
-  const int64_t cu = device_cu_count(), n32 = BH * (K / 32) * (V / 32);
   if (NT <= 4) return 0;
+  const int64_t cu = device_cu_count(), n32 = BH * (K / 32) * (V / 32);
   if (4 * n32 <= cu) return 16;
-  return n32 <= cu || (n32 <= 2 * cu && NT >= 32) ? 32 : 0;
+  return n32 <= cu || (n32 <= 2 * cu && NT >= 32 && K == 128) ? 32 : 0;
 }
 
 __attribute__((visibility("hidden"))) hipError_t chunk_fwd_h_scan(bool f32, int tile, const void* k, const void* v,
