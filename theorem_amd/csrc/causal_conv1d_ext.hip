@@ -40,11 +40,6 @@ __device__ __forceinline__ float conv_param(const void* p, int64_t i, int is_bf1
   return is_bf16 ? (float)reinterpret_cast<const bf16*>(p)[i] : reinterpret_cast<const float*>(p)[i];
 }
 
-template <typename WT>
-__device__ __forceinline__ float conv_param_t(const void* p, int64_t i) {
-  return to_f32(reinterpret_cast<const WT*>(p)[i]);
-}
-
 template <typename XT, int VEC>
 __device__ __forceinline__ void cl_load(const XT* p, float* v) {
   if constexpr (VEC * sizeof(XT) == 16) {
@@ -207,6 +202,36 @@ hipError_t launch_cl_w(int width, int seg, const void* x, const void* weight, co
   return hipGetLastError();
 }
 
+// Steps per lane: waves take a start of about four steps (the window, the
+// taps) and their own steps, on a SIMD one after another in whole waves, and a
+// SIMD needs two to cover their loads; the last segment repeats steps of the
+// one before it.  So a length that leaves the SIMDs two waves each beats a
+// shorter one with four, and both beat two and a half.  us at segments of
+// 8 / 16 / 32 / 64 (two waves per SIMD at the marked one):
+//   bf16 [8, 8192, 4096] 209 / 214 / 196 / 190, [2, 5001, 4352] 42 / 39 / 37 /
+//     44, [1, 1000, 4352] 8.1 / 9.4 / 14 / 24, [4, 2048, 4096] 33 / 31 / 27 /
+//     27*, [4, 5001, 2048] 39 / 33 / 36 / 44, [8, 2500, 6144] 102 / 94 / 100 /
+//     104;
+//   fp32 [4, 2048, 4096] - / 61 / 62 / 51*, [1, 8192, 2048] - / 29 / 27* / 29,
+//     [1, 5001, 4352] - / 39 / 37 / 40, [4, 5001, 2048] - / 69 / 70 / 77, [8,
+//     257, 6144] - / 25 / 25 / 27, [8, 1000, 6144] - / 82 / 81 / 87 (taken: 64).
+inline int cl_segment(int64_t batch, int64_t seqlen, int64_t groups, int depth) {
+  const int64_t simds = 4 * (int64_t)std::max(device_cu_count(), 1);
+  int best = depth;
+  int64_t least = INT64_MAX;
+  for (int seg = kClSeg; seg >= depth; seg /= 2) {
+    const int64_t items = batch * ((seqlen + seg - 1) / seg) * groups;
+    if (seg > seqlen || (seg < kClSeg && !launch_fits((items + kClThreads - 1) / kClThreads, kClThreads))) continue;
+    const int64_t waves = (items + kWave - 1) / kWave;
+    const int64_t cost = std::max<int64_t>((waves + simds - 1) / simds, 2) * (seg + 4);
+    if (cost < least) {
+      least = cost;
+      best = seg;
+    }
+  }
+  return best;
+}
+
 template <typename XT, typename WT>
 hipError_t launch_cl(bool vec_ok, int width, const void* x, const void* weight, const void* bias, void* out,
                      int64_t batch, int64_t seqlen, int64_t dim, int act, hipStream_t s) {
@@ -214,15 +239,7 @@ hipError_t launch_cl(bool vec_ok, int width, const void* x, const void* weight, 
   if (!vec_ok) return launch_cl_w<XT, WT, 1, false>(width, kClSeg, x, weight, bias, out, batch, seqlen, dim, act, s);
   constexpr int kDepth = cl_depth<XT>();
   if (seqlen < kDepth) return launch_cl_w<XT, WT, VEC, false>(width, kClSeg, x, weight, bias, out, batch, seqlen, dim, act, s);
-  // Longest segments that leave every SIMD a few waves (each segment re-reads
-  // W - 1 steps; a lane's steps run one after another): 2 for bf16, 4 for fp32,
-  // whose lanes hold half the channels.  us at segments of 8 / 16 / 32 / 64:
-  // bf16 [8, 8192, 4096] 209 / 214 / 196 / 190, [2, 5001, 4352] 42 / 39 / 37 /
-  // 44, [1, 1000, 4352] 8.7 / 8.4 / 11.8 / 19.6; fp32 [4, 2500, 5120] - / 88 /
-  // 84 / 90.
-  const int64_t waves = (int64_t)std::max(device_cu_count(), 1) * 4 * (sizeof(XT) == 2 ? 2 : 4);
-  int seg = kClSeg;
-  while (seg > kDepth && (seg > seqlen || batch * ((seqlen + seg - 1) / seg) * (dim / VEC) < waves * kWave)) seg /= 2;
+  const int seg = cl_segment(batch, seqlen, dim / VEC, kDepth);
   return launch_cl_w<XT, WT, VEC, true>(width, seg, x, weight, bias, out, batch, seqlen, dim, act, s);
 }
 
@@ -350,8 +367,8 @@ extern "C" int thm_causal_conv1d_fwd_channels_last(const void* x, const void* we
   const int vec = (int)(16 / xe);
   const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && (dim % vec == 0);
   const int64_t groups = vec_ok ? dim / vec : dim;
-  // (Below 2^32 lanes, so the kernel's 32-bit indices hold; segments shorter
-  // than kClSeg are taken for small grids only.)
+  // (Below 2^32 lanes, so the kernel's 32-bit indices hold; cl_segment keeps
+  // shorter segments to it too.)
   if (!launch_fits(batch * ((seqlen + kClSeg - 1) / kClSeg) * ((groups + kClThreads - 1) / kClThreads), kClThreads))
     return THM_ERR_BAD_SHAPE;
   const int wb = (w_dtype == THM_DTYPE_BF16);
