@@ -422,28 +422,12 @@ hipError_t dispatch_kv(int64_t K, int64_t V, const void* k, const void* w, const
   return launch_kv<DELTA, 128, 128>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
 }
 
-// Segments of a call (segments.h plan_segments); one piece for the reference
-// form and on grids that fill the GPU without them.  Periods in us per chunk,
-// from MI355X timings (in one piece -> best of nine plans -> this rule):
-//   bf16, small-grid kernel against transitions and the DMA kernel: B = 1,
-//     H = 16, K = V = 128, 128 chunks 141 -> 104 -> 101 us (with other inputs
-//     every pass 200 -> 111), 32 chunks 38 -> 42 -> 38; H = 4, 64 chunks 71 ->
-//     50 -> 50; K = V = 64, 64 chunks 46 -> 32 -> 32;
-//   fp32, register kernel (at K = 64 the small-grid kernel in one piece): 16
-//     heads of K = V = 128, 32 chunks 137 -> 81 -> 80, 4 heads, 64 chunks 268
-//     -> 74 -> 74; 16 heads of K = V = 64, 64 chunks 97 -> 50 -> 50.  With 128
-//     columns a workgroup (h_seg_cols; kernel trace, sums of the three
-//     launches): 16 heads, 32 chunks 71, 4 heads, 64 chunks 77, 8 heads, 128
-//     chunks 126 (530 in one piece), 32 heads, 16 chunks 60 (72).
+// Segments of a call (seg_plan.h); one piece for the reference form and on
+// grids that fill the GPU without them.
 inline seg::Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, bool delta, bool f32) {
-  const int64_t NT = T / kBT, BH = B * H, nvt = V / kHBV;
-  if (!delta || BH * nvt >= kHDmaMinGrid) return {1, 1, std::max<int64_t>(NT, 1)};
-  if (f32) {
-    if (h_seg_cols(K, V) == 128) return seg::plan_segments(BH, NT, {nvt, (K + V) / 128, V / 128, 4.7, 5.3, 1.65, 6.4});
-    const double period = K == 128 ? 4.7 : 2.5;
-    return seg::plan_segments(BH, NT, {nvt, (K + V) / kHBV, nvt, K == 128 ? period : 1.7, period, 1.2, period});
-  }
-  return seg::plan_segments(BH, NT, {V / 32, 1, nvt, 1.2, 2.2, K == 128 ? 1.65 : 0.9, 2.6});
+  const int64_t NT = T / kBT, BH = B * H;
+  if (!delta || BH * (V / kHBV) >= kHDmaMinGrid) return {1, 1, std::max<int64_t>(NT, 1)};
+  return seg::plan_h(BH, NT, K, V, f32, device_cu_count());
 }
 
 inline int64_t workspace_bytes_of(const seg::Plan& p, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {

@@ -47,14 +47,6 @@ namespace {
 
 constexpr int kBT = 64;
 constexpr int kHBV = 64;  // V-tile width
-// V-tile width of the segment launches (fp32 inputs).  Staging a chunk of k and
-// w (an fp32 -> bf16 hi + lo split of each) and its barriers take a large part
-// of a period and the LDS stage leaves one workgroup per CU: where P and V both
-// make whole tiles of 128, twice the waves share them (period 4.7 us for 64
-// columns -> 5.3 for 128).  B = 2, T = 2048, H = 8: transitions 42.4 -> 27.7 us,
-// outputs 37.2 -> 30.5, combine 8.4 -> 13.3 (8 segments instead of 5).
-constexpr int h_seg_cols(int64_t K, int64_t V) { return K == 128 && V == 128 ? 128 : kHBV; }
-
 // BV columns per workgroup, a wavefront for every 16.
 template <typename IT, int K, int V, bool DELTA, int BV>
 struct HCfg {
@@ -422,7 +414,7 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
                      (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, redo, T, H, NT, BH, NSEG, LEN, p.per)
   if constexpr (DELTA) {
     if (p.out > 1) {
-      constexpr int BV = h_seg_cols(K, V);
+      constexpr int BV = seg::h_seg_cols(K, V);
       const int64_t nt = p.segs(NT), grid = BH * (nt - 1) * ((K + V) / BV);
       if (g) THM_H_LAUNCH(true, false, true, BV, grid, nt - 1, p.len);
       else THM_H_LAUNCH(false, false, true, BV, grid, nt - 1, p.len);

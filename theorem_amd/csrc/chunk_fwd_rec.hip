@@ -312,15 +312,8 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
   }
 }
 
-// Measured at K = V = 128: period 2.0-2.1 us (outputs), 2.3-2.4 (transitions),
-// 1.65 per combine step; whole forwards, unsegmented -> best of ten plans ->
-// this rule's choice: 16 heads: 16 chunks 42 -> 36 -> 36 us, 32 chunks 77 ->
-// 48 -> 48, 128 chunks 276 -> 107 -> 107; 32 heads, 32 chunks 84 -> 66; 4
-// heads, 64 chunks 140 -> 55.  128 workgroups or more without segments do not
-// gain (64 heads, 32 chunks: 86 unsegmented, 96 at best).
 inline Plan plan_of(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
-  const int64_t nvt = V / kTileV;
-  return plan_segments(B * H, T / kBT, {nvt, 1, nvt, 2.02, 2.4, K == 128 ? 1.65 : 0.9, 2.1});
+  return plan_fwd(B * H, T / kBT, K, V, device_cu_count());
 }
 
 struct Workspace {

@@ -9,11 +9,10 @@
 // and the combine kernel runs S <- P S + Q over the segments.
 #pragma once
 
-#include <algorithm>
-
 #include "h_layout.h"
 #include "mfma.h"
 #include "rec_cfg.h"
+#include "seg_plan.h"
 #include "vmem.h"
 
 namespace thm {
@@ -416,61 +415,6 @@ __device__ __forceinline__ bool redo_columns(const uint32_t* redo, int64_t bh, i
 }
 
 // ---------------------------------------------------------------------------
-// Segments of a call: `out` of the output kernel, each of `per` transition
-// segments of `len` chunks (the last may be shorter, none is empty).
-struct Plan {
-  int64_t out, per, len;
-  int64_t segs(int64_t NT) const { return (NT + len - 1) / len; }
-};
-
-// What a plan costs, in us on MI355X (only the ratios matter): workgroups per
-// (b, head) and segment and the serial period of a chunk in the transition and
-// the output kernel, the combine kernel's step, and the period in one piece.
-struct Costs {
-  int64_t one_tiles, t_tiles, o_tiles;
-  double one_period, t_period, c_step, o_period;
-};
-
-// The plan of least estimated time: a launch of workgroups that each walk n
-// chunks takes a start that grows with the share of the CUs in use, and n
-// periods; one CU holds one workgroup of these kernels (LDS), so more
-// workgroups than CUs run in rounds.  Two segments never gain (the transitions
-// of the first alone take about as long as its outputs); a plan has to save
-// 5 %.
-inline Plan plan_segments(int64_t BH, int64_t NT, const Costs& k) {
-  const int64_t cu = std::max<int64_t>(device_cu_count(), 1);
-  auto launch = [&](int64_t wgs, double start, double period, int64_t chunks) {
-    const double share = std::min(1.0, (double)wgs / cu);
-    return (double)((wgs + cu - 1) / cu) * (start + 5.0 * share + period * chunks);
-  };
-  Plan best = {1, 1, std::max<int64_t>(NT, 1)};
-  double t_best = 0.95 * launch(BH * k.one_tiles, 3.0, k.one_period, NT);
-  for (int64_t out = 3; out <= 32 && out <= NT; ++out) {
-    for (int64_t per = 1; per <= 4 && out * per <= NT; ++per) {
-      const int64_t len = (NT + out * per - 1) / (out * per);
-      const int64_t nt = (NT + len - 1) / len;  // transition segments
-      const int64_t no = (nt + per - 1) / per;  // output segments
-      if (no < 3) continue;
-      const double t = launch(BH * (nt - 1) * k.t_tiles, 4.0, k.t_period, len) + 3.0 + k.c_step * (nt - 2) +
-                       launch(BH * k.o_tiles * no, 3.0, k.o_period, len * per);
-      if (t < t_best) {
-        t_best = t;
-        best = {no, per, len};
-      }
-    }
-  }
-  return best;
-}
-
-// Workspace of a plan: P of segments 1 .. nt - 2, the states and the redo
-// flags, in bytes.
-inline int64_t p_bytes(const Plan& p, int64_t BH, int64_t NT, int64_t K) {
-  return p.out > 1 ? (p.segs(NT) - 2) * BH * K * K * 4 : 0;
-}
-inline int64_t s_bytes(const Plan& p, int64_t BH, int64_t NT, int64_t K, int64_t V) {
-  return p.out > 1 ? (p.segs(NT) - 1) * BH * K * V * 4 : 0;
-}
-inline int64_t redo_bytes(const Plan& p, int64_t BH, int64_t V) { return p.out > 1 ? BH * (V / 16) * 4 : 0; }
 
 }  // namespace seg
 }  // namespace
