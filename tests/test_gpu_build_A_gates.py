@@ -32,6 +32,24 @@ def test_A_and_gates(dev, B, T, H, K, adt, logsig):
     assert torch.equal(o, o1) and torch.equal(ht, ht1)
 
 
+@pytest.mark.parametrize("logsig", [False, True])
+def test_intermediates_only_add_outputs(dev, logsig):
+    # Asking for the intermediates changes no bit of o and the final state, and
+    # the g and A returned are those they were formed from.
+    B, T, H, K = 2, 192, 3, 128
+    gen = torch.Generator().manual_seed(1)
+    k = configs.l2norm(torch.randn(B, T, H, K, generator=gen)).to(dev)
+    v = torch.randn(B, T, H, 64, generator=gen).to(dev)
+    beta = torch.sigmoid(torch.randn(B, T, H, generator=gen)).to(dev)
+    a = (torch.randn(B, T, H, generator=gen) if logsig else -0.1 * torch.rand(B, T, H, generator=gen)).to(dev)
+    o, ht = chain.chunk_gated_delta_rule_fwd(k, k, v, beta, None, 0.1, None, True, a=a, a_logsigmoid=logsig)
+    o1, ht1, mid = chain.chunk_gated_delta_rule_fwd(k, k, v, beta, None, 0.1, None, True, a=a, a_logsigmoid=logsig,
+                                                    return_intermediates=True)
+    assert torch.equal(o, o1) and torch.equal(ht, ht1)
+    A, g = chain._build_A_gates(k, beta, a, logsig)
+    assert torch.equal(mid["A"], A) and torch.equal(mid["g"], g)
+
+
 def test_refused():
     f = _capi.load_library().thm_wy_build_A_gates
     ok = dict(k=16, beta=16, a=16, A=16, g=16, B=1, T=64, H=1, K=64, bt=64, kd=0, ad=0, kind=0, sign=1)

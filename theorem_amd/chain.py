@@ -220,7 +220,7 @@ def chunk_gated_delta_rule_fwd(q, k, v, beta, g, scale: float, initial_state=Non
             return _fwd_records(q, k, v, beta, g, _capi.THM_GATE_CUMULATIVE, scale, initial_state, output_final_state)
         kind = _capi.THM_GATE_LOGSIGMOID if a_logsigmoid else _capi.THM_GATE_IDENTITY
         return _fwd_records(q, k, v, beta, a, kind, scale, initial_state, output_final_state)
-    if a is not None and A is None and not fused and not return_intermediates and _gates_with_A(k, beta, a):
+    if a is not None and A is None and not fused and _gates_with_A(k, beta, a):
         A, g = _build_A_gates(k, beta, a, a_logsigmoid)
     elif a is not None:
         g = chunk_local_cumsum(a, logsigmoid=a_logsigmoid)
