@@ -23,7 +23,7 @@ def _both(fn, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("W", [1, 2, 4, 8])
+@pytest.mark.parametrize("W", [1, 2, 3, 4, 8])
 @pytest.mark.parametrize("extra", [0, 1, 3])
 @pytest.mark.parametrize("act", [None, "silu"])
 def test_update(dev, dtype, W, extra, act, monkeypatch):

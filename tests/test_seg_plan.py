@@ -1,5 +1,6 @@
 """The segment plans (theorem_amd/csrc/seg_plan.h) on the host: what every plan
-promises the kernels, and shapes that measured slower or faster in segments."""
+promises the kernels, the plans behind the GPU tests, and shapes that measured
+slower or faster in segments."""
 from __future__ import annotations
 
 import itertools
@@ -40,6 +41,20 @@ def test_every_chunk_in_one_segment(plans):
         assert out >= 3 and per >= 1 and (nt - 1) * ln < NT <= nt * ln, what  # no empty transition segment
         assert (out - 1) * per < nt <= out * per, what                        # nor output segment
         assert ws == ((nt - 2) * BH * K * K + (nt - 1) * BH * K * V + BH * V // 16) * 4, what
+
+
+def test_plans_of_the_gpu_tests(plans):
+    """test_gpu_segment_per.py is about plans of several transition segments per
+    output segment: its shapes have them, some with a remainder in each count."""
+    from tests.test_gpu_segment_per import FWD, H_BF16, H_F32
+
+    calls = [(f, B * H, NT, K, V) for f, shapes in (("fwd", FWD), ("hbf16", H_BF16), ("hf32", H_F32))
+             for B, H, NT, K, V in shapes]
+    got = plans(calls)
+    for c, (out, per, ln, _) in zip(calls, got, strict=True):
+        assert out >= 3 and per >= 2, c
+    assert sum(-(-c[2] // p[2]) % p[1] != 0 for c, p in zip(calls, got)) >= 4
+    assert sum(c[2] % p[2] != 0 for c, p in zip(calls, got)) >= 2
 
 
 @pytest.mark.parametrize("call", [
