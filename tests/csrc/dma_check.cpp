@@ -28,6 +28,10 @@
 //     and k tiles (padded, register-staged): the fragments hold the elements
 //     the products need and are read conflict-free; staging stores are
 //     conflict-free or bounded in conflicts;
+//   * the kernels on chunk records (rec_cfg.h; chunk_fwd_rec.hip, segments.h):
+//     the output kernel's LDS layout, DMA coverage, slot lifetimes and wait
+//     counts; the transition kernel's DMA list over its waves, 3-stage ring and
+//     waits, with and without records; the record's blocks and P's lane order;
 //   * the fused WY kernel's [k | v] tile (nat_row order): staging, transposed
 //     reads and form_L's row reads, all conflict-free;
 //   * chunk_fwd_o's pipelined kernel: its walk (desc_walk_at) maps walk
@@ -52,6 +56,7 @@
 #include "lds_banks.h"
 #include "handout.h"
 #include "pipe_cfg.h"
+#include "rec_cfg.h"
 
 using namespace thm;
 
@@ -501,6 +506,195 @@ static void check_fused() {
     }
 }
 
+// --------------------------------------------------------------------------- chunk records
+
+// The output kernel (chunk_fwd_rec.hip).
+template <int K, int V>
+static void check_rec_output() {
+  using C = rec::OCfg<K>;
+  constexpr int KB2 = C::KB / 2;
+  char what[64];
+  std::snprintf(what, sizeof what, "record output K=%d V=%d", K, V);
+  std::vector<std::pair<int, int>> reg;
+  for (int s = 0; s < 2; ++s) {
+    const int base = s * C::kStage, rb = base + 2 * C::kTileK + C::kTileVB;  // stage_k, _q, _v, _r
+    reg.push_back({base, base + C::kTileK});
+    reg.push_back({base + C::kTileK, base + 2 * C::kTileK});
+    reg.push_back({base + 2 * C::kTileK, rb});
+    reg.push_back({rb, rb + rec::kBlocks * rec::kBlockBytes});
+    reg.push_back({rb + rec::kGateOff, rb + rec::kGateOff + 1024});
+    CHECK(rb + rec::kBytes == base + C::kStage, "%s: stage %d size", what, s);
+  }
+  const int lp = 2 * C::kStage;
+  reg.push_back({lp, lp + C::kPBytes});
+  reg.push_back({lp + C::kPBytes, lp + C::kPBytes + C::kSBytes});
+  reg.push_back({lp + C::kPBytes + C::kSBytes, lp + C::kPBytes + C::kSBytes + C::kVBytes});
+  for (size_t i = 0; i < reg.size(); ++i) {
+    CHECK(reg[i].first % 16 == 0 && reg[i].second <= C::kLds, "%s: LDS region %zu", what, i);
+    for (size_t j = 0; j < i; ++j)
+      CHECK(reg[i].first >= reg[j].second || reg[j].first >= reg[i].second, "%s: LDS regions %zu and %zu overlap", what, i, j);
+  }
+  CHECK(((3 * KB2 + KB2 - 1) * 64 + 63) * 16 + 16 <= C::kSBytes, "%s: S hand-over slots", what);
+  CHECK(((3 * 2 + 1) * 64 + 63) * 16 + 16 <= C::kVBytes, "%s: v_new hand-over slots", what);
+  // The record: ten blocks, each loaded; the gate part's four rows of 64.
+  std::vector<int> blk(rec::kBlocks, 0);
+  for (int wq = 0; wq < 4; ++wq)
+    for (int i = 0; i < C::kADma; ++i) {
+      const int x = C::a_block(wq, i);
+      CHECK(x >= 0 && x < rec::kBlocks, "%s: A block %d", what, x);
+      if (x >= 0 && x < rec::kBlocks) blk[x]++;
+    }
+  for (int x = 0; x < rec::kBlocks; ++x)
+    CHECK(blk[x] == 1 || (x == rec::kBlocks - 1 && blk[x] > 0), "%s: A block %d loaded %d times", what, x, blk[x]);
+  for (const Shape& sh : kShapes) {
+    if (64 * sh.H * (K > V ? K : V) * 2 > (INT64_C(1) << 31)) continue;
+    const int64_t tsk = sh.H * K * 2, tsv = sh.H * V * 2;
+    check_tile_dma(C::kRowK, 4, C::kKDma, tsk, what);
+    check_tile_dma(C::kRowV, 4, C::kVDma, tsv, what);
+    const int64_t NT = sh.T / 64, b = sh.B - 1, hh = sh.H - 1, cc = NT - 1;
+    uint32_t kmax = 0, vmax = 0;
+    for (int P = 0; P < 64 * C::kRowK / 16; ++P) kmax = std::max(kmax, hl::dma_src_off(P, C::kRowK, tsk));
+    for (int P = 0; P < 64 * C::kRowV / 16; ++P) vmax = std::max(vmax, hl::dma_src_off(P, C::kRowV, tsv));
+    const int64_t kc0 = (b * sh.T * sh.H + hh) * K * 2, vc0 = (b * sh.T * sh.H + hh) * V * 2 + (V - 64) * 2;
+    CHECK(kc0 + cc * 64 * tsk + kmax + 16 <= sh.B * sh.T * sh.H * K * 2, "%s: k / q DMA past the tensor", what);
+    CHECK(vc0 + cc * 64 * tsv + vmax + 16 <= sh.B * sh.T * sh.H * V * 2, "%s: v DMA past the tensor", what);
+    CHECK(rec::offset(b * sh.H + hh, cc, NT) + rec::kBytes == sh.B * sh.H * NT * rec::kBytes, "%s: last record", what);
+    Cover co(64, V);
+    for (int vt = 0; vt < V / 64; ++vt)
+      for (int wq = 0; wq < 4; ++wq)
+        for (int ib = 0; ib < 4; ++ib)
+          store_tile(co, [&](int lane) { return (uint64_t)hl::quadT_off(0, vt * 64 + 16 * wq, lane, tsv, 2) + 16 * ib * tsv; },
+                     tsv, 2, what);
+    co.exactly_once(what);
+  }
+  // Slot lifetimes, phases as in check_fused: k, q and gates of chunk x are read
+  // in both of its phases and loaded in phase 1 of chunk x - 1; its A blocks
+  // and v are read in phase 1 and loaded in phase 2 of chunk x - 2.
+  for (int x = 2; x < 6; ++x) {
+    const int kq_issue = 2 * (x - 1), av_issue = 2 * (x - 2) + 1;
+    CHECK(kq_issue > 2 * (x - 2) + 1 && kq_issue < 2 * x, "%s: k / q DMA of chunk %d overlaps a reader", what, x);
+    CHECK(av_issue > 2 * (x - 2) && av_issue < 2 * x, "%s: A / v DMA of chunk %d overlaps a reader", what, x);
+  }
+  // Waits: at the end of chunk c the DMA of chunk c + 1 is in and that of
+  // chunk c + 2 (or a repeat of the last chunk) in flight.
+  for (int NT = 2; NT <= 6; ++NT)
+    for (int wq = 0; wq < 4; ++wq) {
+      WaveOps w;
+      const int nkq = 2 * C::kKDma + (wq == 0), nav = C::kADma + C::kVDma;
+      w.dma(0, nav);
+      w.dma(0, nkq);
+      w.dma(1, nav);
+      for (int c = 0; c < NT; ++c) {
+        w.dma(c + 1 < NT ? c + 1 : -2, nkq);
+        w.dma(c + 2 < NT ? c + 2 : -2, nav);
+        if (c + 1 < NT) w.check_wait(c + 1, C::kWait, what, c);
+      }
+    }
+}
+
+// The transition kernel (segments.h) on records, or (WU) on w and u.
+template <int K, int V, bool WU>
+static void check_transition() {
+  using C = rec::TCfg<K, V, WU>;
+  char what[64];
+  std::snprintf(what, sizeof what, "transition K=%d V=%d WU=%d", K, V, WU);
+  CHECK(C::kWaves * 32 == K + V && C::kPWaves * 32 == K, "%s: columns of [P | Q] over %d waves", what, C::kWaves);
+  CHECK(C::kOffV == C::kTileK && C::kOffR == C::kTileK + (V / 64) * C::kTileVB && C::kOffG + 1024 == C::kStage &&
+            C::kStages * C::kStage <= C::kLds && C::kLds <= 160 * 1024,
+        "%s: stage layout", what);
+  CHECK(WU ? C::kOffG == C::kOffR + C::kTileK : C::kOffG == C::kOffR + rec::kGateOff, "%s: gates", what);
+  // Each KiB of the stage (WU: but the gates', a 256-byte gather) by one
+  // instruction of one wave.
+  std::vector<int> seen(C::kInstr, 0);
+  for (int wi = 0; wi < C::kWaves; ++wi) {
+    const bool last = wi + (C::kDma - 1) * C::kWaves < C::kInstr;
+    for (int i = 0; i < C::kDma; ++i) {
+      const int j = wi + i * C::kWaves;
+      if (i + 1 == C::kDma && !last) continue;
+      CHECK(j < C::kInstr, "%s: wave %d instruction %d past the list", what, wi, i);
+      if (j < C::kInstr) seen[j]++;
+    }
+  }
+  for (int j = 0; j < C::kInstr; ++j) CHECK(seen[j] == 1, "%s: KiB %d of the stage loaded %d times", what, j, seen[j]);
+  CHECK(!WU || (C::kDma - 1) * C::kWaves < C::kInstr, "%s: wave 0, which gathers the gates, has every instruction", what);
+  for (const Shape& sh : kShapes) {
+    if (64 * sh.H * (K > V ? K : V) * 2 > (INT64_C(1) << 31)) continue;
+    const int64_t tsk = sh.H * K * 2, tsv = sh.H * V * 2, NT = sh.T / 64, b = sh.B - 1, hh = sh.H - 1;
+    const int64_t kc = (((b * sh.T + (NT - 1) * 64) * sh.H) + hh) * K * 2, vc = (((b * sh.T + (NT - 1) * 64) * sh.H) + hh) * V * 2;
+    for (int j = 0; j < C::kInstr; ++j)
+      for (int lane = 0; lane < 64; ++lane) {
+        const int at = j * 1024 + 16 * lane;  // in the stage
+        const uint32_t src = C::src_off(j, lane, tsk, tsv);
+        if (at < C::kOffV || (WU && at >= C::kOffR)) {  // k or w row-major tile
+          const auto d = decode((uint32_t)(at - (at < C::kOffV ? 0 : C::kOffR)), C::kRowK);
+          CHECK(C::from_k(j) == (at < C::kOffV) && !C::from_v(j) && (int64_t)src == d.first * tsk + 2 * d.second,
+                "%s: KiB %d lane %d fetched from %u", what, j, lane, src);
+          CHECK(kc + src + 16 <= sh.B * sh.T * sh.H * K * 2, "%s: k / w DMA past the tensor", what);
+        } else if (at < C::kOffR) {  // the v tile of columns 64 t ..
+          const int t = (at - C::kOffV) / C::kTileVB;
+          const auto d = decode((uint32_t)((at - C::kOffV) % C::kTileVB), C::kRowV);
+          CHECK(C::from_v(j) && !C::from_k(j) && (int64_t)src == d.first * tsv + 2 * (64 * t + d.second),
+                "%s: KiB %d lane %d fetched from %u", what, j, lane, src);
+          CHECK(vc + src + 16 <= sh.B * sh.T * sh.H * V * 2, "%s: v / u DMA past the tensor", what);
+        } else {  // the record, contiguous
+          CHECK(!C::from_k(j) && !C::from_v(j) && (int)src == at - C::kOffR && src + 16 <= (uint32_t)rec::kBytes,
+                "%s: KiB %d lane %d fetched from %u", what, j, lane, src);
+        }
+      }
+  }
+  // Waits and the ring, replaying a wave's issue order: chunks 0 and 1 (or a
+  // repeat) first; at chunk c the wait, a barrier, the DMA of chunk c + 2 (or
+  // a repeat of the last) into the stage chunk c - 1 was read from.
+  for (int gated = 0; gated <= (WU ? 1 : 0); ++gated)
+    for (int wi = 0; wi < C::kWaves; ++wi)
+      for (int n = 1; n <= 6; ++n) {
+        WaveOps w;
+        const bool last = wi + (C::kDma - 1) * C::kWaves < C::kInstr, gathers = gated && wi == 0;
+        const int per = C::kDma - !last + gathers;
+        w.dma(0, per);
+        w.dma(n > 1 ? 1 : -2, per);
+        int st = 0, sn = 2 % C::kStages;
+        for (int c = 0; c < n; ++c) {
+          w.check_wait(c, gathers ? C::kWait + (C::kStages - 2) : last ? C::kWait : C::kWait - (C::kStages - 2), what, c);
+          CHECK(st == c % C::kStages && sn == (c + 2) % C::kStages && sn != st && sn != (c + 1) % C::kStages,
+                "%s: chunk %d in stage %d, chunk %d into stage %d", what, c, st, c + 2, sn);
+          w.dma(c + 2 < n ? c + 2 : -2, per);
+          st = st == C::kStages - 1 ? 0 : st + 1;
+          sn = sn == C::kStages - 1 ? 0 : sn + 1;
+        }
+      }
+}
+
+// The record's block order and lanes against the recurrence kernels' reads; P's
+// lanes; the segments' workspace.
+static void check_rec_blocks() {
+  int p = 0;
+  for (int ib = 0; ib < 4; ++ib)
+    for (int jb = 0; jb <= ib; ++jb, ++p) {
+      CHECK(rec::block(ib, jb) == p, "record block (%d, %d) at %d", ib, jb, rec::block(ib, jb));
+      // a_frags reads block (ib, 2 s2) and, up to the diagonal, the next one.
+      CHECK(jb % 2 == 0 || rec::block(ib, jb) == rec::block(ib, jb - 1) + 1, "record block (%d, %d)", ib, jb);
+    }
+  CHECK(p == rec::kBlocks, "%d blocks in a record", p);
+  const int parts[4] = {rec::kG, rec::kEg, rec::kEgl, rec::kBeta};
+  for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 4; ++j)
+      CHECK(parts[i] >= 0 && parts[i] + 64 <= 256 && (i == j || parts[i] >= parts[j] + 64 || parts[j] >= parts[i] + 64),
+            "gate parts %d and %d of a record", i, j);
+  for (int lane = 0; lane < 64; ++lane) {  // held: row 4 grp + li / 4, columns 4 (li % 4) ..
+    const int row = 4 * (lane >> 4) + ((lane & 15) >> 2), col = 4 * (lane & 3), s = rec::p_slot(lane);
+    CHECK((s & 15) == row && 4 * (s >> 4) == col, "P slot %d of lane %d", s, lane);
+  }
+  for (int64_t K : {64, 128})
+    for (int64_t V : {64, 128})
+      for (int64_t BH : {1, 5})
+        for (int64_t nt : {3, 7}) {
+          CHECK(rec::p_off(1, 0, BH, K) == 0 && rec::p_off(nt - 2, BH - 1, BH, K) + K * K * 4 == (nt - 2) * BH * K * K * 4 &&
+                    rec::s_off(0, 0, BH, K, V) == 0 && rec::s_off(nt - 2, BH - 1, BH, K, V) + K * V * 4 == (nt - 1) * BH * K * V * 4,
+                "segment workspace");
+        }
+}
+
 // --------------------------------------------------------------------------- small-grid chunk_fwd_h
 
 // The register-staged small-grid kernel (chunk_fwd_h_small.h): the memory
@@ -894,33 +1088,35 @@ static void check_nat_row_reads(int n, int kcols, const char* what) {
 }
 
 // The WY inversion's 16x16 fp32 blocks (wy_blocks.h through h_layout.h): the
-// accumulator writes are conflict-free, block_mm's operand reads at most
-// 2-way, and each access lands on the element its role names, inside the
-// block's rows.
+// accumulator writes are conflict-free, the row reads aligned, each access lands
+// on the element its role names, inside the block, and the substitution's reads
+// of one element of each diagonal block lie in different banks.
 static void check_wy_blocks() {
   const char* what = "WY inversion blocks";
-  for (int r = 0; r < 4; ++r) {
-    uint32_t addr[64];
-    for (int lane = 0; lane < 64; ++lane) {
-      const int o = hl::wy_put_off(lane, r);
-      CHECK(o / hl::kWyPitch == 4 * (lane >> 4) + r && o % hl::kWyPitch == (lane & 15), "%s: put lane %d", what, lane);
-      addr[lane] = 4 * o;
+  for (int p = 0; p < 10; ++p)
+    for (int r = 0; r < 4; ++r) {
+      uint32_t addr[64];
+      for (int lane = 0; lane < 64; ++lane) {
+        const int o = hl::wy_put_off(lane, r);
+        CHECK(o / hl::kWyPitch == 4 * (lane >> 4) + r && o % hl::kWyPitch == (lane & 15), "%s: put lane %d", what, lane);
+        addr[lane] = 4 * (p * hl::kWyBlk + o);
+      }
+      check_banks(addr, 4, kLdsWrite, what, r, p);
     }
-    check_banks(addr, 4, kLdsWrite, what, r, 0);
-  }
-  for (int q = 0; q < 4; ++q) {
-    uint32_t pa[64], qa[64];
+  for (int p = 0; p < 10; ++p)
     for (int lane = 0; lane < 64; ++lane) {
-      const int a = hl::wy_a_off(lane, q), b = hl::wy_b_off(lane, q);
-      CHECK(a / hl::kWyPitch == (lane & 15) && a % hl::kWyPitch == 4 * q + (lane >> 4), "%s: A operand lane %d", what, lane);
-      CHECK(b / hl::kWyPitch == 4 * q + (lane >> 4) && b % hl::kWyPitch == (lane & 15), "%s: B operand lane %d", what, lane);
-      pa[lane] = 4 * a;
-      qa[lane] = 4 * b;
+      const int a = hl::wy_row_off(lane);
+      CHECK(a / hl::kWyPitch == (lane & 15) && a % hl::kWyPitch == 4 * (lane >> 4) && a + 4 <= hl::kWyBlk, "%s: row lane %d",
+            what, lane);
+      CHECK(4 * (p * hl::kWyBlk + a) % 16 == 0, "%s: row read of block %d lane %d misaligned", what, p, lane);
     }
-    check_banks(pa, 4, kLdsRead, what, q, 0, 2);
-    check_banks(qa, 4, kLdsRead, what, q, 1, 2);
-  }
-  CHECK(hl::kWyPitch >= 16, "%s: pitch below the block's width", what);
+  for (int r = 0; r < 16; ++r)
+    for (int e = 0; e < r; ++e) {
+      std::set<int> banks;
+      for (int d = 0; d < 4; ++d) banks.insert((rec::block(d, d) * hl::kWyBlk + r * hl::kWyPitch + e) % 32);
+      CHECK(banks.size() == 4, "%s: element (%d, %d) of the diagonal blocks in %zu banks", what, r, e, banks.size());
+    }
+  CHECK(hl::kWyPitch >= 16 && hl::kWyBlk >= 16 * hl::kWyPitch, "%s: pitch or block too small", what);
 }
 
 // The XCD-aware tile order of recompute_w_u and the A-builder: a bijection of
@@ -1184,6 +1380,15 @@ int main() {
   F_ALL(64, 128)
   F_ALL(128, 64)
   F_ALL(128, 128)
+  check_rec_blocks();
+#define R_ALL(K, V)               \
+  check_rec_output<K, V>();       \
+  check_transition<K, V, false>(); \
+  check_transition<K, V, true>();
+  R_ALL(64, 64)
+  R_ALL(64, 128)
+  R_ALL(128, 64)
+  R_ALL(128, 128)
   for (int K : {64, 128})
     for (int V : {64, 128}) {
       char what[96];

@@ -9,7 +9,7 @@ pipelined kernel hands out its tiles at run time (dyn_tile) and loads them with
 32-bit per-lane offsets.  A slip there
 would fault the GPU or race rather than fail a numerical test, so
 tests/csrc/dma_check.cpp evaluates the very index functions and layout
-constants the kernels use (theorem_amd/csrc/h_layout.h, pipe_cfg.h) on the
+constants the kernels use (theorem_amd/csrc/h_layout.h, pipe_cfg.h, rec_cfg.h) on the
 host: DMA coverage and global bounds, read/write consistency of the swizzle,
 bank conflicts, store coverage and the wait counts.  The tile-load addressing
 it checks replaces kernels/chunk_fwd_h/kernel.py:103-114 (Triton block
@@ -150,7 +150,32 @@ MUTATIONS = [
     ("h_layout.h", "constexpr int kWyPitch = 20;", "constexpr int kWyPitch = 17;",
      "WY blocks: pitch 17 (2-way accumulator writes)"),
     ("h_layout.h", "constexpr int kWyPitch = 20;", "constexpr int kWyPitch = 16;",
-     "WY blocks: pitch 16 (4-way A operand reads)"),
+     "WY blocks: pitch 16 (2-way accumulator writes)"),
+    ("h_layout.h", "constexpr int kWyBlk = 16 * kWyPitch + 4;", "constexpr int kWyBlk = 16 * kWyPitch;",
+     "WY blocks: diagonal blocks unpadded (one bank for the substitution's reads)"),
+    ("h_layout.h", "return (lane & 15) * kWyPitch + 4 * (lane >> 4); }", "return (lane & 15) * kWyPitch + 2 * (lane >> 4); }",
+     "WY blocks: row reads overlap"),
+    ("rec_cfg.h", "  static constexpr int kWait = kAvDma;", "  static constexpr int kWait = kAvDma + 1;",
+     "record output: wait one op too loose"),
+    ("rec_cfg.h", "return wq + 4 * i < kBlocks ? wq + 4 * i : kBlocks - 1; }",
+     "return wq + 4 * i < kBlocks - 1 ? wq + 4 * i : kBlocks - 2; }",
+     "record output: the last A block not loaded"),
+    ("rec_cfg.h", "static constexpr int kLds = 2 * kStage + kPBytes + kSBytes + kVBytes;",
+     "static constexpr int kLds = 2 * kStage + kPBytes + kSBytes;",
+     "record output: v_new slots past the workgroup's LDS"),
+    ("rec_cfg.h", "static constexpr int kWait = (kStages - 2) * kDma;", "static constexpr int kWait = (kStages - 2) * kDma + 1;",
+     "transition: wait one op too loose"),
+    ("rec_cfg.h", "static constexpr int kDma = (kInstr + kWaves - 1) / kWaves;", "static constexpr int kDma = kInstr / kWaves;",
+     "transition: the list's last round dropped"),
+    ("rec_cfg.h", "(uint32_t)((x / kPer) * kRowV)", "(uint32_t)((x / kPer) * kRowK)",
+     "transition: the second v tile from the wrong columns"),
+    ("rec_cfg.h", "kOffG = kInstr * 1024 - (WU ? 0 : 1024);", "kOffG = kInstr * 1024;",
+     "transition: gates read past the record"),
+    ("rec_cfg.h", "{ return ib * (ib + 1) / 2 + jb; }", "{ return ib * (ib - 1) / 2 + jb; }",
+     "record: block order"),
+    ("rec_cfg.h", "return 16 * (lane & 3) + 4 * (lane >> 4) + ((lane & 15) >> 2); }",
+     "return 16 * (lane >> 4) + 4 * (lane & 3) + ((lane & 15) >> 2); }",
+     "P: lanes of the transposed block"),
     ("h_layout.h", "return half_swz && ((t >> 3) & 1); }", "return half_swz && ((t >> 2) & 1); }",
      "recompute_w_u output staging: half swap by the wrong token bit"),
     ("h_layout.h", "return (uint32_t)((t * hp + head) * row_bytes + ((q ^ (t & 7)) << 4));",
@@ -168,7 +193,7 @@ def test_dma_layout_check_catches_planted_slip(tmp_path, header, old, new, what)
     assert text.count(old) == 1, f"mutation site not found in {header}: {old}"
     mut = tmp_path / "mut"
     mut.mkdir()
-    for h in ("h_layout.h", "pipe_cfg.h", "handout.h"):
+    for h in ("h_layout.h", "pipe_cfg.h", "handout.h", "rec_cfg.h"):
         (mut / h).write_text((CSRC / h).read_text())
     (mut / header).write_text(text.replace(old, new))
     r = _build_and_run(tmp_path, include_first=mut)

@@ -376,7 +376,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   }
 
   if constexpr (TRANS) {
-    const int slot = 16 * (li & 3) + 4 * grp + (li >> 2);  // of row 4 grp + li / 4 (acc_to_row_quads)
+    const int slot = rec::p_slot(lane);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       if (is_p)

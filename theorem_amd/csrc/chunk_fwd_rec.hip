@@ -120,8 +120,7 @@ chunk_output_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, cons
     const char* rb = r0 + c * rec::kBytes;
 #pragma unroll
     for (int i = 0; i < C::kADma; ++i) {
-      int x = wq + 4 * i;
-      x = x < rec::kBlocks ? x : rec::kBlocks - 1;
+      const int x = C::a_block(wq, i);
       dma_b128(rb, (uint32_t)(x * rec::kBlockBytes + 16 * lane),
                __builtin_amdgcn_readfirstlane(lds_address(stage_r(s)) + x * rec::kBlockBytes));
     }

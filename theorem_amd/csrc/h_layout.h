@@ -116,21 +116,20 @@ THM_HD constexpr uint32_t xtr_frag_off(int k0, int half, int c0, int lane, int r
 }
 
 // The WY inversion's 16x16 fp32 blocks in LDS (wy_blocks.h), rows kWyPitch
-// floats apart.  Under gfx950's LDS bank model (4-byte writes and reads in
-// 32-lane passes over 32 banks) a pitch of 20 makes the accumulator writes
-// (block_put, form_L) conflict-free and leaves block_mm's operand reads
-// 2-way; no pitch makes all three conflict-free (17 left all three 2-way:
-// A-builder 110.8 -> 105.5 us at config 4, fused WY 233.2 -> 231.4,
-// bit-identical).
+// floats apart.  Under gfx950's LDS bank model (4-byte writes in 32-lane passes
+// over 32 banks) a pitch of 20 makes the accumulator writes (block_put,
+// form_L) conflict-free and aligns the products' 16-byte row reads (17 left
+// the writes 2-way: A-builder 110.8 -> 105.5 us at config 4, fused WY 233.2 ->
+// 231.4, bit-identical).  Blocks are kWyBlk floats apart, 4 over the rows: the
+// substitution reads one element of each of the four diagonal blocks (packed
+// blocks 0, 2, 5, 9) in one instruction, which then lie in different banks.
 // Float offsets within a block, lane (g = lane / 16, l = lane % 16):
-//   accumulator row 4 g + r, column l;  A operand row l, column 4 q + g;
-//   B operand row 4 q + g, column l.
+//   put: row 4 g + r, column l (accumulator form, also the B operand's);
+//   row: row l, columns 4 g .. 4 g + 3 in one 16-byte read (A operand).
 constexpr int kWyPitch = 20;
+constexpr int kWyBlk = 16 * kWyPitch + 4;
 THM_HD constexpr int wy_put_off(int lane, int r) { return (4 * (lane >> 4) + r) * kWyPitch + (lane & 15); }
-THM_HD constexpr int wy_a_off(int lane, int q) { return (lane & 15) * kWyPitch + 4 * q + (lane >> 4); }
-//   (wy_row_off: A operand row l, columns 4 g .. 4 g + 3 in one 16-byte read)
 THM_HD constexpr int wy_row_off(int lane) { return (lane & 15) * kWyPitch + 4 * (lane >> 4); }
-THM_HD constexpr int wy_b_off(int lane, int q) { return (4 * q + (lane >> 4)) * kWyPitch + (lane & 15); }
 
 // recompute_w_u's output staging tile: the w (or u) rows of the tile's 64
 // tokens x hp heads in their global order (physical row t hp + head), each

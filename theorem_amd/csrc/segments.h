@@ -35,7 +35,7 @@ __device__ __forceinline__ bf16x8 row_frag(const char* tile, int ib, int s2, int
 // A operands of row block ib, contraction step s2, of the record's A: hi and
 // lo.  Block (ib, 2 s2 + 1) lies above the diagonal for ib = 2 s2: zero.
 __device__ __forceinline__ void a_frags(const char* r, int ib, int s2, int lane, bf16x8& ah, bf16x8& al) {
-  const int p = ib * (ib + 1) / 2 + 2 * s2;
+  const int p = rec::block(ib, 2 * s2);
   const u32x4 x0 = *reinterpret_cast<const u32x4*>(r + p * rec::kBlockBytes + 16 * lane);
   u32x4 x1 = {0u, 0u, 0u, 0u};
   if (2 * s2 + 1 <= ib) x1 = *reinterpret_cast<const u32x4*>(r + (p + 1) * rec::kBlockBytes + 16 * lane);
@@ -109,21 +109,17 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
   const char* const g0 = WU && HAS_G ? reinterpret_cast<const char*>(g) + ((b * T + sp.c0 * kBT) * H + hh) * 4 : nullptr;
 
   // This wave's DMA instructions of a chunk: j = wi + i kWaves of the list
-  // (k tile, v tiles, record or w tile); wave 0 also gathers the gates for WU.  Lane offset, LDS offset and source per i.
+  // (k tile, v tiles, record or w tile), each to its KiB of the stage; wave 0
+  // also gathers the gates for WU.
   uint32_t voff[C::kDma], loff[C::kDma];
   bool from_k[C::kDma], from_v[C::kDma];
 #pragma unroll
   for (int i = 0; i < C::kDma; ++i) {
     const int j = wi + i * C::kWaves;
-    constexpr int kPer = C::kTileVB / 1024;  // instructions per v tile
-    from_k[i] = j < C::kKInstr;
-    from_v[i] = !from_k[i] && j < C::kKInstr + C::kVInstr;
-    const int x = from_k[i] ? j : from_v[i] ? j - C::kKInstr : j - C::kKInstr - C::kVInstr;
-    voff[i] = from_k[i]   ? hl::dma_src_off(x * 64 + lane, C::kRowK, tsk)
-              : from_v[i] ? hl::dma_src_off((x % kPer) * 64 + lane, C::kRowV, tsv) + (uint32_t)((x / kPer) * C::kRowV)
-              : WU        ? hl::dma_src_off(x * 64 + lane, C::kRowK, tsk)
-                          : (uint32_t)(x * 1024 + lane * 16);
-    loff[i] = (uint32_t)(j * 1024);  // the stage holds the tiles in the list's order
+    from_k[i] = C::from_k(j);
+    from_v[i] = C::from_v(j);
+    voff[i] = C::src_off(j, lane, tsk, tsv);
+    loff[i] = (uint32_t)(j * 1024);
   }
   const bool last_dma = wi + (C::kDma - 1) * C::kWaves < C::kInstr;  // else one instruction fewer
   // Chunk c into the stage at byte `st`.
@@ -184,9 +180,9 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
     }
     if (!active) continue;
     const char* tk = lds + st;
-    const char* tv = tk + C::kTileK + v_tile;
-    const char* tr = tk + C::kTileK + C::kNVT * C::kTileVB;  // the record, or the w tile
-    const float* gp = reinterpret_cast<const float*>(tk + C::kInstr * 1024 - (WU ? 0 : 1024));
+    const char* tv = tk + C::kOffV + v_tile;
+    const char* tr = tk + C::kOffR;  // the record, or the w tile
+    const float* gp = reinterpret_cast<const float*>(tk + C::kOffG);
 
     bf16x8 sb[CT][KB2];
 #pragma unroll
@@ -305,12 +301,10 @@ chunk_transition_kernel(const bf16* __restrict__ k, const bf16* __restrict__ w, 
   wait_vmcnt<0>();  // no DMA may still target this workgroup's LDS when it exits
   if (!active) return;
 
-  // P in 16 x 16 blocks (row block, column block) of A-operand lanes: lane
-  // (grp, li) holds P[16 kb + li][16 nb + 4 grp .. + 3]; after acc_to_row_quads
-  // lane (g, 4 a + b) holds row 4 g + a, columns 4 b .. + 3.  Q in blocks
-  // (column block, row block) of accumulator lanes.
+  // P in 16 x 16 blocks (row block, column block) of A-operand lanes (rec_cfg.h
+  // p_slot), Q in blocks (column block, row block) of accumulator lanes.
   if (is_p) {
-    const int slot = 16 * (li & 3) + 4 * grp + (li >> 2);
+    const int slot = rec::p_slot(lane);
     char* const pb = pbuf + rec::p_off(seg, bh, BH, K) + (n0 / 16) * 1024 + 16 * slot;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)

@@ -5,7 +5,7 @@
 // e^{g_i - g_j}, the chunk's A = (I + L)^{-1} is block lower triangular in
 // 16 x 16 blocks:
 //   X_ii = (I + L_ii)^{-1}                        (forward substitution)
-//   X_ij = -X_ii sum_{m=j}^{i-1} L_im X_mj        (i > j, by distance i - j)
+//   X_ij = -X_ii sum_{m=j}^{i-1} L_im X_mj        (i > j, a column j per wave)
 // Lower blocks (i, j), j <= i < 4, are stored packed (blk(i, j)) in LDS with
 // row pitch kBP floats.  The math follows the reference's `_build_A`
 // (kernels/recompute_w_u/reference.py:48-91: a torch matmul for M and
@@ -20,9 +20,7 @@ namespace wy {
 
 constexpr int kBT = 64;
 constexpr int kBP = hl::kWyPitch;  // LDS pitch (floats) of a 16x16 block (h_layout.h)
-// Floats per block, 4 over the rows: the four diagonal blocks (the substitution
-// reads all of them in one instruction) then start on different banks.
-constexpr int kBlk = 16 * kBP + 4;
+constexpr int kBlk = hl::kWyBlk;   // floats per block
 constexpr int kLdsFloats = 10 * kBlk + 10 * kBlk;  // L, X
 
 // Packed index of lower block (i, j), j <= i < 4.

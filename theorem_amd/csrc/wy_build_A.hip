@@ -9,7 +9,7 @@
 // L = sign M (strictly lower) and 16x16 blocks L_ij, X = (I + L)^{-1} is block
 // lower triangular:
 //   X_ii = (I + L_ii)^{-1}                        (forward substitution)
-//   X_ij = -X_ii sum_{m=j}^{i-1} L_im X_mj        (i > j, by distance i - j)
+//   X_ij = -X_ii sum_{m=j}^{i-1} L_im X_mj        (i > j, a column j per wave)
 //   1. k k^T on v_mfma_f32_16x16x32_bf16: lane (g, j) holds features
 //      8g .. 8g+7 of token j of a 16-token block, so the A fragment of block ib
 //      and the B fragment of block jb are the same kind of 16-byte row load
