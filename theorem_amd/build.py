@@ -42,7 +42,7 @@ SOURCES = [
 
 # Per-unit code generation.  Forcing MFMA accumulators into VGPRs (no AGPR
 # copies) measured faster for these units (recompute_w_u bf16 275.1 -> 271.6 us,
-# the bf16 register chunk_fwd_h at config 3 25.5 -> 24.4 us, config 4
+# a bf16 register form of chunk_fwd_h at config 3 25.5 -> 24.4 us, config 4
 # bit-identical outputs) and slower for the fp32 register chunk_fwd_h and the
 # fp32 chunk_fwd_o (775 -> 884 and 883 -> 927 us), so it is not global.
 MFMA_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]

@@ -20,9 +20,8 @@
 //     (thm_chunk_fwd_h_ws): long sequences cut into segments (segments.h).
 // This unit is compiled with MFMA accumulators forced into VGPRs
 // (theorem_amd/build.py).
-#include "chunk_fwd_h_reg.h"
+#include "chunk_fwd_h.h"
 #include "chunk_fwd_h_small.h"
-
 #include "pipe_cfg.h"
 #include "segments.h"
 

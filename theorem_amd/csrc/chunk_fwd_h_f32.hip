@@ -24,7 +24,7 @@ hipError_t launch_f32(const void* k, const void* w, const void* vu, const void* 
     if (p.out == 1 && B * H * (V / kHBV) < kHDmaMinGrid)
       return launch_h_small<float, K, V, kHSmallNW, DELTA>(k, w, vu, g, h0, h, vnew, ht, B, T, H, s);
   }
-  return launch_h<float, K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
+  return launch_h<K, V, DELTA>(k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);
 }
 
 template <bool DELTA>
@@ -39,9 +39,9 @@ hipError_t dispatch_f32(int64_t K, int64_t V, const void* k, const void* w, cons
 
 }  // namespace
 
-__attribute__((visibility("hidden"))) hipError_t chunk_fwd_h_f32(bool delta, int64_t K, int64_t V, const void* k, const void* w, const void* vu,
-                           const void* g, const void* h0, void* h, void* vnew, void* ht, char* ws, int64_t out, int64_t per,
-                           int64_t len, int64_t B, int64_t T, int64_t H, hipStream_t s) {
+hipError_t chunk_fwd_h_f32(bool delta, int64_t K, int64_t V, const void* k, const void* w, const void* vu,
+                           const void* g, const void* h0, void* h, void* vnew, void* ht, char* ws, int64_t out,
+                           int64_t per, int64_t len, int64_t B, int64_t T, int64_t H, hipStream_t s) {
   const seg::Plan p = {out, per, len};
   return delta ? dispatch_f32<true>(K, V, k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s)
                : dispatch_f32<false>(K, V, k, w, vu, g, h0, h, vnew, ht, ws, p, B, T, H, s);

@@ -1,6 +1,5 @@
-// Gated DeltaNet inter-chunk state recurrence, register-prefetch kernel
-// (included by chunk_fwd_h.hip for bf16 inputs and by chunk_fwd_h_f32.hip for
-// fp32 inputs; the two are compiled with different code-generation options).
+// Gated DeltaNet inter-chunk state recurrence, register-prefetch kernel for
+// fp32 inputs (instantiated in chunk_fwd_h_f32.hip).
 //
 // For one (b, head), state S [K x V] fp32 (h0 or 0 at chunk 0), per chunk c
 // with g_last = g at the chunk's last token:
@@ -29,14 +28,11 @@
 // Workgroups map XCD-aware: the V-tiles of one (b, head) share an XCD (and its
 // L2), so k and w are fetched from HBM once per (b, head).
 //
-// bf16 inputs on grids that fill the GPU use a second kernel
-// (chunk_fwd_h.hip): chunk tiles arrive by global -> LDS DMA instead of
-// through registers, and the K rows of the state are split over two waves per
-// SIMD.
+// Every product takes its fp32 operands as bf16 hi + lo and drops lo lo (~2^-16).
+// bf16 inputs have kernels of their own (chunk_fwd_h.hip, chunk_fwd_h_small.h).
 #pragma once
 
-#include <type_traits>
-
+#include "chunk_fwd_h.h"
 #include "h_layout.h"
 #include "mfma.h"
 #include "segments.h"
@@ -45,21 +41,17 @@
 namespace thm {
 namespace {
 
-constexpr int kBT = 64;
-constexpr int kHBV = 64;  // V-tile width
 // BV columns per workgroup, a wavefront for every 16.
-template <typename IT, int K, int V, bool DELTA, int BV>
+template <int K, int V, bool DELTA, int BV>
 struct HCfg {
   static constexpr int kThreads = 4 * BV;
-  static constexpr bool kSplit = std::is_same<IT, float>::value;
-  static constexpr int kEB = (int)sizeof(IT);
-  static constexpr int kVE = 16 / kEB;               // elements per 16-byte load
+  static constexpr int kVE = 4;                      // elements per 16-byte load
   static constexpr int kKPitch = K + 8;              // bf16 elements (16-byte pad)
-  static constexpr int kUPitch = BV + kVE;         // IT elements (16-byte pad)
+  static constexpr int kUPitch = BV + kVE;           // floats (16-byte pad)
   static constexpr int kKTile = kBT * kKPitch;       // bf16 elements
-  static constexpr int kUTile = kBT * kUPitch;       // IT elements
-  // bf16 elements of one stage: k (hi[, lo]), w (hi[, lo]) when DELTA
-  static constexpr int kBf16PerStage = (kSplit ? 2 : 1) * (DELTA ? 2 : 1) * kKTile;
+  static constexpr int kUTile = kBT * kUPitch;       // floats
+  // bf16 elements of one stage: k (hi, lo), w (hi, lo) when DELTA
+  static constexpr int kBf16PerStage = 2 * (DELTA ? 2 : 1) * kKTile;
   // per-thread 16-byte load slots of one chunk
   static constexpr int kKCPR = K / kVE;              // 16-byte chunks per k / w row
   static constexpr int kKLoads = kBT * kKCPR / kThreads;
@@ -68,58 +60,53 @@ struct HCfg {
   static_assert(kThreads % kKCPR == 0 && kThreads % kUCPR == 0, "slot mapping");
   static_assert(kBT * kKCPR % kThreads == 0 && kBT * kUCPR % kThreads == 0, "slot count");
   static constexpr int kStageBytes =
-      kBf16PerStage * 2 + kUTile * kEB + kBT * (int)sizeof(float);
+      kBf16PerStage * 2 + (kUTile + kBT) * (int)sizeof(float);
   // Double-buffer the stage when two fit in 128 KiB of LDS; otherwise one stage
-  // (fp32 inputs with K = 128) and a barrier before it is overwritten.
+  // (K = 128) and a barrier before it is overwritten.
   static constexpr int kStages = (2 * kStageBytes <= 128 * 1024) ? 2 : 1;
 };
 
-template <typename IT>
 struct HStage {
   bf16* khi;
   bf16* klo;
   bf16* whi;
   bf16* wlo;
-  IT* u;
+  float* u;
   float* g;
 };
 
 // One chunk's loads, in registers.
-template <typename IT, int K, int V, bool DELTA, int BV>
+template <int K, int V, bool DELTA, int BV>
 struct HPrefetch {
-  using C = HCfg<IT, K, V, DELTA, BV>;
+  using C = HCfg<K, V, DELTA, BV>;
   u32x4 k[C::kKLoads];
   u32x4 w[DELTA ? C::kKLoads : 1];
   u32x4 u[C::kULoads];
   float g;  // gate of token lane_id() of the chunk
 };
 
-__device__ __forceinline__ const char* cptr(const void* p, int64_t byte_off) {
-  return reinterpret_cast<const char*>(p) + byte_off;
-}
-
 // DEEP: two register sets, two chunks ahead (see the chunk loop below).
 // Segments (segments.h): a workgroup walks the `len` chunks of its segment,
 // from the combine kernel's state in sbuf.  TRANS: the transition kernel of
 // this form, over column tiles of [P | Q]; only the final state is written, P
 // in A-operand blocks and Q in accumulator blocks, both fp32.
-template <typename IT, int K, int V, bool DELTA, bool HAS_G, bool DEEP, bool TRANS, int BV>
+template <int K, int V, bool DELTA, bool HAS_G, bool DEEP, bool TRANS, int BV>
 __global__ void __launch_bounds__(4 * BV)
-chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT* __restrict__ vu,
+chunk_fwd_h_kernel(const float* __restrict__ k, const float* __restrict__ w, const float* __restrict__ vu,
                    const float* __restrict__ g, const float* __restrict__ h0,
-                   float* __restrict__ hout, IT* __restrict__ vnew, float* __restrict__ ht,
+                   float* __restrict__ hout, float* __restrict__ vnew, float* __restrict__ ht,
                    char* __restrict__ pbuf, char* __restrict__ sbuf, const uint32_t* __restrict__ redo,
                    int64_t T, int64_t H,
                    int64_t NTotal, int64_t BH, int64_t nseg, int64_t len, int64_t per) {
-  using C = HCfg<IT, K, V, DELTA, BV>;
-  using St = HStage<IT>;
-  using Pf = HPrefetch<IT, K, V, DELTA, BV>;
+  using C = HCfg<K, V, DELTA, BV>;
+  using St = HStage;
+  using Pf = HPrefetch<K, V, DELTA, BV>;
   constexpr int KB = K / 16;
   constexpr int NPT = TRANS ? K / BV : 0;  // column tiles of P, ahead of the V-tiles
   constexpr int NVT = NPT + V / BV;
-  constexpr int EB = C::kEB;
+  constexpr int EB = 4;  // bytes per element
   __shared__ __attribute__((aligned(16))) bf16 lds_b[C::kStages * C::kBf16PerStage];
-  __shared__ __attribute__((aligned(16))) IT lds_u[C::kStages * C::kUTile];
+  __shared__ __attribute__((aligned(16))) float lds_u[C::kStages * C::kUTile];
   __shared__ __attribute__((aligned(16))) float lds_g[C::kStages * kBT];
 
   // XCD-aware block mapping: the column tiles of one (b, head, segment) share an XCD.
@@ -139,9 +126,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
     St st;
     bf16* base = lds_b + i * C::kBf16PerStage;
     st.khi = base;
-    st.klo = base + (C::kSplit ? C::kKTile : 0);
-    st.whi = base + (C::kSplit ? 2 : 1) * C::kKTile;
-    st.wlo = st.whi + (C::kSplit ? C::kKTile : 0);
+    st.klo = base + C::kKTile;
+    st.whi = base + 2 * C::kKTile;
+    st.wlo = st.whi + C::kKTile;
     st.u = lds_u + i * C::kUTile;
     st.g = lds_g + i * kBT;
     return st;
@@ -195,17 +182,12 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
 #pragma unroll
     for (int it = 0; it < C::kKLoads; ++it) {
       const int off = (kj0 + it * (C::kThreads / C::kKCPR)) * C::kKPitch + kcol;
-      if constexpr (C::kSplit) {
-        float vals[4];
-        unpack16(pf.k[it], vals, 0.f);
-        lds_put4(st.khi + off, st.klo + off, vals, true);
-        if constexpr (DELTA) {
-          unpack16(pf.w[it], vals, 0.f);
-          lds_put4(st.whi + off, st.wlo + off, vals, true);
-        }
-      } else {
-        *reinterpret_cast<u32x4*>(st.khi + off) = pf.k[it];
-        if constexpr (DELTA) *reinterpret_cast<u32x4*>(st.whi + off) = pf.w[it];
+      float vals[4];
+      unpack16(pf.k[it], vals, 0.f);
+      lds_put4(st.khi + off, st.klo + off, vals, true);
+      if constexpr (DELTA) {
+        unpack16(pf.w[it], vals, 0.f);
+        lds_put4(st.whi + off, st.wlo + off, vals, true);
       }
     }
 #pragma unroll
@@ -239,8 +221,8 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
 
   // v_new rows j = 16 jb + 4 grp + r of this lane's column, relative to the chunk base.
   // (h and v_new are stored one element per lane: 16 consecutive lanes cover
-  // 64 / 32 contiguous bytes of a row.  The row-quad re-layout of the DMA
-  // kernel below is slower here: 31.0 against 25.6 us at config 3.)
+  // 64 contiguous bytes of a row.  The row-quad re-layout of the bf16 DMA kernel
+  // was slower in a bf16 form of this one: 31.0 against 25.6 us at config 3.)
   const uint32_t vn_off = (uint32_t)(4 * grp * tok_stride_v + vcol * EB);
   auto store_state = [&](int64_t c) {
     char* hb = reinterpret_cast<char*>(hout) + ((b * NTotal + sp.c0 + c) * H + hh) * (int64_t)(K * V) * 4;
@@ -283,7 +265,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
     for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = to_f32(cs.u[(16 * jb + 4 * grp + r) * C::kUPitch + ucol]);
+        const float x = cs.u[(16 * jb + 4 * grp + r) * C::kUPitch + ucol];
         vn[jb][r] = is_p ? 0.f : x;
       }
 
@@ -294,8 +276,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
       for (int s = 0; s < K / 32; ++s) {
         const float f[8] = {S[2 * s][0], S[2 * s][1], S[2 * s][2], S[2 * s][3],
                             S[2 * s + 1][0], S[2 * s + 1][1], S[2 * s + 1][2], S[2 * s + 1][3]};
-        if constexpr (C::kSplit) split_bf16x8(f, sh[s], sl[s]);
-        else sh[s] = to_bf16x8(f);
+        split_bf16x8(f, sh[s], sl[s]);
       }
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb) {
@@ -305,11 +286,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
         for (int s = 0; s < K / 32; ++s) {
           const bf16x8 wf = load8_paired(wrow, 32 * s);
           a = mfma16x16x32(wf, sh[s], a);
-          if constexpr (C::kSplit) {
-            a = mfma16x16x32(wf, sl[s], a);
-            const bf16x8 wl = load8_paired(cs.wlo + (16 * jb + li) * C::kKPitch, 32 * s);
-            a = mfma16x16x32(wl, sh[s], a);
-          }
+          a = mfma16x16x32(wf, sl[s], a);
+          const bf16x8 wl = load8_paired(cs.wlo + (16 * jb + li) * C::kKPitch, 32 * s);
+          a = mfma16x16x32(wl, sh[s], a);
         }
         vn[jb] -= a;
       }
@@ -327,8 +306,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
         f[r] = vn[2 * s][r] * fast_exp(gl - cs.g[j0]);
         f[4 + r] = vn[2 * s + 1][r] * fast_exp(gl - cs.g[j0 + 16]);
       }
-      if constexpr (C::kSplit) split_bf16x8(f, vh[s], vl[s]);
-      else vh[s] = to_bf16x8(f);
+      split_bf16x8(f, vh[s], vl[s]);
     }
     const float decay = fast_exp(gl);
 #pragma unroll
@@ -339,11 +317,9 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
         const int r0 = tr_row_paired(32 * s, 0), r1 = tr_row_paired(32 * s, 1);
         const bf16x8 kf = frag_tr(cs.khi, C::kKPitch, r0, r1, 16 * kb);
         S[kb] = mfma16x16x32(kf, vh[s], S[kb]);
-        if constexpr (C::kSplit) {
-          S[kb] = mfma16x16x32(kf, vl[s], S[kb]);
-          const bf16x8 kl = frag_tr(cs.klo, C::kKPitch, r0, r1, 16 * kb);
-          S[kb] = mfma16x16x32(kl, vh[s], S[kb]);
-        }
+        S[kb] = mfma16x16x32(kf, vl[s], S[kb]);
+        const bf16x8 kl = frag_tr(cs.klo, C::kKPitch, r0, r1, 16 * kb);
+        S[kb] = mfma16x16x32(kl, vh[s], S[kb]);
       }
     }
     if constexpr (!DELTA) store_state(c);  // state after chunk c
@@ -362,7 +338,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
         for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<IT*>(vb + vn_off + (16 * jb + r) * tok_stride_v) = from_f32<IT>(vn[jb][r]);
+            *reinterpret_cast<float*>(vb + vn_off + (16 * jb + r) * tok_stride_v) = vn[jb][r];
       }
     }
   };
@@ -394,12 +370,7 @@ chunk_fwd_h_kernel(const IT* __restrict__ k, const IT* __restrict__ w, const IT*
   }
 }
 
-// Grids of at least this many workgroups are bandwidth-bound: the register
-// kernel then prefetches two chunks ahead (DEEP), and bf16 inputs take the
-// DMA pipeline of chunk_fwd_h.hip instead.
-constexpr int64_t kHDmaMinGrid = 256;
-
-template <typename IT, int K, int V, bool DELTA>
+template <int K, int V, bool DELTA>
 hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g, const void* h0,
                     void* h, void* vnew, void* ht, char* ws, const seg::Plan& p, int64_t B, int64_t T,
                     int64_t H, hipStream_t s) {
@@ -409,9 +380,9 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
   char* const sbuf = ws + seg::p_bytes(p, BH, NT, K);
   uint32_t* const redo = (uint32_t*)(sbuf + seg::s_bytes(p, BH, NT, K, V));
 #define THM_H_LAUNCH(HG, DP, TR, BV, GRID, NSEG, LEN)                                                       \
-  hipLaunchKernelGGL((chunk_fwd_h_kernel<IT, K, V, DELTA, HG, DP, TR, BV>), dim3((unsigned)(GRID)),         \
-                     dim3(4 * BV), 0, s, (const IT*)k, (const IT*)w, (const IT*)vu, (const float*)g,        \
-                     (const float*)h0, (float*)h, (IT*)vnew, (float*)ht, pbuf, sbuf, redo, T, H, NT, BH, NSEG, LEN, p.per)
+  hipLaunchKernelGGL((chunk_fwd_h_kernel<K, V, DELTA, HG, DP, TR, BV>), dim3((unsigned)(GRID)),             \
+                     dim3(4 * BV), 0, s, (const float*)k, (const float*)w, (const float*)vu, (const float*)g, \
+                     (const float*)h0, (float*)h, (float*)vnew, (float*)ht, pbuf, sbuf, redo, T, H, NT, BH, NSEG, LEN, p.per)
   if constexpr (DELTA) {
     if (p.out > 1) {
       constexpr int BV = seg::h_seg_cols(K, V);
@@ -446,9 +417,5 @@ hipError_t launch_h(const void* k, const void* w, const void* vu, const void* g,
   return hipGetLastError();
 }
 
-// fp32 inputs, defined in chunk_fwd_h_f32.hip (out, per, len: seg::Plan).
 }  // namespace
-__attribute__((visibility("hidden"))) hipError_t chunk_fwd_h_f32(bool delta, int64_t K, int64_t V, const void* k, const void* w, const void* vu,
-                           const void* g, const void* h0, void* h, void* vnew, void* ht, char* ws, int64_t out, int64_t per,
-                           int64_t len, int64_t B, int64_t T, int64_t H, hipStream_t s);
 }  // namespace thm

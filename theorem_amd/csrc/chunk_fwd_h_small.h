@@ -2,10 +2,10 @@
 // workgroups than CUs): a role-split kernel for the chunk latency.  Included
 // by chunk_fwd_h.hip (bf16 inputs) and chunk_fwd_h_f32.hip (fp32 inputs).
 //
-// The math is the register kernel's (chunk_fwd_h_reg.h), operation for
-// operation, so h, v_new and the final state are bit-identical to it (fp32
-// inputs: k and w staged as bf16 hi + lo, S and the gated v_new split the
-// same way, three MFMAs per product):
+// For fp32 inputs the math is the register kernel's (chunk_fwd_h_reg.h),
+// operation for operation (k and w staged as bf16 hi + lo, S and the gated
+// v_new split the same way, three MFMAs per product), so h, v_new and the final
+// state are bit-identical to it; bf16 inputs take one MFMA per product:
 //   reference form (DELTA = false; vu = v)                kernels/chunk_fwd_h/
 //     S <- e^{g_last} S + k_c^T (v_c e^{g_last - g_c});  h[c] = S      reference.py:50-97
 //   delta form (DELTA = true; vu = u)
@@ -38,6 +38,7 @@
 // fewer bytes through its LDS and address unit per chunk.
 #pragma once
 
+#include "chunk_fwd_h.h"
 #include "h_layout.h"
 #include "mfma.h"
 #include "pipe_cfg.h"
@@ -50,7 +51,7 @@ using pipe::SCfg;
 
 // State waves per workgroup (V-tile of 32 columns).  At config 3 (B=2,
 // T=1024, H=3, K=V=64, bf16), per launch with HIP events: 1 state wave
-// 15.9 us, 2 15.6, 4 21.6; the register kernel 26.8.
+// 15.9 us, 2 15.6, 4 21.6; a bf16 form of the register kernel 26.8.
 constexpr int kHSmallNW = 2;
 
 template <typename IT, int K, int V, int NW, bool DELTA, bool HAS_G>
