@@ -155,9 +155,11 @@ int thm_chunk_fwd_h(const void* k, const void* w, const void* vu, const void* g,
  * are deterministic per shape; they agree with thm_chunk_fwd_h's to the
  * rounding of the state).  The segments' maps are formed without the states
  * and may overflow where those do not: columns whose states at the segments'
- * starts are not all finite are walked in one piece instead.  workspace: at least thm_chunk_fwd_h_workspace bytes
- * (0: none needed), 16-byte aligned, owned by the call until it has run on
- * `stream`; otherwise as thm_chunk_fwd_h.
+ * starts are not all finite are walked in one piece instead.  workspace: at
+ * least thm_chunk_fwd_h_workspace bytes (0: none needed), 16-byte aligned, owned
+ * by the call until it has run on `stream`.  h0 and ht must not overlap (the
+ * last segment may write ht while the first still reads h0); otherwise as
+ * thm_chunk_fwd_h.
  */
 int64_t thm_chunk_fwd_h_workspace(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V,
                                   int32_t kv_dtype, int32_t flags);
@@ -249,7 +251,8 @@ int thm_chunk_gated_delta_fwd_a(const void* q, const void* k, const void* v, con
  *   bytes (its contents before and after are undefined), owned by the call
  *   until it has run on `stream`.  Long sequences of few heads are cut into
  *   segments that run side by side, chosen from the shape and the device's CU
- *   count only, so results are deterministic per shape.
+ *   count only, so results are deterministic per shape.  h0 and ht must not
+ *   overlap.
  */
 int64_t thm_chunk_gated_delta_rule_workspace(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V);
 int thm_chunk_gated_delta_rule_fwd(const void* q, const void* k, const void* v, const void* beta,

@@ -14,14 +14,14 @@
 // Launches:
 //   1. records (wy_build_A.hip): A, gates and factors of every chunk;
 //   2. where the sequences alone leave the GPU idle, the state at the start of
-//      each of several segments of the sequences (transition and combine
-//      kernels below);
+//      each of several segments of the sequences (segments.h, the transition
+//      and combine kernels; how many, seg_plan.h);
 //   3. the output kernel, one workgroup per (b, head, segment, 64-column
 //      V-tile).
 //
 // Segments (segments.h) cost less than twice the recurrence's own work,
 // against a serial chain shorter by their number: B = 1, T = 8192, H = 16,
-// K = V = 128 (32 workgroups of 128 chunks without them) 276 -> 107 us for the
+// K = V = 128 (32 workgroups of 128 chunks without them) 274 -> 116 us for the
 // whole forward.
 #include "h_layout.h"
 #include "mfma.h"

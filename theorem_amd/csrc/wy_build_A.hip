@@ -170,16 +170,16 @@ wy_build_A_kernel(const IT* __restrict__ k, const float* __restrict__ beta,
 // in LDS and the MFMA fragments are read from there.  The arithmetic is the
 // one-tile kernel's, so A is bit-identical.
 // Workgroups per CU: 4.  The inversion's latency chain, not memory, sets this
-// kernel's time (timing-only copies at config 4: 105.4 us; without the
-// inversion 26.6, without the next tile's loads 99.5, without the stores of
-// A 95.2), so the more tiles a CU inverts at once the better:
+// kernel's time, so the more tiles a CU inverts at once the better (times at
+// config 4 with an earlier inversion, whose off-diagonal products went through
+// LDS: without the inversion a quarter of the time; wy_blocks.h has today's):
 //   * the k loads go through one 32-bit per-lane offset on a wave-uniform
 //     base (h_layout.h o_blk_lane / o_blk_step; 64-bit addresses spilled at
 //     3 workgroups): 2 -> 3 per CU, 140 -> 116 us;
-//   * the X and T blocks share the k tile's LDS (31.7 KB per workgroup
-//     instead of 48.6) and form_L reads its k fragments per block
-//     (wy::form_L_lds; 120 VGPRs at K = 128, no scratch): 3 -> 4 per CU,
-//     105.7 -> 96.3 us.  5 per CU spill (140 us).
+//   * the X blocks share the k tile's LDS (31.9 KB per workgroup at K = 128
+//     instead of 44.9) and form_L reads its k fragments per block
+//     (wy::form_L_lds; 114 VGPRs at K = 128, no scratch): 3 -> 4 per CU,
+//     105.7 -> 96.3 us.  5 per CU spilled (140 us).
 // A is bit-identical throughout.
 template <int K>
 constexpr int ab_pipe_wgs_per_cu() { return 4; }
@@ -197,8 +197,8 @@ wy_build_A_pipe_kernel(const bf16* __restrict__ k, const float* __restrict__ bet
   constexpr int kLoads = kBT * kCPR / kABThreads;     // per thread
   static_assert(kBT * kCPR % kABThreads == 0, "staging split");
   // The k tile is read only up to the barrier after form_L and restaged
-  // after the barrier that follows the store of A, so the inversion's X and T
-  // blocks share its LDS.
+  // after the barrier that follows the store of A, so the inversion's X blocks
+  // share its LDS.
   constexpr int kKBytes = kBT * kPitch * 2, kXBytes = 10 * kBlk * 4;
   __shared__ __attribute__((aligned(16))) char kxt[kKBytes > kXBytes ? kKBytes : kXBytes];
   bf16* const ks = reinterpret_cast<bf16*>(kxt);
