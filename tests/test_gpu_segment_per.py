@@ -65,3 +65,29 @@ def test_delta_form(dev, dt, B, H, NT, K, V, state):
         h, vn, ht = (got[0][b:b + 1, :, hh:hh + 1], got[1][b:b + 1, :, hh:hh + 1], got[2][b:b + 1, hh:hh + 1])
         for name, x, e in (("h", h, exp[0]), ("v_new", vn, exp[1]), ("final state", ht, exp[2])):
             assert_close(x, e, tol, tol, f"{name} of ({b}, {hh})")
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("delta", [True, False])
+def test_capture(dev, dt, delta):
+    # Neither the segments nor the reference form's scan keep anything between
+    # calls: a captured call replays to the eager result.
+    B, T, H, K, V = (1, 64 * 100, 3, 128, 128) if delta else (2, 64 * 16, 3, 64, 64)
+    d = configs.make_h_inputs(B, T, H, K, V, seed=5, device=dev, dtype=dt, gate="mild", h0_std=0.1)
+    h0, w, u = d.pop("h0"), d.pop("w"), d.pop("u")
+    assert (_capi.load_library().thm_chunk_fwd_h_workspace(B, T, H, K, V, _capi.THM_DTYPE[dt], int(delta)) > 0) == delta
+    d.update(dict(w=w, u=u) if delta else dict(v=u), initial_state=h0, output_final_state=True)
+    run = lambda: chunk_fwd_h.custom_kernel(d)  # noqa: E731
+    ref = run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run()
+    for _ in range(3):
+        for x in got:
+            x.zero_()
+        graph.replay()
+        eager = run()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(ref, got))
+        assert all(torch.equal(x, y) for x, y in zip(ref, eager))
