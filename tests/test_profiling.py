@@ -62,6 +62,12 @@ def test_unknown_unit_raises_and_cli_takes_units_keys(tmp_path):
     rec = json.loads(out.read_text())["chunk_fwd_h"]
     assert rec["source_digest"] == profiling.source_digest(profiling.UNITS["chunk_fwd_h"])
     assert rec["hbm_read_bytes"] == 8 * 1024 * 2 and rec["hbm_write_bytes"] == 4 * 1024
+    # rocprofv3 prints some kernels demangled, with colons in the name.
+    name = "void thm::(anonymous namespace)::kernel<128>"
+    _counter_csv(kern, [(name + "(int)", "FETCH_SIZE", 8.0), (name + "(int)", "WRITE_SIZE", 4.0)])
+    spec = f"wy_build_A=wy_build_A:{name}:24576:{kern}:{kern}"
+    assert profiling.main(["profiling", "traffic", str(out), str(calib), str(calib), "1048576", spec]) == 0
+    assert json.loads(out.read_text())["wy_build_A"]["hbm_read_bytes"] == 8 * 1024 * 2
 
 
 def _counter_csv(path: Path, rows):

@@ -110,7 +110,8 @@ def main(argv: list[str]) -> int:
     targets = {}
     for spec in argv[6:]:
         name, rest = spec.split("=", 1)
-        unit, sym, alg, fdir, wdir = rest.split(":")
+        unit, rest = rest.split(":", 1)
+        sym, alg, fdir, wdir = rest.rsplit(":", 3)  # (a demangled symbol has colons of its own)
         targets[name] = (UNITS.get(unit, unit), sym, int(alg), fdir, wdir)
     res = traffic_summary(cfd, cwd, copy_bytes, targets)
     Path(out).write_text(json.dumps(res, indent=1) + "\n")
